@@ -182,3 +182,42 @@ def test_zgeev_qr_kernel_variants(ctx, variant, n):
         _eig_check(ctx, A)
     finally:
         assert ctx.lib.vrc_tune_set(b"zgeev.qr_variant", -1) == 0
+
+
+@pytest.mark.parametrize("variant", [0, 2, 4])
+@pytest.mark.parametrize("n", [2, 4, 31, 32, 33, 47, 50, 63, 64, 66])
+def test_zgeev_window_edges(ctx, variant, n):
+    """Sizes at the edges of the QR kernels' windows (32, 48, 64) and of the single-wavefront
+    Schur form's two lane layouts (32), with entries of order one, entries whose squares leave
+    the range of the fast rotations (1e140, 1e-140), and a cyclic shift (rotations with an
+    exactly zero first entry)."""
+    rng = np.random.default_rng(3000 + n)
+    A = crand(rng, 2, n, n)
+    shift = np.roll(np.eye(n), 1, axis=0).astype(complex)
+    assert ctx.lib.vrc_tune_set(b"zgeev.qr_variant", variant) == 0
+    try:
+        for scale in (1.0, 1e140, 1e-140):
+            _eig_check(ctx, A * scale)
+        w, _ = _eig_check_values(ctx, shift[None])
+        assert np.abs(w[0] ** n - 1.0).max() < 1e-12 * n * n
+    finally:
+        assert ctx.lib.vrc_tune_set(b"zgeev.qr_variant", -1) == 0
+
+
+def _eig_check_values(ctx, A):
+    """Eigenvalues and vectors with the residual checked (no comparison of sorted spectra:
+    eigenvalues of one modulus sort arbitrarily)."""
+    import torch
+    batch, n, _ = A.shape
+    dA = to_dev_colmajor(A)
+    w = torch.zeros((batch, n), dtype=torch.complex128, device="cuda")
+    VR = torch.zeros_like(dA)
+    info = torch.zeros(batch, dtype=torch.int32, device="cuda")
+    ctx.check(ctx.lib.vrc_zgeev(ctx.h, n, ptr(dA), n, n * n, ptr(w), n, ptr(VR), n, n * n, ptr(info), batch),
+              "zgeev")
+    ctx.sync()
+    assert info.cpu().numpy().tolist() == [0] * batch
+    W, V = w.cpu().numpy(), from_dev_colmajor(VR)
+    for b in range(batch):
+        assert np.abs(A[b] @ V[b] - V[b] * W[b][None, :]).max() < 1e-12 * n * np.linalg.norm(A[b], 2)
+    return W, V

@@ -176,7 +176,8 @@ std::string autotune_stack(vrc_ctx& c, int nx, int ny, const std::vector<StackIn
   // A switch is searched only where it can change what runs: the QR switches only when the
   // best setting so far launches a QR kernel, the bulge count of each QR kernel only when it
   // launches that kernel, and a deflation window only when, clamped to the window limit
-  // (W - 1) of each kernel launched, it differs from the best one's.
+  // (W - 1) of each kernel launched, it differs from the best one's (-1, the automatic window,
+  // differs from all).
   constexpr unsigned QR_ANY = 0u, QR_W64 = (1u << 0) | (1u << 1), QR_W48 = 1u << 2, QR_W32 = 1u << 4;
   constexpr unsigned QR_ALL = QR_W64 | QR_W48 | QR_W32;
   auto aed_effective = [](int v, unsigned kernels) {
@@ -198,7 +199,7 @@ std::string autotune_stack(vrc_ctx& c, int nx, int ny, const std::vector<StackIn
     };
     const std::vector<Switch> space = {
         {&TuneKnobs::qr_variant, {0, 2, 4}, QR_ALL},
-        {&TuneKnobs::aed, {16, 20, 24, 32, 40, 48}, QR_ALL},
+        {&TuneKnobs::aed, {8, 12, 16, 20, 24, 32, 40, 48}, QR_ALL},
         {&TuneKnobs::bulges, {6, 8, 10, 12, 14, 16}, QR_W64},
         {&TuneKnobs::bulges_w48, {4, 6, 8, 10, 12}, QR_W48},
         {&TuneKnobs::bulges_w32, {3, 4, 5, 6, 7}, QR_W32},

@@ -33,7 +33,6 @@ constexpr int QW = 64;         // maximal QR window
 constexpr int NBUL = 16;       // most bulges per sweep (2 shifts each)
 constexpr int QR_NMIN = 48;    // active blocks this small are finished in LDS
 constexpr int EXC_SWEEPS = 6;  // sweeps without deflation before exceptional shifts
-constexpr int AED_NW = 24;     // default deflation window (measured best of 16..64 at N = 882)
 constexpr int AED_NIBBLE = 14; // skip the sweep when the window deflated more than this percentage
 
 __device__ inline double wsum(double v) {
@@ -56,31 +55,50 @@ __device__ inline void house(cd alpha, double xnorm, double& beta, cd& tau, cd& 
   scale = crecip(mk(alpha.x - beta, alpha.y));
 }
 
-// The same reflector for alpha and x = (y, z) (z = 0 for a 2-vector) with one square root
-// and two divisions: sqrt(|alpha|^2 + |y|^2 + |z|^2) directly and 1/(alpha - beta) as
-// conj(d) / |d|^2. Used when every component lies in [2^-400, 2^400] (no overflow or
-// underflow in the squares); otherwise the scaled form above.
-__device__ inline void house_small(cd alpha, cd y, cd z, double& beta, cd& tau, cd& scale) {
-  const double m = fmax(fmax(fmax(fabs(alpha.x), fabs(alpha.y)), fmax(fabs(y.x), fabs(y.y))),
-                        fmax(fabs(z.x), fabs(z.y)));
-  const double xn2 = cnorm2(y) + cnorm2(z);
-  if (!(m <= 0x1p400 && (m >= 0x1p-400 || m == 0.0))) {
-    house(alpha, hypot(cabsv(y), cabsv(z)), beta, tau, scale);
+// 1/sqrt(v) and 1/v for normal positive (nonzero) v: the hardware estimate (about 23 good
+// bits) and one third-order Newton step, within about one unit in the last place.
+__device__ __forceinline__ double rsqrt_nr(double v) {
+  const double y = __builtin_amdgcn_rsq(v);
+  const double e = fma(-v * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double rcp_nr(double v) {
+  const double y = __builtin_amdgcn_rcp(v);
+  const double e = fma(-v, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+// Squares of values whose sum lies in this range neither overflow nor lose small parts.
+__device__ __forceinline__ bool squares_safe(double s) { return s <= 0x1p800 && s >= 0x1p-800; }
+
+// The reflector of house() for |x|^2 = xn2 without a division or a square root in the
+// chain: 1/|(alpha, x)| from one reciprocal square root, 1/(alpha - beta) as conj(d) / |d|^2.
+// Out of range of the squares: house().
+__device__ __forceinline__ void house_fast(cd alpha, double xn2, double& beta, cd& tau, cd& scale) {
+  const double d2 = cnorm2(alpha) + xn2;
+  if (__builtin_expect(!squares_safe(d2), 0)) {
+    house(alpha, sqrt(xn2), beta, tau, scale);
     return;
   }
-  if (xn2 == 0.0 && alpha.y == 0.0) {
-    beta = alpha.x;
-    tau = mk(0.0, 0.0);
-    scale = mk(0.0, 0.0);
-    return;
-  }
-  const double nrm = sqrt(cnorm2(alpha) + xn2);
-  beta = alpha.x >= 0.0 ? -nrm : nrm;
-  const double rb = 1.0 / beta;
-  tau = mk((beta - alpha.x) * rb, -alpha.y * rb);
+  const double rs = rsqrt_nr(d2);
+  beta = -copysign(d2 * rs, alpha.x);
+  const double rb = -copysign(rs, alpha.x);
   const double dx = alpha.x - beta, dy = alpha.y;
-  const double id = 1.0 / (dx * dx + dy * dy);
+  const double id = rcp_nr(dx * dx + dy * dy);
+  tau = mk((beta - alpha.x) * rb, -dy * rb);
   scale = mk(dx * id, -dy * id);
+  if (xn2 == 0.0 && dy == 0.0) {
+    beta = alpha.x;
+    tau = scale = mk(0.0, 0.0);
+  }
+}
+
+// The same for x = (y, z) (z = 0 for a 2-vector).
+__device__ __forceinline__ void house_small(cd alpha, cd y, cd z, double& beta, cd& tau, cd& scale) {
+  const double xn2 = cnorm2(y) + cnorm2(z);
+  if (__builtin_expect(squares_safe(cnorm2(alpha) + xn2), 1))
+    house_fast(alpha, xn2, beta, tau, scale);
+  else
+    house(alpha, hypot(cabsv(y), cabsv(z)), beta, tau, scale);
 }
 
 // ===================================================================== Hessenberg
@@ -576,9 +594,6 @@ struct QrLds {
   QMat<W> Hw;
   QMat<W> U;
   cd shifts[2 * NBUL];
-  cd rv1[NBUL], rv2[NBUL], rtau[NBUL];
-  double rbeta[NBUL];
-  int rsize[NBUL], rrow[NBUL], rcol[NBUL];
   int redi[T];
   cd aedv[64];  // written by every lane of a wavefront
   int ctl[4];
@@ -694,18 +709,67 @@ __device__ inline bool negl_lds(const Mat& Hw, int k, int l, int i, double smlnu
   return false;
 }
 
+// Complex Givens rotation with real c (LAPACK zlartg semantics):
+// [c s; -conj(s) c] [f; g] = [r; 0].
+__device__ inline void givens_scaled(cd f, cd g, double& c, cd& s, cd& r) {
+  const double f1 = cabsv(f), g1 = cabsv(g);
+  if (g1 == 0.0) {
+    c = 1.0;
+    s = mk(0.0, 0.0);
+    r = f;
+  } else if (f1 == 0.0) {
+    c = 0.0;
+    s = cscale(cconj(g), 1.0 / g1);
+    r = mk(g1, 0.0);
+  } else {
+    const double d = hypot(f1, g1);
+    const cd ph = cscale(f, 1.0 / f1);
+    c = f1 / d;
+    s = cscale(cmul(ph, cconj(g)), 1.0 / d);
+    r = cscale(ph, d);
+  }
+}
+// One reciprocal square root: with a = 1 / (|f| d), d^2 = |f|^2 + |g|^2, the rotation is
+// c = |f|^2 a, s = f conj(g) a, r = f d^2 a. Used when |f|^2 d^2 stays well inside the range.
+__device__ __forceinline__ void givens_fast(cd f, cd g, double& c, cd& s, cd& r) {
+  const double f2 = cnorm2(f), d2 = f2 + cnorm2(g);
+  if (__builtin_expect(!(f2 >= 0x1p-400 && d2 <= 0x1p400), 0)) {
+    givens_scaled(f, g, c, s, r);
+    return;
+  }
+  const double a = rsqrt_nr(f2 * d2);
+  c = f2 * a;
+  s = cscale(cmulc(f, g), a);
+  r = cscale(f, d2 * a);
+}
+
 // Eigenvalue of the 2x2 block [[a, b], [c, d]] closest to d.
 __device__ inline cd wilkinson(cd a, cd b, cd c, cd d) {
-  cd u = cmul(csqrt_principal(b), csqrt_principal(c));
-  double su = cabs1(u);
+  const cd x = cscale(csub(a, d), 0.5), u2 = cmul(b, c);
+  const double xx = cnorm2(x), uu = cnorm2(u2);
+  if (uu == 0.0 && cabs1(b) * cabs1(c) == 0.0) return d;
+  const cd z = cadd(cmul(x, x), u2);
+  const double m2 = cnorm2(z);
+  // y = sqrt(z) with |z| = sqrt(m2), h = (|Re z| + |z|) / 2, one part sqrt(h), the other Im z / (2 sqrt(h))
+  if (xx <= 0x1p200 && uu <= 0x1p400 && m2 >= 0x1p-400) {
+    const double h = 0.5 * (fabs(z.x) + m2 * rsqrt_nr(m2));
+    const double rh = rsqrt_nr(h);
+    const double p = h * rh, q = 0.5 * z.y * rh;
+    cd y = z.x >= 0.0 ? mk(p, q) : mk(fabs(q), copysign(p, z.y));
+    if (x.x * y.x + x.y * y.y < 0.0) y = cneg(y);
+    const cd v = cadd(x, y);
+    const double v2 = cnorm2(v);
+    if (v2 >= 0x1p-400) return csub(d, cscale(cmulc(u2, v), rcp_nr(v2)));
+  }
+  const cd u = cmul(csqrt_principal(b), csqrt_principal(c));
+  const double su = cabs1(u);
   if (su == 0.0) return d;
-  cd x = cscale(csub(a, d), 0.5);
-  double sx = cabs1(x);
-  double sc = fmax(su, sx);
-  cd xs = cscale(x, 1.0 / sc), us = cscale(u, 1.0 / sc);
+  const double sx = cabs1(x);
+  const double sc = fmax(su, sx);
+  const cd xs = cscale(x, 1.0 / sc), us = cscale(u, 1.0 / sc);
   cd y = cscale(csqrt_principal(cadd(cmul(xs, xs), cmul(us, us))), sc);
   if (sx > 0.0) {
-    cd xn = cscale(x, 1.0 / sx);
+    const cd xn = cscale(x, 1.0 / sx);
     if (xn.x * y.x + xn.y * y.y < 0.0) y = cneg(y);
   }
   return csub(d, cmul(u, cdiv(u, cadd(x, y))));
@@ -719,33 +783,56 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
+// v of lane l (the same l in every lane).
+__device__ __forceinline__ double lane_value(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
 }
+__device__ __forceinline__ cd lane_value(cd v, int l) { return mk(lane_value(v.x, l), lane_value(v.y, l)); }
+// All LDS reads issued so far have returned (a loop whose body reads registers loaded before
+// it would otherwise wait for its own reads at the same place).
+__device__ __forceinline__ void lds_wait() { __builtin_amdgcn_s_waitcnt(0xc07f); }
+__device__ __forceinline__ cd pick(bool c, cd a, cd b) { return mk(c ? a.x : b.x, c ? a.y : b.y); }
 
 // Complete Schur decomposition of the s x s Hessenberg block in Hw (s <= QW) by
-// single-shift QR, run by ONE wavefront (lane = column / row index), accumulating the
-// transform into U when wantU (U must hold the identity or an earlier transform).
-// Subdiagonal entries are set to exact zeros on deflation, so Hw ends upper
-// triangular. Returns 0 on success, else (index of the unconverged eigenvalue + 1).
-template <class Mat>
-__device__ int wave_schur(Mat& Hw, Mat& U, int s, bool wantU, int lane) {
+// single-shift QR, run by ONE wavefront, accumulating the transform into U when WU (U must
+// hold the identity or an earlier transform). Subdiagonal entries are set to exact zeros on
+// deflation, so Hw ends upper triangular. Returns 0 on success, else (index of the
+// unconverged eigenvalue + 1).
+//
+// A sweep is one serial chain of rotations, so the chain alone is kept short: the entries the
+// next rotation needs (rows k .. k+2 of columns k, k+1) stay in registers, the same in every
+// lane, and never wait for LDS. Row k + 1 as it stands (lane = column) and column k + 1 as it
+// stands (lane = row) are carried in registers from step to step, so each step reads one new
+// row and one new column, neither of which the chain waits for, and writes one finished row
+// and column. HALF (s <= 32): lanes 0..31 rotate the rows of Hw and lanes 32..63 those of U.
+// 32 x 32 random blocks: 0.34 us per rotation (about 100 FP64 instructions, issue-bound); with
+// the whole step through LDS and a reflector with a square root and two divisions 0.68 us.
+template <bool HALF, bool WU, class Mat>
+__device__ __forceinline__ int wave_schur_impl(Mat& Hw, Mat& U, int s, int lane) {
   const double smlnum = SAFMIN * ((double)s / ULP);
   const int itmax = 30 * (s > 10 ? s : 10);
+  const int col = lane < s ? lane : s - 1;
+  const bool ulane = HALF && lane >= 32;
+  int row = HALF ? (lane & 31) : lane;
+  const bool rowin = row < s;
+  if (!rowin) row = s - 1;
+  cd* const cr = ulane ? &U[row][0] : &Hw[row][0];  // this lane's row in the column rotations
+  // the lane writes column k when k >= cfrom, row k when its column >= k + 2
+  const int cfrom = ulane ? ((WU && rowin) ? -1 : 1 << 20) : lane;
+  const int rcol = lane < s ? lane : -1;
   int i = s - 1;
   while (i >= 0) {
     int l = 0;
     bool conv = false;
     for (int its = 0; its <= itmax; ++its) {
+      wave_sync();
       const bool ng = (lane >= 1 && lane <= i) ? negl_lds(Hw, lane, 0, i, smlnum) : false;
       const unsigned long long mask = __ballot(ng);
-      const int k = mask ? 63 - __clzll(mask) : 0;
+      l = mask ? 63 - __clzll(mask) : 0;
       wave_sync();
-      if (k > 0 && lane == 0) Hw[k][k - 1] = mk(0.0, 0.0);
+      if (l > 0 && lane == 0) Hw[l][l - 1] = mk(0.0, 0.0);
       wave_sync();
-      l = k;
       if (l >= i) {
         conv = true;
         break;
@@ -758,79 +845,127 @@ __device__ int wave_schur(Mat& Hw, Mat& U, int s, bool wantU, int lane) {
       } else {
         sh = wilkinson(Hw[i - 1][i - 1], Hw[i - 1][i], Hw[i][i - 1], Hw[i][i]);
       }
-      for (int k2 = l; k2 < i; ++k2) {
-        cd x, y;
-        if (k2 == l) {
-          x = csub(Hw[l][l], sh);
-          y = Hw[l + 1][l];
-        } else {
-          x = Hw[k2][k2 - 1];
-          y = Hw[k2 + 1][k2 - 1];
+      // chain state: (x, y) = column k - 1 of rows k, k + 1; (p, q) = column k of rows k, k + 1
+      cd p = Hw[l][l], q = Hw[l + 1][l];
+      cd x = csub(p, sh), y = q;
+      cd rc = Hw[l][col];  // row k, lane = column (columns > k)
+      cd cc = cr[l];       // column k, lane = row (rows < k of Hw; every row of U)
+      cd uc = (WU && !HALF) ? U[row][l] : mk(0.0, 0.0);
+      lds_wait();
+      for (int k = l; k < i; ++k) {
+        const cd n = Hw[k + 1][col];
+        const cd u = Hw[k + 1][k + 1];
+        const cd w = Hw[k + 2 <= i ? k + 2 : i][k + 1];  // below the block: y, q are not used
+        const cd b = cr[k + 1];
+        const cd ub = (WU && !HALF) ? U[row][k + 1] : mk(0.0, 0.0);
+        double c;
+        cd sn, r;
+        givens_fast(x, y, c, sn, r);
+        const cd sc = cconj(sn);
+        const cd t = lane_value(rc, k + 1);
+        // rows k, k + 1 of columns k, k + 1
+        const cd p1 = cadd(cscale(p, c), cmul(sn, q)), q1 = csub(cscale(q, c), cmul(sc, p));
+        const cd t1 = cadd(cscale(t, c), cmul(sn, u)), u1 = csub(cscale(u, c), cmul(sc, t));
+        // columns k, k + 1 of row k + 1 and of row k + 2 (whose column k is zero)
+        x = cadd(cscale(q1, c), cmul(sc, u1));
+        p = csub(cscale(u1, c), cmul(sn, q1));
+        y = cmul(sc, w);
+        q = cscale(w, c);
+        // rows k, k + 1 of the columns right of them
+        const cd rk = cadd(cscale(rc, c), cmul(sn, n));
+        rc = csub(cscale(n, c), cmul(sc, rc));
+        // columns k, k + 1 of the rows above (row k enters here) and of U
+        const cd a0 = pick(lane == k, p1, cc), b0 = pick(lane == k, t1, b);
+        const cd ck = cadd(cscale(a0, c), cmul(sc, b0));
+        cc = csub(cscale(b0, c), cmul(sn, a0));
+        const bool sub = rcol == (k > l ? k - 1 : -2);  // the subdiagonal entry left behind
+        if ((rcol >= k + 2) | sub) Hw[k][lane] = pick(sub, r, rk);
+        if (cfrom <= k) cr[k] = ck;
+        if (WU && !HALF) {
+          const cd uk = cadd(cscale(uc, c), cmul(sc, ub));
+          uc = csub(cscale(ub, c), cmul(sn, uc));
+          if (rowin) U[row][k] = uk;
         }
-        double beta;
-        cd tau, scale;
-        house_small(x, y, mk(0.0, 0.0), beta, tau, scale);
-        const cd v1 = cmul(y, scale);
         wave_sync();
-        if (tau.x == 0.0 && tau.y == 0.0) continue;
-        if (lane < s) {
-          const int j = lane;
-          if (k2 > l && j == k2 - 1) {
-            Hw[k2][j] = mk(beta, 0.0);
-            Hw[k2 + 1][j] = mk(0.0, 0.0);
-          } else {
-            const cd h1 = Hw[k2][j], h2 = Hw[k2 + 1][j];
-            const cd sm = cmul(cconj(tau), cadd(h1, cmul(cconj(v1), h2)));
-            Hw[k2][j] = csub(h1, sm);
-            Hw[k2 + 1][j] = csub(h2, cmul(sm, v1));
-          }
-        }
-        wave_sync();
-        if (lane < s) {
-          const cd c1 = Hw[lane][k2], c2 = Hw[lane][k2 + 1];
-          const cd sm = cmul(tau, cadd(c1, cmul(c2, v1)));
-          Hw[lane][k2] = csub(c1, sm);
-          Hw[lane][k2 + 1] = csub(c2, cmul(sm, cconj(v1)));
-          if (wantU) {
-            const cd u1 = U[lane][k2], u2 = U[lane][k2 + 1];
-            const cd su = cmul(tau, cadd(u1, cmul(u2, v1)));
-            U[lane][k2] = csub(u1, su);
-            U[lane][k2 + 1] = csub(u2, cmul(su, cconj(v1)));
-          }
-        }
-        wave_sync();
+      }
+      if (rcol > i) Hw[i][lane] = rc;
+      if (cfrom < i) cr[i] = cc;
+      if (WU && !HALF && rowin) U[row][i] = uc;
+      if (lane == 0) {
+        Hw[i][i] = p;
+        Hw[i][i - 1] = x;
       }
     }
     if (!conv) return i + 1;
     i = l - 1;
   }
+  wave_sync();
   return 0;
 }
 
-// Complex Givens rotation (LAPACK zlartg semantics): [cs sn; -conj(sn) cs] [f; g] = [r; 0].
-__device__ inline void givens(cd f, cd g, double& cs, cd& sn) {
-  const double f1 = cabsv(f), g1 = cabsv(g);
-  if (g1 == 0.0) {
-    cs = 1.0;
-    sn = mk(0.0, 0.0);
-  } else if (f1 == 0.0) {
-    cs = 0.0;
-    sn = cscale(cconj(g), 1.0 / g1);
-  } else {
-    const double d = sqrt(f1 * f1 + g1 * g1);
-    cs = f1 / d;
-    sn = cscale(cmul(cscale(f, 1.0 / f1), cconj(g)), 1.0 / d);
-  }
+template <class Mat>
+__device__ __forceinline__ int wave_schur(Mat& Hw, Mat& U, int s, bool wantU, int lane) {
+  if (!wantU) return wave_schur_impl<false, false>(Hw, U, s, lane);
+  if (s <= 32) return wave_schur_impl<true, true>(Hw, U, s, lane);
+  return wave_schur_impl<false, true>(Hw, U, s, lane);
 }
 
-// Swap the adjacent diagonal entries k, k+1 of the n x n upper-triangular T by a Givens
-// rotation (LAPACK ztrexc step), updating the Schur vectors U (n rows). One wavefront.
+// Moves the diagonal entry j of the n x n upper-triangular T up to position to by Givens
+// swaps of adjacent entries (LAPACK ztrexc), updating the Schur vectors U (n rows). One
+// wavefront, n <= 32: the moving row (lane = column) and the moving column (lane = row; lanes
+// 32.. carry U's) stay in registers, as in wave_schur_impl.
 template <class Mat>
-__device__ void wave_swap(Mat& T, Mat& U, int n, int k, int lane) {
+__device__ __forceinline__ void wave_move_up(Mat& T, Mat& U, int n, int j, int to, int lane) {
+  if (j <= to) return;
+  const bool ulane = lane >= 32;
+  int row = lane & 31;
+  const bool rowin = row < n;
+  if (!rowin) row = n - 1;
+  const int col = lane < n ? lane : n - 1;
+  cd* const cr = ulane ? &U[row][0] : &T[row][0];
+  const int cfrom = ulane ? (rowin ? -1 : 1 << 20) : lane;  // writes column k + 1 when k >= cfrom
+  const int rcol = lane < n ? lane : -1;
+  const cd lam = T[j][j];
+  const cd dg = T[col][col];  // the diagonal, lane = index
+  cd mr = T[j][col];          // the moving row, columns > k + 1
+  cd mc = cr[j];              // the moving column, rows <= k (every row of U)
+  cd xc = cr[j - 1];          // column k
+  wave_sync();
+  lds_wait();
+  for (int k = j - 1; k >= to; --k) {
+    const cd xr = T[k][col];
+    const cd xn = cr[k > 0 ? k - 1 : 0];  // the next step's column (this step leaves it alone)
+    const cd t11 = lane_value(dg, k);
+    const cd g = lane_value(mc, k);  // T[k][k + 1]
+    double c;
+    cd sn, r;
+    givens_fast(g, csub(lam, t11), c, sn, r);
+    const cd sc = cconj(sn);
+    const cd cdn = pick(lane == k, g, csub(cscale(mc, c), cmul(sn, xc)));  // column k + 1, rows <= k
+    mc = cadd(cscale(xc, c), cmul(sc, mc));
+    const cd rdn = csub(cscale(mr, c), cmul(sc, xr));  // row k + 1, columns >= k + 2
+    mr = pick(lane == k + 1, g, cadd(cscale(xr, c), cmul(sn, mr)));  // T[k][k + 1] keeps its value
+    xc = xn;
+    wave_sync();
+    // row k + 1 from the diagonal on; column k + 1 down to row k (every row of U)
+    if (rcol > k) T[k + 1][lane] = pick(lane == k + 1, t11, rdn);
+    if (cfrom <= k) cr[k + 1] = cdn;
+    wave_sync();
+  }
+  if (rcol > to) T[to][lane] = mr;
+  if (cfrom < to) cr[to] = mc;
+  if (lane == 0) T[to][to] = lam;
+  wave_sync();
+}
+
+// Swap the adjacent diagonal entries k, k+1 of the n x n upper-triangular T (n > 32: one swap
+// at a time, through LDS), updating the Schur vectors U (n rows). One wavefront.
+template <class Mat>
+__device__ __forceinline__ void wave_swap(Mat& T, Mat& U, int n, int k, int lane) {
   const cd t11 = T[k][k], t22 = T[k + 1][k + 1];
   double cs;
-  cd sn;
-  givens(T[k][k + 1], csub(t22, t11), cs, sn);
+  cd sn, r;
+  givens_fast(T[k][k + 1], csub(t22, t11), cs, sn, r);
   wave_sync();
   if (lane >= k + 2 && lane < n) {  // rows k, k+1 from column k+2 on
     const cd x = T[k][lane], y = T[k + 1][lane];
@@ -858,27 +993,47 @@ __device__ void wave_swap(Mat& T, Mat& U, int n, int k, int lane) {
 // T <- G^H T on rows r0..r0+len-1 (columns c0..n-1), then T <- T G on those columns
 // (rows 0..rows_t-1) and U <- U G (rows 0..n-1), G = I - tau v v^H with v in vv[0..len).
 template <class Mat>
-__device__ void wave_reflect(Mat& T, Mat& U, const cd* vv, cd tau, int r0, int len, int c0, int n, int rows_t,
-                             int lane) {
-  const cd ct = cconj(tau);
-  if (lane >= c0 && lane < n) {
+__device__ __forceinline__ void wave_reflect(Mat& T, Mat& U, const cd* vv, cd tau, int r0, int len, int c0, int n,
+                                             int rows_t, int lane) {
+  // e_q, q < len, at step doubles apart: sum f(v_q) e_q and e_q -= d g(v_q), four at a time
+  auto dot = [&](const cd* e, int step, bool conjv) {
     cd d = mk(0.0, 0.0);
-    for (int q = 0; q < len; ++q) d = cadd(d, cmul(cconj(vv[q]), T[r0 + q][lane]));
-    d = cmul(ct, d);
-    for (int q = 0; q < len; ++q) T[r0 + q][lane] = csub(T[r0 + q][lane], cmul(vv[q], d));
+    int q = 0;
+    for (; q + 4 <= len; q += 4) {
+      cd a[4], v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a[k] = e[(q + k) * step], v[k] = vv[q + k];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d = cadd(d, conjv ? cmulc(a[k], v[k]) : cmul(a[k], v[k]));
+    }
+    for (; q < len; ++q) d = cadd(d, conjv ? cmulc(e[q * step], vv[q]) : cmul(e[q * step], vv[q]));
+    return d;
+  };
+  auto axpy = [&](cd* e, int step, cd d, bool conjv) {
+    int q = 0;
+    for (; q + 4 <= len; q += 4) {
+      cd a[4], v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a[k] = e[(q + k) * step], v[k] = vv[q + k];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) e[(q + k) * step] = csub(a[k], conjv ? cmulc(d, v[k]) : cmul(d, v[k]));
+    }
+    for (; q < len; ++q) e[q * step] = csub(e[q * step], conjv ? cmulc(d, vv[q]) : cmul(d, vv[q]));
+  };
+  if (lane >= c0 && lane < n) {
+    const cd d = cmul(cconj(tau), dot(&T[r0][lane], (int)(&T[1][0] - &T[0][0]), true));
+    axpy(&T[r0][lane], (int)(&T[1][0] - &T[0][0]), d, false);
   }
   wave_sync();
-  if (lane < n) {
-    if (lane < rows_t) {
-      cd d = mk(0.0, 0.0);
-      for (int q = 0; q < len; ++q) d = cadd(d, cmul(T[lane][r0 + q], vv[q]));
-      d = cmul(tau, d);
-      for (int q = 0; q < len; ++q) T[lane][r0 + q] = csub(T[lane][r0 + q], cmul(d, cconj(vv[q])));
+  if (n <= 32) {  // lanes 0..31 the rows of T, lanes 32..63 those of U
+    const int row = lane & 31;
+    if (lane >= 32 ? row < n : row < rows_t) {
+      cd* e = lane >= 32 ? &U[row][r0] : &T[row][r0];
+      axpy(e, 1, cmul(tau, dot(e, 1, false)), true);
     }
-    cd e = mk(0.0, 0.0);
-    for (int q = 0; q < len; ++q) e = cadd(e, cmul(U[lane][r0 + q], vv[q]));
-    e = cmul(tau, e);
-    for (int q = 0; q < len; ++q) U[lane][r0 + q] = csub(U[lane][r0 + q], cmul(e, cconj(vv[q])));
+  } else if (lane < n) {
+    if (lane < rows_t) axpy(&T[lane][r0], 1, cmul(tau, dot(&T[lane][r0], 1, false)), true);
+    axpy(&U[lane][r0], 1, cmul(tau, dot(&U[lane][r0], 1, false)), true);
   }
   wave_sync();
 }
@@ -963,7 +1118,10 @@ __device__ int aed(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz
         if (defl) {
           --ns;
         } else {
-          for (int k = j - 1; k >= ilst; --k) wave_swap(T, U, nw, k, lane);
+          if (nw <= 32)
+            wave_move_up(T, U, nw, j, ilst, lane);
+          else
+            for (int k = j - 1; k >= ilst; --k) wave_swap(T, U, nw, k, lane);
           ++ilst;
         }
       }
@@ -976,11 +1134,11 @@ __device__ int aed(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz
         if (ns > 1) {
           // reflect the spike s * conj(U[0][0..ns)) onto e1 (zlaqr3 "reflect spike back")
           cd w = lane < ns ? cconj(U[0][lane]) : mk(0.0, 0.0);
-          const double xn = sqrt(wsum(lane >= 1 && lane < ns ? cnorm2(w) : 0.0));
+          const double xn2 = wsum(lane >= 1 && lane < ns ? cnorm2(w) : 0.0);
           const cd alpha = cconj(U[0][0]);
           double beta;
           cd tau, scale;
-          house(alpha, xn, beta, tau, scale);
+          house_fast(alpha, xn2, beta, tau, scale);
           wave_sync();
           L.aedv[lane] = lane == 0 ? mk(1.0, 0.0) : (lane < ns ? cmul(w, scale) : mk(0.0, 0.0));
           wave_sync();
@@ -990,10 +1148,10 @@ __device__ int aed(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz
             const int len = ns - c - 1;
             const cd a0 = T[c + 1][c];
             const cd xv = (lane >= c + 2 && lane < ns) ? T[lane][c] : mk(0.0, 0.0);
-            const double xnc = sqrt(wsum(cnorm2(xv)));
+            const double xnc2 = wsum(cnorm2(xv));
             double bc;
             cd tc, sc;
-            house(a0, xnc, bc, tc, sc);
+            house_fast(a0, xnc2, bc, tc, sc);
             wave_sync();
             if (lane < len) L.aedv[lane] = lane == 0 ? mk(1.0, 0.0) : cmul(T[c + 1 + lane][c], sc);
             wave_sync();
@@ -1077,11 +1235,142 @@ __device__ int find_lo(QrLds<C::W, C::T>& L, cd* H, long ldh, int N, int hi) {
   return lo;
 }
 
-// One multishift sweep over the active block [lo, hi] with nbul bulges (shifts in L.shifts).
+// A bulge of the chase, owned by one wave for a whole window. The reflector (v1, v2, tau)
+// stays in the wave's registers between the row and the column operations of a step, and
+// the two columns of U that the next step touches again (u0, u1) stay there between steps:
+// the step then reads one column of U and writes one. LDS bandwidth bounds the chase (three
+// rows and three columns of the window read and written per bulge and step).
+struct Bulge {
+  cd v1, v2, tau;
+  cd u0, u1;
+};
+struct ChasePos {
+  int lo, hi, ws, w, t0, t1;
+};
+
+// The step's reflectors from the bulges' three entries (columns left of the bulge are zero)
+// applied to their rows, lane = column. Bulges NJ at once (b[m], index bb[m]), so that one's
+// dependency chain hides the other's; the rows of different bulges are disjoint, so the waves
+// need no barrier here.
+template <class C, int NJ>
+__device__ __forceinline__ void chase_rows(QrLds<C::W, C::T>& L, const ChasePos& cp, int tt, Bulge* const (&b)[NJ],
+                                           const int (&bb)[NJ], int lane) {
+  cd h1[NJ], h2[NJ], h3[NJ], e1[NJ], e2[NJ], e3[NJ];
+#pragma unroll
+  for (int m = 0; m < NJ; ++m) {
+    const int p = cp.lo - 1 + tt - 3 * bb[m];
+    const int r1 = p + 1 - cp.ws, r3 = r1 + (p + 3 <= cp.hi ? 2 : 1);
+    const int j0 = r1 > 0 ? r1 - 1 : 0, j = j0 + lane;
+    const int jc = j < cp.w ? j : cp.w - 1;
+    h1[m] = L.Hw[r1][jc];
+    h2[m] = L.Hw[r1 + 1][jc];
+    h3[m] = L.Hw[r3][jc];
+    e1[m] = L.Hw[r1][j0];
+    e2[m] = L.Hw[r1 + 1][j0];
+    e3[m] = L.Hw[r3][j0];
+  }
+#pragma unroll
+  for (int m = 0; m < NJ; ++m) {
+    const int p = cp.lo - 1 + tt - 3 * bb[m];
+    const bool three = p + 3 <= cp.hi, fresh = p == cp.lo - 1;
+    const int r1 = p + 1 - cp.ws;
+    const int j = (r1 > 0 ? r1 - 1 : 0) + lane;
+    cd x = e1[m], y = e2[m], z = e3[m];
+    if (fresh) {  // a new bulge: the first column of (H - s1)(H - s2); lane 0 holds column lo
+      const cd s1 = L.shifts[2 * bb[m]], s2 = L.shifts[2 * bb[m] + 1];
+      const cd h11 = x, h21 = y, h12 = lane_value(h1[m], 1), h22 = lane_value(h2[m], 1), h32 = lane_value(h3[m], 1);
+      const double sc = cabs1(csub(h11, s2)) + cabs1(h21);
+      if (sc == 0.0) {
+        x = y = z = mk(0.0, 0.0);
+      } else {
+        const cd h21s = cscale(h21, 1.0 / sc);
+        x = cadd(cmul(h21s, h12), cmul(csub(h11, s1), cscale(csub(h11, s2), 1.0 / sc)));
+        y = cmul(h21s, csub(cadd(h11, h22), cadd(s1, s2)));
+        z = cmul(h21s, h32);
+      }
+    }
+    if (!three) z = h3[m] = mk(0.0, 0.0);
+    double beta;
+    cd tau, scale;
+    house_small(x, y, z, beta, tau, scale);
+    const cd v1 = cmul(y, scale), v2 = cmul(z, scale);
+    b[m]->v1 = v1;
+    b[m]->v2 = v2;
+    b[m]->tau = tau;
+    const cd sm = cmul(cconj(tau), cadd(cadd(h1[m], cmulc(h2[m], v1)), cmulc(h3[m], v2)));
+    // the bulge's own column (absent for a new bulge) becomes (beta, 0, 0)
+    const bool own = !fresh && lane == 0;
+    const cd o1 = pick(own, mk(beta, 0.0), csub(h1[m], sm));
+    const cd o2 = pick(own, mk(0.0, 0.0), csub(h2[m], cmul(sm, v1)));
+    const cd o3 = pick(own, mk(0.0, 0.0), csub(h3[m], cmul(sm, v2)));
+    if (j < cp.w) {
+      L.Hw[r1][j] = o1;
+      L.Hw[r1 + 1][j] = o2;
+      if (three) L.Hw[r1 + 2][j] = o3;
+    }
+  }
+}
+
+// The same reflectors on the columns of the window (rows down to the bulge's last row + 1;
+// below it the columns hold exact zeros) and on those of U, lane = row.
+template <class C, int NJ>
+__device__ __forceinline__ void chase_cols(QrLds<C::W, C::T>& L, const ChasePos& cp, int tt, Bulge* const (&b)[NJ],
+                                           const int (&bb)[NJ], int lane) {
+  cd c1[NJ], c2[NJ], c3[NJ], u3[NJ];
+  const int row = lane < cp.w ? lane : cp.w - 1;
+#pragma unroll
+  for (int m = 0; m < NJ; ++m) {
+    const int p = cp.lo - 1 + tt - 3 * bb[m];
+    const int r1 = p + 1 - cp.ws, r3 = r1 + (p + 3 <= cp.hi ? 2 : 1);
+    c1[m] = L.Hw[row][r1];
+    c2[m] = L.Hw[row][r1 + 1];
+    c3[m] = L.Hw[row][r3];
+    u3[m] = L.U[row][r3];
+    if (tt == cp.t0 || p == cp.lo - 1) {  // the bulge's first step in this window
+      b[m]->u0 = L.U[row][r1];
+      b[m]->u1 = L.U[row][r1 + 1];
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < NJ; ++m) {
+    const int p = cp.lo - 1 + tt - 3 * bb[m];
+    const bool three = p + 3 <= cp.hi;
+    const int r1 = p + 1 - cp.ws;
+    const cd v1 = b[m]->v1, v2 = b[m]->v2, tau = b[m]->tau;
+    if (!three) c3[m] = u3[m] = mk(0.0, 0.0);
+    const cd sm = cmul(tau, cadd(cadd(c1[m], cmul(c2[m], v1)), cmul(c3[m], v2)));
+    const cd su = cmul(tau, cadd(cadd(b[m]->u0, cmul(b[m]->u1, v1)), cmul(u3[m], v2)));
+    const cd w0 = csub(b[m]->u0, su), w1 = csub(b[m]->u1, cmulc(su, v1)), w2 = csub(u3[m], cmulc(su, v2));
+    const cd o1 = csub(c1[m], sm), o2 = csub(c2[m], cmulc(sm, v1)), o3 = csub(c3[m], cmulc(sm, v2));
+    b[m]->u0 = w1;
+    b[m]->u1 = w2;
+    if (lane < cp.w) {
+      L.U[row][r1] = w0;
+      if (!three) {
+        L.U[row][r1 + 1] = w1;
+      } else if (tt == cp.t1 - 1) {  // leaving the window
+        L.U[row][r1 + 1] = w1;
+        L.U[row][r1 + 2] = w2;
+      }
+      if (lane <= r1 + 3) {
+        L.Hw[row][r1] = o1;
+        L.Hw[row][r1 + 1] = o2;
+        if (three) L.Hw[row][r1 + 2] = o3;
+      }
+    }
+  }
+}
+
+// One multishift sweep over the active block [lo, hi] with nbul bulges (shifts in L.shifts);
+// wave v owns the bulges v, v + T/64, ... A chase step has two barriers: after the rows and
+// after the columns.
 template <class C>
 __device__ void qr_sweep(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz, int lo, int hi, int nbul,
                          long long* st) {
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  constexpr int NW = C::T / 64;
+  constexpr int MB = ((C::W - 9) / 3 < NBUL ? (C::W - 9) / 3 : NBUL) / NW + 1 & ~1;  // bulges per wave, even
+  static_assert(MB * NW >= ((C::W - 9) / 3 < NBUL ? (C::W - 9) / 3 : NBUL), "every bulge has a wave");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int adv = C::W - 3 * nbul - 1;
   const int T_end = (hi - 2) - (lo - 1) + 3 * (nbul - 1) + 1;
   for (int t0 = 0; t0 < T_end; t0 += adv) {
@@ -1095,96 +1384,33 @@ __device__ void qr_sweep(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, lo
     const int w = we - ws + 1;
     const long long c0 = wall_clock64();
     lds_load_block<C>(L, H, ldh, ws, w);
+    const ChasePos cp = {lo, hi, ws, w, t0, t1};
+    Bulge bul[MB];
     for (int tt = t0; tt < t1; ++tt) {
-      // reflectors of all bulges at this step, from the current window state
-      if (t < nbul) {
-        const int bb = t;
-        const int p = lo - 1 + tt - 3 * bb;
-        int size = 0;
-        if (p >= lo - 1 && p <= hi - 2) {
-          cd x, y, z = mk(0.0, 0.0);
-          size = (p + 3 <= hi) ? 3 : 2;
-          if (p == lo - 1) {
-            const int a = lo - ws;
-            const cd s1 = L.shifts[2 * bb], s2 = L.shifts[2 * bb + 1];
-            const cd h11 = L.Hw[a][a], h21 = L.Hw[a + 1][a], h12 = L.Hw[a][a + 1];
-            const cd h22 = L.Hw[a + 1][a + 1];
-            const cd h32 = (size == 3) ? L.Hw[a + 2][a + 1] : mk(0.0, 0.0);
-            const double sc = cabs1(csub(h11, s2)) + cabs1(h21);
-            if (sc == 0.0) {
-              x = y = mk(0.0, 0.0);
-            } else {
-              const cd h21s = cscale(h21, 1.0 / sc);
-              x = cadd(cmul(h21s, h12), cmul(csub(h11, s1), cscale(csub(h11, s2), 1.0 / sc)));
-              y = cmul(h21s, csub(cadd(h11, h22), cadd(s1, s2)));
-              z = cmul(h21s, h32);
-            }
-            L.rcol[bb] = -1;
-          } else {
-            const int a = p - ws;
-            x = L.Hw[a + 1][a];
-            y = L.Hw[a + 2][a];
-            if (size == 3) z = L.Hw[a + 3][a];
-            L.rcol[bb] = a;
-          }
-          double beta;
-          cd tau, scale;
-          house_small(x, y, z, beta, tau, scale);
-          L.rv1[bb] = cmul(y, scale);
-          L.rv2[bb] = cmul(z, scale);
-          L.rtau[bb] = tau;
-          L.rbeta[bb] = beta;
-          L.rrow[bb] = p + 1 - ws;
-          if (tau.x == 0.0 && tau.y == 0.0) size = 0;
-        }
-        L.rsize[bb] = size;
+      // bulge bb is active when lo - 1 <= p <= hi - 2, p = lo - 1 + tt - 3 bb
+      auto active = [&](int bb) { return bb < nbul && tt >= 3 * bb && lo - 1 + tt - 3 * bb <= hi - 2; };
+#pragma unroll
+      for (int m = 0; m < MB; m += 2) {
+        const int b0 = wave + m * NW, b1 = b0 + NW;
+        const bool a0 = active(b0), a1 = active(b1);
+        if (a0 && a1)
+          chase_rows<C, 2>(L, cp, tt, {&bul[m], &bul[m + 1]}, {b0, b1}, lane);
+        else if (a0)
+          chase_rows<C, 1>(L, cp, tt, {&bul[m]}, {b0}, lane);
+        else if (a1)
+          chase_rows<C, 1>(L, cp, tt, {&bul[m + 1]}, {b1}, lane);
       }
       __syncthreads();
-      // row operations: wave v takes bulges v, v + T/64, ...; lane = column. Columns left
-      // of the bulge's own column hold exact zeros in its rows and are skipped.
-      for (int bb = wave; bb < nbul; bb += C::T / 64) {
-        const int sz = L.rsize[bb];
-        if (sz == 0) continue;
-        const int r1 = L.rrow[bb], rc = L.rcol[bb];
-        const int j = (r1 > 0 ? r1 - 1 : 0) + lane;
-        if (j >= w) continue;
-        if (j == rc) {
-          L.Hw[r1][j] = mk(L.rbeta[bb], 0.0);
-          L.Hw[r1 + 1][j] = mk(0.0, 0.0);
-          if (sz == 3) L.Hw[r1 + 2][j] = mk(0.0, 0.0);
-          continue;
-        }
-        const cd v1 = L.rv1[bb], v2 = L.rv2[bb], ct = cconj(L.rtau[bb]);
-        cd h1 = L.Hw[r1][j], h2 = L.Hw[r1 + 1][j];
-        cd h3 = sz == 3 ? L.Hw[r1 + 2][j] : mk(0.0, 0.0);
-        cd sm = cadd(h1, cmul(cconj(v1), h2));
-        if (sz == 3) sm = cadd(sm, cmul(cconj(v2), h3));
-        sm = cmul(ct, sm);
-        L.Hw[r1][j] = csub(h1, sm);
-        L.Hw[r1 + 1][j] = csub(h2, cmul(sm, v1));
-        if (sz == 3) L.Hw[r1 + 2][j] = csub(h3, cmul(sm, v2));
-      }
-      __syncthreads();
-      // column operations on the window (rows down to the bulge's last row + 1; below it
-      // the columns hold exact zeros) and on U (every row): pairs (matrix, bulge) over the
-      // waves, lane = row
-      for (int q = wave; q < 2 * nbul; q += C::T / 64) {
-        const int mat = q >= nbul ? 1 : 0, bb = q - mat * nbul;
-        const int sz = L.rsize[bb];
-        if (sz == 0) continue;
-        const int r1 = L.rrow[bb];
-        const int i = lane;
-        if (i >= w || (mat == 0 && i > r1 + 3)) continue;
-        auto& M = mat == 0 ? L.Hw : L.U;
-        const cd v1 = L.rv1[bb], v2 = L.rv2[bb], tu = L.rtau[bb];
-        cd c1 = M[i][r1], c2 = M[i][r1 + 1];
-        cd c3 = sz == 3 ? M[i][r1 + 2] : mk(0.0, 0.0);
-        cd sm = cadd(c1, cmul(c2, v1));
-        if (sz == 3) sm = cadd(sm, cmul(c3, v2));
-        sm = cmul(tu, sm);
-        M[i][r1] = csub(c1, sm);
-        M[i][r1 + 1] = csub(c2, cmul(sm, cconj(v1)));
-        if (sz == 3) M[i][r1 + 2] = csub(c3, cmul(sm, cconj(v2)));
+#pragma unroll
+      for (int m = 0; m < MB; m += 2) {
+        const int b0 = wave + m * NW, b1 = b0 + NW;
+        const bool a0 = active(b0), a1 = active(b1);
+        if (a0 && a1)
+          chase_cols<C, 2>(L, cp, tt, {&bul[m], &bul[m + 1]}, {b0, b1}, lane);
+        else if (a0)
+          chase_cols<C, 1>(L, cp, tt, {&bul[m]}, {b0}, lane);
+        else if (a1)
+          chase_cols<C, 1>(L, cp, tt, {&bul[m + 1]}, {b1}, lane);
       }
       __syncthreads();
     }
@@ -1286,7 +1512,7 @@ __device__ void hqr_body(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, long sH, 
         L.shifts[t] = cadd(hk, mk(0.75 * sub, 0.0));
       }
       __syncthreads();
-    } else if (nsa >= nbul) {
+    } else if (nsa >= 2) {
       // the undeflated window eigenvalues nearest the bottom serve as shifts
       if (nsa < ns) {
         nbul = nsa / 2 > 0 ? nsa / 2 : 1;
@@ -1576,11 +1802,11 @@ __global__ __launch_bounds__(256) void balance_kernel(int N, cd* A, long lda, lo
   }
 }
 
-static int g_aed_window = AED_NW;
+static int g_aed_window = -1;  // -1: automatic (aed_window_for)
 static int g_bulges = 12;
 static int g_max_sweeps = 0;  // 0: 30 * max(N, 10), LAPACK zlahqr's iteration budget
 void zgeev_set_max_sweeps(int n) { g_max_sweeps = n < 0 ? 0 : n; }
-void zgeev_set_aed(int window) { g_aed_window = window < 0 ? 0 : (window > QW ? QW : window); }
+void zgeev_set_aed(int window) { g_aed_window = window < -1 ? 0 : (window > QW ? QW : window); }
 void zgeev_set_bulges(int nb) { g_bulges = nb < 1 ? 1 : (nb > NBUL ? NBUL : nb); }
 // 0: hqr_kernel (W = 64, window products from registers), 1: hqr_lds_kernel (W = 64,
 // window products staged through LDS), 2: hqr_w48_kernel (W = 48, two matrices per CU),
@@ -1623,6 +1849,19 @@ std::vector<int> zgeev_launch_plan(int n, int units, int per_unit) {
   if (units % per) plan.push_back(units % per);
   return plan;
 }
+// Deflation window of QR kernel variant v at size n. The window's Schur form is the longest
+// serial part of a small problem, its deflations and shifts pay at large n. Measured best of
+// 6 .. 28 (QR stage, ms; in brackets the former fixed 24): 64-wide kernel N = 50 8: 2.1 (5.3),
+// N = 98 8: 6.3 (9.8), N = 126 12: 8.6, 8: 8.9, N = 162 16: 12.9, 12: 13.4, N = 242 16: 23.2
+// (25.3), N = 338 16 and 24: 42.5, N = 450 24: 75.5, 16: 81.9, N = 882 24: 305, 20: 319; 32-wide
+// kernel in full launches N = 98 8: 10.9 (17.6), N = 162 12: 27.7, 8: 29.3, N = 242 12: 61.1
+// (74.2), N = 450 12 and 16: 296; 48-wide kernel N = 882 20: 688, 24: 691.
+static int aed_window_for(int v, int n) {
+  if (g_aed_window >= 0) return g_aed_window;
+  if (v == 4) return n <= 128 ? 8 : 12;
+  if (v == 2) return 20;
+  return n <= 112 ? 8 : (n <= 144 ? 12 : (n <= 360 ? 16 : 24));
+}
 int zgeev_get_aed() { return g_aed_window; }
 int zgeev_get_bulges() { return g_bulges; }
 
@@ -1654,17 +1893,18 @@ void zgeev_factors(hipStream_t s, int n, cd* A, long lda, long sA, cd* w, long s
     long long* stp = want ? sb.as<long long>() : nullptr;
     const int qv = qr_variant_for(n, batch);
     g_qr_ran.fetch_or(1u << qv, std::memory_order_relaxed);
+    const int aed = aed_window_for(qv, n);
     if (qv == 4) {
-      hqr_w32_kernel<<<batch, 128, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, g_aed_window, g_bulges_w32,
+      hqr_w32_kernel<<<batch, 128, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, aed, g_bulges_w32,
                                            g_max_sweeps);
     } else if (qv == 2) {
-      hqr_w48_kernel<<<batch, 256, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp,
-                                           g_aed_window < 48 ? g_aed_window : 47, g_bulges_w48, g_max_sweeps);
+      hqr_w48_kernel<<<batch, 256, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, aed, g_bulges_w48,
+                                           g_max_sweeps);
     } else if (qv == 1) {
-      hqr_lds_kernel<<<batch, QT, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, g_aed_window, g_bulges,
+      hqr_lds_kernel<<<batch, QT, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, aed, g_bulges,
                                           g_max_sweeps);
     } else {
-      hqr_kernel<<<batch, QT, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, g_aed_window, g_bulges,
+      hqr_kernel<<<batch, QT, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, aed, g_bulges,
                                       g_max_sweeps);
     }
     launch_check("hqr");
