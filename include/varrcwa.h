@@ -58,10 +58,10 @@ const char* vrc_version(void);
  * pass) and resets. */
 int vrc_timing_enable(vrc_ctx* ctx, int on);
 /* Kernel tuning switches (process-wide; no reference counterpart). Keys:
- * "zgemm.large_tile" (default 1): 128x64-tile ZGEMM for m >= 128, n >= 64, else the
- * 64x64 tile; "zgemm.large_tile_min_k" (default 129): smallest k for the 128x64 tile;
- * "zgemm.big_waves", "zgemm.small_waves" (default 8, or 4): wavefronts per workgroup of the
- * 128x64 and 64x64 tiles; "zgemm.big_n" (default 128, or 64): a 128x128 tile for n >= 128; "zgeev.aed_window" (default -1 = chosen by N and QR kernel, 0 = off, at most 64): deflation-window
+ * "zgemm.small_waves" (default 8, or 4): wavefronts per workgroup of the 64x64-tile ZGEMM
+ * ("zgemm.large_tile", "zgemm.large_tile_min_k", "zgemm.big_waves" and "zgemm.big_n", switches of
+ * larger tiles that are gone, are accepted without effect);
+ * "zgeev.aed_window" (default -1 = chosen by N and QR kernel, 0 = off, at most 64): deflation-window
  * size of the aggressive early deflation in the QR iteration; "zgeev.bulges" (default 12,
  * 1..16): double-shift bulges chased per QR sweep; "rcwa.group" (default 64): slices of
  * RCWAIntegrator::compute solved per eigensolve launch (1: one slice at a time, as the

@@ -36,6 +36,25 @@ def test_zgemm_ops(ctx, opA, opB):
     assert np.abs(got - ref).max() <= 1e-13 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("opA,opB", [(0, 0), (2, 0), (0, 2), (1, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [(1, 1, 1, 1), (16, 17, 15, 2), (31, 33, 32, 3), (33, 64, 65, 1),
+                                         (97, 49, 31, 40), (65, 81, 16, 130), (98, 98, 33, 300)])
+def test_zgemm_tile_edges(ctx, opA, opB, m, n, k, batch):
+    """Both ZGEMM tiles at the edges of their 16x16 blocks, of their K chunks (16, 32) and of
+    the rule that picks one (few workgroups: 32x32, many: 64x64), NaN in C with beta = 0."""
+    import torch
+    rng = np.random.default_rng(m + 100 * n + k)
+    A = crand(rng, batch, *((m, k) if opA == 0 else (k, m)))
+    B = crand(rng, batch, *((k, n) if opB == 0 else (n, k)))
+    dA, dB = to_dev_colmajor(A), to_dev_colmajor(B)
+    dC = torch.full((batch, n, m), float("nan"), dtype=torch.complex128, device="cuda")
+    ctx.check(ctx.lib.vrc_zgemm(ctx.h, opA, opB, m, n, k, cplx(1), ptr(dA), A.shape[1], A.shape[1] * A.shape[2],
+                                ptr(dB), B.shape[1], B.shape[1] * B.shape[2], cplx(0), ptr(dC), m, m * n, batch),
+              "zgemm")
+    ref = opm(A, opA) @ opm(B, opB)
+    assert np.abs(from_dev_colmajor(dC) - ref).max() <= 1e-13 * np.abs(ref).max()
+
+
 def test_zgemm_large_and_beta0(ctx):
     rng = np.random.default_rng(1)
     m = n = k = 300

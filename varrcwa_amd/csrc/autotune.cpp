@@ -30,7 +30,7 @@ TuneKnobs tune_get() {
   k.qr_variant = zgeev_get_qr_variant();
   k.bulges_w48 = zgeev_get_bulges_w48();
   k.bulges_w32 = zgeev_get_bulges_w32();
-  zgemm_get_knobs(&k.big_n, &k.big_waves, &k.small_waves, &k.big_min_k);
+  k.small_waves = zgemm_get_small_waves();
   return k;
 }
 
@@ -40,10 +40,7 @@ void tune_put(const TuneKnobs& k) {
   zgeev_set_qr_variant(k.qr_variant);
   zgeev_set_bulges_w48(k.bulges_w48);
   zgeev_set_bulges_w32(k.bulges_w32);
-  zgemm_set_big_n(k.big_n);
-  zgemm_set_big_waves(k.big_waves);
   zgemm_set_small_waves(k.small_waves);
-  zgemm_set_big_min_k(k.big_min_k);
 }
 
 void tune_apply(int N) {
@@ -72,10 +69,8 @@ void tune_manual_begin() {
 static std::string knobs_text(const TuneKnobs& k) {
   char b[256];
   snprintf(b, sizeof(b),
-           "qr_variant %d aed_window %d bulges %d bulges_w48 %d bulges_w32 %d big_n %d big_waves %d small_waves %d "
-           "large_tile_min_k %d",
-           k.qr_variant, k.aed, k.bulges, k.bulges_w48, k.bulges_w32, k.big_n, k.big_waves, k.small_waves,
-           k.big_min_k);
+           "qr_variant %d aed_window %d bulges %d bulges_w48 %d bulges_w32 %d small_waves %d", k.qr_variant, k.aed,
+           k.bulges, k.bulges_w48, k.bulges_w32, k.small_waves);
   return b;
 }
 
@@ -91,8 +86,9 @@ void tune_clear() {
   g_table.clear();
 }
 
-// Cache file: one line per N, "N aed bulges big_n big_waves small_waves big_min_k
-// [qr_variant [bulges_w48 bulges_w32]]" (without qr_variant the QR kernel is left to the
+// Cache file: one line per N, "N aed bulges - - small_waves - [qr_variant [bulges_w48
+// bulges_w32]]" (the three fields marked - held switches of ZGEMM tiles that are gone: read
+// and ignored, written as 0; without qr_variant the QR kernel is left to the
 // automatic choice, -1; without the last two the bulge counts of QR variants 2 and 4 are
 // their defaults, 8 and 6); lines starting with '#' are comments. Later lines for the same
 // N win.
@@ -100,8 +96,7 @@ void tune_save(const std::string& path, int N, const TuneKnobs& k, const std::st
   std::ofstream f(path, std::ios::app);
   if (!f) throw ArgFailure("cannot append to the tuning cache " + path);
   f << "# " << note << "\n"
-    << N << " " << k.aed << " " << k.bulges << " " << k.big_n << " " << k.big_waves << " " << k.small_waves << " "
-    << k.big_min_k << " " << k.qr_variant << " " << k.bulges_w48 << " " << k.bulges_w32 << "\n";
+    << N << " " << k.aed << " " << k.bulges << " 0 0 " << k.small_waves << " 0 " << k.qr_variant << " " << k.bulges_w48 << " " << k.bulges_w32 << "\n";
 }
 
 int tune_load(const std::string& path) {
@@ -114,7 +109,8 @@ int tune_load(const std::string& path) {
     std::istringstream is(line);
     int N;
     TuneKnobs k{};
-    if (!(is >> N >> k.aed >> k.bulges >> k.big_n >> k.big_waves >> k.small_waves >> k.big_min_k) || N < 2)
+    int gone[3];
+    if (!(is >> N >> k.aed >> k.bulges >> gone[0] >> gone[1] >> k.small_waves >> gone[2]) || N < 2)
       throw ArgFailure("malformed tuning cache line: " + line);
     k.qr_variant = -1;
     k.bulges_w48 = 8;
@@ -203,10 +199,7 @@ std::string autotune_stack(vrc_ctx& c, int nx, int ny, const std::vector<StackIn
         {&TuneKnobs::bulges, {6, 8, 10, 12, 14, 16}, QR_W64},
         {&TuneKnobs::bulges_w48, {4, 6, 8, 10, 12}, QR_W48},
         {&TuneKnobs::bulges_w32, {3, 4, 5, 6, 7}, QR_W32},
-        {&TuneKnobs::big_n, {64, 128}, QR_ANY},
-        {&TuneKnobs::big_waves, {4, 8}, QR_ANY},
-        {&TuneKnobs::small_waves, {4, 8}, QR_ANY},
-        {&TuneKnobs::big_min_k, {33, 65, 129}, QR_ANY}};
+        {&TuneKnobs::small_waves, {4, 8}, QR_ANY}};
     bool out_of_time = false;
     for (const Switch& sw : space) {
       if (sw.kernels != QR_ANY && !(sw.kernels & ran_best)) continue;

@@ -1,10 +1,11 @@
 // Complex128 dense kernels for gfx950: FP64-MFMA ZGEMM (strided and descriptor
 // batched) and the elementwise matrix kernels used between the factorizations.
 //
-// ZGEMM tiles: 64x64 and 128x64 output per workgroup (8 wavefronts by default; 4-wave
-// variants selectable) from v_mfma_f64_16x16x4f64 blocks, K staged through LDS in
-// chunks of 16 complex values, real and imaginary planes kept separate so that one
-// complex multiply-add is four real MFMAs (standard 4M product, no 3M/Gauss trick).
+// ZGEMM tiles: 64x64 output per workgroup (8 wavefronts by default; a 4-wave variant
+// selectable), or 32x32 where few tiles would leave CUs idle, from v_mfma_f64_16x16x4f64
+// blocks, K staged through LDS in chunks of 16 (32) complex values, real and imaginary planes
+// kept separate so that one complex multiply-add is four real MFMAs (standard 4M product, no
+// 3M/Gauss trick).
 #include "vrc_common.hpp"
 #include "vrc_internal.hpp"
 
@@ -245,422 +246,90 @@ __device__ __forceinline__ void zgemm_tile8(int m, int n, int k, cd alpha, const
     }
 }
 
-// ---------------------------------------------------------------- large-tile ZGEMM
-// 128x64 output per 256-thread workgroup: 2x2 wavefronts, each 64x32 = 4x2 blocks of
-// v_mfma_f64_16x16x4f64 (re and im accumulators: 128 registers). K in chunks of 16;
-// the next chunk is fetched from memory into registers while the current one is
-// multiplied out of LDS. LDS rows are padded by one double so that both the staging
-// stores (along m or along k) and the MFMA operand reads are free of bank conflicts.
-constexpr int GB_M = 128, GB_N = 64, GB_K = 16;
+// 32x32 output per 256-thread workgroup (four waves, one 16x16 block each) with K in chunks of
+// 32, for products whose larger tiles would leave most CUs without a workgroup (single
+// matrices and short right-hand sides): latency-bound there, so the tile is small, a barrier
+// covers 32 k, and the four real products go to four accumulators (no dependent MFMA pairs).
+constexpr int GS_T = 32, GS_K = 32, GS_THREADS = 256;
 
 template <int OPA, int OPB>
-__device__ __forceinline__ void zgemm_tile_big(int m, int n, int k, cd alpha, const cd* __restrict__ A, long lda,
-                                               const cd* __restrict__ B, long ldb, cd beta, cd* __restrict__ C,
-                                               long ldc, int tm, int tn) {
-  __shared__ double As_re[GB_K][GB_M + 1];
-  __shared__ double As_im[GB_K][GB_M + 1];
-  __shared__ double Bs_re[GB_K][GB_N + 1];
-  __shared__ double Bs_im[GB_K][GB_N + 1];
+__device__ __forceinline__ void zgemm_tile32(int m, int n, int k, cd alpha, const cd* __restrict__ A, long lda,
+                                             const cd* __restrict__ B, long ldb, cd beta, cd* __restrict__ C, long ldc,
+                                             int tm, int tn) {
+  __shared__ double As_re[GS_K][GS_T + 1];
+  __shared__ double As_im[GS_K][GS_T + 1];
+  __shared__ double Bs_re[GS_K][GS_T + 1];
+  __shared__ double Bs_im[GS_K][GS_T + 1];
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = t >> 6;
   const int wr = wave >> 1, wc = wave & 1;
-  const int row0 = tm * GB_M, col0 = tn * GB_N;
-
-  d4 accR[4][2], accI[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      accR[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-      accI[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-    }
-  // element e = t + 256*i of the A tile (8 per thread) and of the B tile (4 per thread)
-  auto a_coord = [&](int e, int& r, int& c) {
-    if (OPA == OP_N) { r = e & 127; c = e >> 7; } else { c = e & 15; r = e >> 4; }
-  };
-  auto b_coord = [&](int e, int& c, int& j) {
-    if (OPB == OP_N) { c = e & 15; j = e >> 4; } else { j = e & 63; c = e >> 6; }
-  };
-  cd ra[8], rb[4];
+  const int row0 = tm * GS_T, col0 = tn * GS_T;
+  const bool live = __builtin_amdgcn_readfirstlane(row0 + wr * 16 < m && col0 + wc * 16 < n);
+  d4 rr = d4{0.0, 0.0, 0.0, 0.0}, ii = rr, ri = rr, ir = rr;
+  // element q of this thread: (x, y) = (t & 31, (t >> 5) + 8 q), x along the operand's columns
+  const int x = t & 31, y = t >> 5;
+  cd pa[4], pb[4];
   auto fetch = [&](int kk) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      int r, c;
-      a_coord(t + 256 * i, r, c);
-      const int gr = row0 + r, gc = kk + c;
+    for (int q = 0; q < 4; ++q) {
+      const int yy = y + 8 * q;
       cd v = mk(0.0, 0.0);
-      if (gr < m && gc < k) v = (OPA == OP_N) ? A[gr + (long)gc * lda] : A[gc + (long)gr * lda];
-      if (OPA == OP_C) v.y = -v.y;
-      ra[i] = v;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int c, j;
-      b_coord(t + 256 * i, c, j);
-      const int gc = kk + c, gj = col0 + j;
-      cd v = mk(0.0, 0.0);
-      if (gc < k && gj < n) v = (OPB == OP_N) ? B[gc + (long)gj * ldb] : B[gj + (long)gc * ldb];
-      if (OPB == OP_C) v.y = -v.y;
-      rb[i] = v;
-    }
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      int r, c;
-      a_coord(t + 256 * i, r, c);
-      As_re[c][r] = ra[i].x;
-      As_im[c][r] = ra[i].y;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int c, j;
-      b_coord(t + 256 * i, c, j);
-      Bs_re[c][j] = rb[i].x;
-      Bs_im[c][j] = rb[i].y;
+      if (OPA == OP_N) {
+        if (row0 + x < m && kk + yy < k) v = A[(row0 + x) + (long)(kk + yy) * lda];
+      } else {
+        if (row0 + yy < m && kk + x < k) v = A[(kk + x) + (long)(row0 + yy) * lda];
+        if (OPA == OP_C) v.y = -v.y;
+      }
+      pa[q] = v;
+      v = mk(0.0, 0.0);
+      if (OPB == OP_N) {
+        if (kk + x < k && col0 + yy < n) v = B[(kk + x) + (long)(col0 + yy) * ldb];
+      } else {
+        if (kk + yy < k && col0 + x < n) v = B[(col0 + x) + (long)(kk + yy) * ldb];
+        if (OPB == OP_C) v.y = -v.y;
+      }
+      pb[q] = v;
     }
   };
   fetch(0);
-  for (int kk = 0; kk < k; kk += GB_K) {
-    stash();
+  for (int kk = 0; kk < k; kk += GS_K) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int yy = y + 8 * q;
+      (OPA == OP_N ? As_re[yy][x] : As_re[x][yy]) = pa[q].x;
+      (OPA == OP_N ? As_im[yy][x] : As_im[x][yy]) = pa[q].y;
+      (OPB == OP_N ? Bs_re[x][yy] : Bs_re[yy][x]) = pb[q].x;
+      (OPB == OP_N ? Bs_im[x][yy] : Bs_im[yy][x]) = pb[q].y;
+    }
     __syncthreads();
-    if (kk + GB_K < k) fetch(kk + GB_K);
+    if (kk + GS_K < k) fetch(kk + GS_K);
+    if (live) {
 #pragma unroll
-    for (int s = 0; s < GB_K / 4; ++s) {
-      const int kr = s * 4 + (lane >> 4);
-      double ar[4], ai[4], nai[4], br[2], bi[2];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        ar[b] = As_re[kr][wr * 64 + b * 16 + (lane & 15)];
-        ai[b] = As_im[kr][wr * 64 + b * 16 + (lane & 15)];
-        nai[b] = -ai[b];
+      for (int s = 0; s < GS_K / 4; ++s) {
+        const int kr = s * 4 + (lane >> 4);
+        const double ar = As_re[kr][wr * 16 + (lane & 15)], ai = As_im[kr][wr * 16 + (lane & 15)];
+        const double br = Bs_re[kr][wc * 16 + (lane & 15)], bi = Bs_im[kr][wc * 16 + (lane & 15)];
+        rr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, rr, 0, 0, 0);
+        ii = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, ii, 0, 0, 0);
+        ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, ri, 0, 0, 0);
+        ir = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, ir, 0, 0, 0);
       }
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        br[b] = Bs_re[kr][wc * 32 + b * 16 + (lane & 15)];
-        bi[b] = Bs_im[kr][wc * 32 + b * 16 + (lane & 15)];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], br[j], accR[i][j], 0, 0, 0);
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai[i], bi[j], accR[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], bi[j], accI[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], br[j], accI[i][j], 0, 0, 0);
-        }
     }
     __syncthreads();
   }
   const bool beta0 = (beta.x == 0.0 && beta.y == 0.0);
+  const int gc = col0 + wc * 16 + (lane & 15);
+  if (gc >= n) return;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int gc = col0 + wc * 32 + j * 16 + (lane & 15);
-      if (gc >= n) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gr = row0 + wr * 64 + i * 16 + (lane >> 4) + 4 * r;
-        if (gr >= m) continue;
-        cd out = cmul(alpha, mk(accR[i][j][r], accI[i][j][r]));
-        cd* cp = C + gr + (long)gc * ldc;
-        if (!beta0) out = cadd(out, cmul(beta, *cp));
-        *cp = out;
-      }
-    }
-}
-
-// The 128x64 tile on eight waves (512 threads): wave w owns rows 32*(w>>1) .. +32 and
-// columns 32*(w&1) .. +32 (2x2 blocks of 16x16); the K chunk is staged as above.
-constexpr int GB8_THREADS = 512;
-
-template <int OPA, int OPB>
-__device__ __forceinline__ void zgemm_tile_big8(int m, int n, int k, cd alpha, const cd* __restrict__ A, long lda,
-                                                const cd* __restrict__ B, long ldb, cd beta, cd* __restrict__ C,
-                                                long ldc, int tm, int tn) {
-  __shared__ double As_re[GB_K][GB_M + 1];
-  __shared__ double As_im[GB_K][GB_M + 1];
-  __shared__ double Bs_re[GB_K][GB_N + 1];
-  __shared__ double Bs_im[GB_K][GB_N + 1];
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int wr = wave >> 1, wc = wave & 1;
-  const int row0 = tm * GB_M, col0 = tn * GB_N;
-
-  d4 accR[2][2], accI[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      accR[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-      accI[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-    }
-  // element e = t + 512*i of the A tile (4 per thread) and of the B tile (2 per thread)
-  auto a_coord = [&](int e, int& r, int& c) {
-    if (OPA == OP_N) { r = e & 127; c = e >> 7; } else { c = e & 15; r = e >> 4; }
-  };
-  auto b_coord = [&](int e, int& c, int& j) {
-    if (OPB == OP_N) { c = e & 15; j = e >> 4; } else { j = e & 63; c = e >> 6; }
-  };
-  cd ra[4], rb[2];
-  auto fetch = [&](int kk) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int r, c;
-      a_coord(t + GB8_THREADS * i, r, c);
-      const int gr = row0 + r, gc = kk + c;
-      cd v = mk(0.0, 0.0);
-      if (gr < m && gc < k) v = (OPA == OP_N) ? A[gr + (long)gc * lda] : A[gc + (long)gr * lda];
-      if (OPA == OP_C) v.y = -v.y;
-      ra[i] = v;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      int c, j;
-      b_coord(t + GB8_THREADS * i, c, j);
-      const int gc = kk + c, gj = col0 + j;
-      cd v = mk(0.0, 0.0);
-      if (gc < k && gj < n) v = (OPB == OP_N) ? B[gc + (long)gj * ldb] : B[gj + (long)gc * ldb];
-      if (OPB == OP_C) v.y = -v.y;
-      rb[i] = v;
-    }
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int r, c;
-      a_coord(t + GB8_THREADS * i, r, c);
-      As_re[c][r] = ra[i].x;
-      As_im[c][r] = ra[i].y;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      int c, j;
-      b_coord(t + GB8_THREADS * i, c, j);
-      Bs_re[c][j] = rb[i].x;
-      Bs_im[c][j] = rb[i].y;
-    }
-  };
-  fetch(0);
-  for (int kk = 0; kk < k; kk += GB_K) {
-    stash();
-    __syncthreads();
-    if (kk + GB_K < k) fetch(kk + GB_K);
-#pragma unroll
-    for (int s = 0; s < GB_K / 4; ++s) {
-      const int kr = s * 4 + (lane >> 4);
-      double ar[2], ai[2], nai[2], br[2], bi[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        ar[b] = As_re[kr][wr * 32 + b * 16 + (lane & 15)];
-        ai[b] = As_im[kr][wr * 32 + b * 16 + (lane & 15)];
-        nai[b] = -ai[b];
-        br[b] = Bs_re[kr][wc * 32 + b * 16 + (lane & 15)];
-        bi[b] = Bs_im[kr][wc * 32 + b * 16 + (lane & 15)];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], br[j], accR[i][j], 0, 0, 0);
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai[i], bi[j], accR[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], bi[j], accI[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], br[j], accI[i][j], 0, 0, 0);
-        }
-    }
-    __syncthreads();
+  for (int r = 0; r < 4; ++r) {
+    const int gr = row0 + wr * 16 + (lane >> 4) + 4 * r;
+    if (gr >= m) continue;
+    cd out = cmul(alpha, mk(rr[r] - ii[r], ri[r] + ir[r]));
+    cd* cp = C + gr + (long)gc * ldc;
+    if (!beta0) out = cadd(out, cmul(beta, *cp));
+    *cp = out;
   }
-  const bool beta0 = (beta.x == 0.0 && beta.y == 0.0);
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int gc = col0 + wc * 32 + j * 16 + (lane & 15);
-      if (gc >= n) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gr = row0 + wr * 32 + i * 16 + (lane >> 4) + 4 * r;
-        if (gr >= m) continue;
-        cd out = cmul(alpha, mk(accR[i][j][r], accI[i][j][r]));
-        cd* cp = C + gr + (long)gc * ldc;
-        if (!beta0) out = cadd(out, cmul(beta, *cp));
-        *cp = out;
-      }
-    }
-}
-
-// 128x128 tile on eight waves: wave w owns rows 64*(w>>2) .. +64 and columns 32*(w&3) .. +32
-// (4x2 blocks of 16x16); K chunk of 16 staged through LDS as above.
-constexpr int GQ_N = 128;
-
-template <int OPA, int OPB>
-__device__ __forceinline__ void zgemm_tile_sq(int m, int n, int k, cd alpha, const cd* __restrict__ A, long lda,
-                                              const cd* __restrict__ B, long ldb, cd beta, cd* __restrict__ C,
-                                              long ldc, int tm, int tn) {
-  __shared__ double As_re[GB_K][GB_M + 1];
-  __shared__ double As_im[GB_K][GB_M + 1];
-  __shared__ double Bs_re[GB_K][GQ_N + 1];
-  __shared__ double Bs_im[GB_K][GQ_N + 1];
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int wr = wave >> 2, wc = wave & 3;
-  const int row0 = tm * GB_M, col0 = tn * GQ_N;
-  d4 accR[4][2], accI[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      accR[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-      accI[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-    }
-  // element e = t + 512*i of the A tile (4 per thread) and of the B tile (4 per thread)
-  auto a_coord = [&](int e, int& r, int& c) {
-    if (OPA == OP_N) { r = e & 127; c = e >> 7; } else { c = e & 15; r = e >> 4; }
-  };
-  auto b_coord = [&](int e, int& c, int& j) {
-    if (OPB == OP_N) { c = e & 15; j = e >> 4; } else { j = e & 127; c = e >> 7; }
-  };
-  cd ra[4], rb[4];
-  auto fetch = [&](int kk) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int r, c;
-      a_coord(t + GB8_THREADS * i, r, c);
-      const int gr = row0 + r, gc = kk + c;
-      cd v = mk(0.0, 0.0);
-      if (gr < m && gc < k) v = (OPA == OP_N) ? A[gr + (long)gc * lda] : A[gc + (long)gr * lda];
-      if (OPA == OP_C) v.y = -v.y;
-      ra[i] = v;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int c, j;
-      b_coord(t + GB8_THREADS * i, c, j);
-      const int gc = kk + c, gj = col0 + j;
-      cd v = mk(0.0, 0.0);
-      if (gc < k && gj < n) v = (OPB == OP_N) ? B[gc + (long)gj * ldb] : B[gj + (long)gc * ldb];
-      if (OPB == OP_C) v.y = -v.y;
-      rb[i] = v;
-    }
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int r, c;
-      a_coord(t + GB8_THREADS * i, r, c);
-      As_re[c][r] = ra[i].x;
-      As_im[c][r] = ra[i].y;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int c, j;
-      b_coord(t + GB8_THREADS * i, c, j);
-      Bs_re[c][j] = rb[i].x;
-      Bs_im[c][j] = rb[i].y;
-    }
-  };
-  fetch(0);
-  for (int kk = 0; kk < k; kk += GB_K) {
-    stash();
-    __syncthreads();
-    if (kk + GB_K < k) fetch(kk + GB_K);
-#pragma unroll
-    for (int s = 0; s < GB_K / 4; ++s) {
-      const int kr = s * 4 + (lane >> 4);
-      double ar[4], ai[4], nai[4], br[2], bi[2];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        ar[b] = As_re[kr][wr * 64 + b * 16 + (lane & 15)];
-        ai[b] = As_im[kr][wr * 64 + b * 16 + (lane & 15)];
-        nai[b] = -ai[b];
-      }
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        br[b] = Bs_re[kr][wc * 32 + b * 16 + (lane & 15)];
-        bi[b] = Bs_im[kr][wc * 32 + b * 16 + (lane & 15)];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], br[j], accR[i][j], 0, 0, 0);
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai[i], bi[j], accR[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], bi[j], accI[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], br[j], accI[i][j], 0, 0, 0);
-        }
-    }
-    __syncthreads();
-  }
-  const bool beta0 = (beta.x == 0.0 && beta.y == 0.0);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int gc = col0 + wc * 32 + j * 16 + (lane & 15);
-      if (gc >= n) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gr = row0 + wr * 64 + i * 16 + (lane >> 4) + 4 * r;
-        if (gr >= m) continue;
-        cd out = cmul(alpha, mk(accR[i][j][r], accI[i][j][r]));
-        cd* cp = C + gr + (long)gc * ldc;
-        if (!beta0) out = cadd(out, cmul(beta, *cp));
-        *cp = out;
-      }
-    }
-}
-
-// 1-D grid over (batch, n tile, m tile) with m tiles fastest. Workgroup ids are dealt
-// to the 8 XCDs round-robin; the id is remapped so that every XCD works on one
-// contiguous range of tiles (tiles of the same matrices share that XCD's L2).
-template <int OPA, int OPB>
-__global__ __launch_bounds__(GT_THREADS) void zgemm_big_kernel(int m, int n, int k, cd alpha, const cd* A, long lda,
-                                                               long sA, const cd* B, long ldb, long sB, cd beta,
-                                                               cd* C, long ldc, long sC, int gm, int gn, long total) {
-  const long id = blockIdx.x;
-  const long q = total / 8, rr = total % 8;
-  const long x = id % 8, slot = id / 8;
-  const long logical = x * q + (x < rr ? x : rr) + slot;
-  const long per = (long)gm * gn;
-  const long b = logical / per;
-  const int rem = (int)(logical - b * per);
-  const int tn = rem / gm, tm = rem - tn * gm;
-  zgemm_tile_big<OPA, OPB>(m, n, k, alpha, A + b * sA, lda, B + b * sB, ldb, beta, C + b * sC, ldc, tm, tn);
-}
-
-template <int OPA, int OPB>
-__global__ __launch_bounds__(GB8_THREADS) void zgemm_big8_kernel(int m, int n, int k, cd alpha, const cd* A, long lda,
-                                                                 long sA, const cd* B, long ldb, long sB, cd beta,
-                                                                 cd* C, long ldc, long sC, int gm, int gn,
-                                                                 long total) {
-  const long id = blockIdx.x;
-  const long q = total / 8, rr = total % 8;
-  const long x = id % 8, slot = id / 8;
-  const long logical = x * q + (x < rr ? x : rr) + slot;
-  const long per = (long)gm * gn;
-  const long b = logical / per;
-  const int rem = (int)(logical - b * per);
-  const int tn = rem / gm, tm = rem - tn * gm;
-  zgemm_tile_big8<OPA, OPB>(m, n, k, alpha, A + b * sA, lda, B + b * sB, ldb, beta, C + b * sC, ldc, tm, tn);
-}
-
-template <int OPA, int OPB>
-__global__ __launch_bounds__(GB8_THREADS) void zgemm_sq_kernel(int m, int n, int k, cd alpha, const cd* A, long lda,
-                                                               long sA, const cd* B, long ldb, long sB, cd beta,
-                                                               cd* C, long ldc, long sC, int gm, int gn, long total) {
-  const long id = blockIdx.x;
-  const long q = total / 8, rr = total % 8;
-  const long x = id % 8, slot = id / 8;
-  const long logical = x * q + (x < rr ? x : rr) + slot;
-  const long per = (long)gm * gn;
-  const long b = logical / per;
-  const int rem = (int)(logical - b * per);
-  const int tn = rem / gm, tm = rem - tn * gm;
-  zgemm_tile_sq<OPA, OPB>(m, n, k, alpha, A + b * sA, lda, B + b * sB, ldb, beta, C + b * sC, ldc, tm, tn);
 }
 
 // Scale-only path for k == 0 (C = beta*C), shared by both batch modes.
@@ -689,13 +358,24 @@ __global__ __launch_bounds__(GT_THREADS) void zgemm_strided_kernel(int m, int n,
   zgemm_tile<OPA, OPB>(m, n, k, alpha, A + b * sA, lda, B + b * sB, ldb, beta, C + b * sC, ldc, tm, tn);
 }
 
+// Transposed operands: six waves per SIMD (80 registers) measured 63.2 TFLOP/s at 250 x 882^3 (C,
+// N) against 59.9; plain operands run best as the compiler allocates them (64.8 against 63.4).
 template <int OPA, int OPB>
-__global__ __launch_bounds__(512) void zgemm_strided8_kernel(int m, int n, int k, cd alpha, const cd* A, long lda,
+__global__ __launch_bounds__(512, OPA == OP_N && OPB == OP_N ? 1 : 6) void zgemm_strided8_kernel(int m, int n, int k, cd alpha, const cd* A, long lda,
                                                             long sA, const cd* B, long ldb, long sB, cd beta, cd* C,
                                                             long ldc, long sC) {
   const int tm = blockIdx.x, tn = blockIdx.y;
   const long b = blockIdx.z;
   zgemm_tile8<OPA, OPB>(m, n, k, alpha, A + b * sA, lda, B + b * sB, ldb, beta, C + b * sC, ldc, tm, tn);
+}
+
+template <int OPA, int OPB>
+__global__ __launch_bounds__(GS_THREADS) void zgemm_small_kernel(int m, int n, int k, cd alpha, const cd* A, long lda,
+                                                                long sA, const cd* B, long ldb, long sB, cd beta,
+                                                                cd* C, long ldc, long sC) {
+  const int tm = blockIdx.x, tn = blockIdx.y;
+  const long b = blockIdx.z;
+  zgemm_tile32<OPA, OPB>(m, n, k, alpha, A + b * sA, lda, B + b * sB, ldb, beta, C + b * sC, ldc, tm, tn);
 }
 
 template <int OPA, int OPB>
@@ -711,71 +391,47 @@ __global__ __launch_bounds__(GT_THREADS) void zgemm_desc_kernel(const GemmDesc* 
   zgemm_tile<OPA, OPB>(d.m, d.n, d.k, d.alpha, d.A, d.lda, d.B, d.ldb, d.beta, d.C, d.ldc, tm, tn);
 }
 
-static bool g_big_gemm = true;  // large-tile kernel for m >= 128, n >= 64 (switchable for comparison)
-static int g_big_waves = 8;     // wavefronts of the large-tile kernel (4 or 8)
-void zgemm_set_big_waves(int w) { g_big_waves = w == 8 ? 8 : 4; }
 static int g_small_waves = 8;   // wavefronts of the 64x64-tile kernel (4 or 8)
-static int g_big_n = 128;       // columns of the large tile (128 for n >= 128, else 64)
-void zgemm_set_big_n(int nn) { g_big_n = nn == 128 ? 128 : 64; }
 void zgemm_set_small_waves(int w) { g_small_waves = w == 8 ? 8 : 4; }
-static int g_big_min_k = 129;   // ... and k at least this (short-k updates run better on the 64x64 tile)
-void zgemm_set_big(bool on) { g_big_gemm = on; }
-void zgemm_set_big_min_k(int k) { g_big_min_k = k; }
-void zgemm_get_knobs(int* big_n, int* big_waves, int* small_waves, int* big_min_k) {
-  *big_n = g_big_n;
-  *big_waves = g_big_waves;
-  *small_waves = g_small_waves;
-  *big_min_k = g_big_min_k;
+int zgemm_get_small_waves() { return g_small_waves; }
+
+// 32x32 instead of 64x64 tiles? A 64x64 workgroup takes about 0.14 us per unit of k, a 32x32 one
+// 0.054 us, one per CU at a time either way while workgroups are few, so the smaller tile wins
+// while its rounds over the 256 CUs cost less (single matrices and short right-hand sides;
+// us with 64 / 32: 162^3 26 / 12, 450^3 65 / 27, 882^3 126 / 141, 64 x 484 x 64 12 / 6, 16
+// products of 242^3 43 / 54), or where 64 fits the edges so badly that 32 saves a third of the
+// tiles (256 products 81 x 81 x 128: 74 / 56). Tiles of 128x64 and 128x128 were slower than 64x64
+// at every size measured (N = 242 .. 1250, batches of 1 .. 2000; 250 products of 882^3: 22.2 ms
+// against 21.3) and are gone.
+static bool zgemm_use_32(int m, int n, int k, int batch) {
+  const long n64 = (long)cdiv_up(m, GT_M) * cdiv_up(n, GT_N) * batch;
+  const long n32 = (long)cdiv_up(m, GS_T) * cdiv_up(n, GS_T) * batch;
+  const long r64 = (n64 + 255) / 256, r32 = (n32 + 255) / 256;
+  if (k <= 16) return r32 == 1;  // half a chunk of the 32x32 kernel
+  if (r32 <= 8) return 27 * r32 < 70 * r64;
+  return 37 * n32 < 129 * n64;
 }
 
 void zgemm_strided(hipStream_t s, int opA, int opB, int m, int n, int k, cd alpha, const cd* A, long lda,
                    long sA, const cd* B, long ldb, long sB, cd beta, cd* C, long ldc, long sC, int batch) {
   if (m <= 0 || n <= 0 || batch <= 0) return;
-  if (g_big_gemm && g_big_n == 128 && k > 0 && k >= g_big_min_k && m >= GB_M && n >= GQ_N) {
-    const int gm = cdiv_up(m, GB_M), gn = cdiv_up(n, GQ_N);
-    const long total = (long)gm * gn * batch;
-    dim3 grid((unsigned)total);
-#define VRC_SQ(OA, OB) \
-  zgemm_sq_kernel<OA, OB><<<grid, GB8_THREADS, 0, s>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, gm, gn, total)
+  if (k > 0 && zgemm_use_32(m, n, k, batch)) {
+    dim3 grid(cdiv_up(m, GS_T), cdiv_up(n, GS_T), batch);
+#define VRC_S32(OA, OB) \
+  zgemm_small_kernel<OA, OB><<<grid, GS_THREADS, 0, s>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC)
     switch (opA * 3 + opB) {
-      case 0: VRC_SQ(OP_N, OP_N); break;
-      case 1: VRC_SQ(OP_N, OP_T); break;
-      case 2: VRC_SQ(OP_N, OP_C); break;
-      case 3: VRC_SQ(OP_T, OP_N); break;
-      case 4: VRC_SQ(OP_T, OP_T); break;
-      case 5: VRC_SQ(OP_T, OP_C); break;
-      case 6: VRC_SQ(OP_C, OP_N); break;
-      case 7: VRC_SQ(OP_C, OP_T); break;
-      default: VRC_SQ(OP_C, OP_C); break;
+      case 0: VRC_S32(OP_N, OP_N); break;
+      case 1: VRC_S32(OP_N, OP_T); break;
+      case 2: VRC_S32(OP_N, OP_C); break;
+      case 3: VRC_S32(OP_T, OP_N); break;
+      case 4: VRC_S32(OP_T, OP_T); break;
+      case 5: VRC_S32(OP_T, OP_C); break;
+      case 6: VRC_S32(OP_C, OP_N); break;
+      case 7: VRC_S32(OP_C, OP_T); break;
+      default: VRC_S32(OP_C, OP_C); break;
     }
-#undef VRC_SQ
-    launch_check("zgemm_sq");
-    return;
-  }
-  if (g_big_gemm && k > 0 && k >= g_big_min_k && m >= GB_M && n >= GB_N) {
-    const int gm = cdiv_up(m, GB_M), gn = cdiv_up(n, GB_N);
-    const long total = (long)gm * gn * batch;
-    dim3 grid((unsigned)total);
-#define VRC_BIG(OA, OB)                                                                                              \
-  if (g_big_waves == 8)                                                                                              \
-    zgemm_big8_kernel<OA, OB><<<grid, GB8_THREADS, 0, s>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, \
-                                                           gm, gn, total);                                           \
-  else                                                                                                               \
-    zgemm_big_kernel<OA, OB><<<grid, GT_THREADS, 0, s>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC,   \
-                                                         gm, gn, total)
-    switch (opA * 3 + opB) {
-      case 0: VRC_BIG(OP_N, OP_N); break;
-      case 1: VRC_BIG(OP_N, OP_T); break;
-      case 2: VRC_BIG(OP_N, OP_C); break;
-      case 3: VRC_BIG(OP_T, OP_N); break;
-      case 4: VRC_BIG(OP_T, OP_T); break;
-      case 5: VRC_BIG(OP_T, OP_C); break;
-      case 6: VRC_BIG(OP_C, OP_N); break;
-      case 7: VRC_BIG(OP_C, OP_T); break;
-      default: VRC_BIG(OP_C, OP_C); break;
-    }
-#undef VRC_BIG
-    launch_check("zgemm_big");
+#undef VRC_S32
+    launch_check("zgemm_small");
     return;
   }
   dim3 grid(cdiv_up(m, GT_M), cdiv_up(n, GT_N), batch);

@@ -88,24 +88,11 @@ int vrc_pool_trim(vrc_ctx* c) {
 int vrc_tune_set(const char* key, long long value) {
   if (!key) return -1;
   tune_manual_begin();
-  if (std::strcmp(key, "zgemm.large_tile") == 0) {
-    zgemm_set_big(value != 0);
-    return 0;
-  }
-  if (std::strcmp(key, "zgemm.large_tile_min_k") == 0) {
-    zgemm_set_big_min_k((int)value);
-    return 0;
-  }
-  if (std::strcmp(key, "zgemm.big_waves") == 0) {
-    zgemm_set_big_waves((int)value);
-    return 0;
-  }
+  // switches of tiles that are gone: accepted, without effect
+  for (const char* old : {"zgemm.large_tile", "zgemm.large_tile_min_k", "zgemm.big_waves", "zgemm.big_n"})
+    if (std::strcmp(key, old) == 0) return 0;
   if (std::strcmp(key, "zgemm.small_waves") == 0) {
     zgemm_set_small_waves((int)value);
-    return 0;
-  }
-  if (std::strcmp(key, "zgemm.big_n") == 0) {
-    zgemm_set_big_n((int)value);
     return 0;
   }
   if (std::strcmp(key, "redheffer.max_depth") == 0) {

@@ -92,13 +92,8 @@ void health_note_gamma(hipStream_t s, const cd* gam, long count);
 // ---------------------------------------------------------------- blas.hip
 void zgemm_strided(hipStream_t s, int opA, int opB, int m, int n, int k, cd alpha, const cd* A, long lda, long sA,
                    const cd* B, long ldb, long sB, cd beta, cd* C, long ldc, long sC, int batch);
-void zgemm_set_big(bool on);  // large-tile kernel on/off (default on)
-void zgemm_set_big_min_k(int k);  // smallest k for the large-tile kernel
-void zgemm_set_big_waves(int w);  // wavefronts of the large-tile kernel (4 or 8)
 void zgemm_set_small_waves(int w);  // wavefronts of the 64x64-tile kernel (4 or 8)
-void zgemm_set_big_n(int n);        // columns of the large tile (64 or 128)
-void zgemm_desc(hipStream_t s, int opA, int opB, const GemmDesc* d_desc, int count, int max_m, int max_n);
-void zgemm_get_knobs(int* big_n, int* big_waves, int* small_waves, int* big_min_k);
+int zgemm_get_small_waves();
 void zgeam(hipStream_t s, int m, int n, cd a, const cd* A, long lda, long sA, cd b, const cd* B, long ldb, long sB,
            cd* C, long ldc, long sC, int batch);
 void zset(hipStream_t s, int m, int n, cd diag, cd off, cd* C, long ldc, long sC, int batch);
@@ -166,7 +161,7 @@ unsigned zgeev_take_qr_kernels();
 // ---------------------------------------------------------------- autotune.cpp
 // The kernel switches an autotuned harmonic count overrides (process-wide values).
 struct TuneKnobs {
-  int aed, bulges, big_n, big_waves, small_waves, big_min_k;
+  int aed, bulges, small_waves;
   int qr_variant;              // -1 (automatic), 0, 2 or 4 (zgeev_set_qr_variant)
   int bulges_w48, bulges_w32;  // bulges per sweep of QR variants 2 and 4 (bulges: 0 and 1)
 };
