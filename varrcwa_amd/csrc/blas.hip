@@ -248,8 +248,9 @@ __device__ __forceinline__ void zgemm_tile8(int m, int n, int k, cd alpha, const
 
 // 32x32 output per 256-thread workgroup (four waves, one 16x16 block each) with K in chunks of
 // 32, for products whose larger tiles would leave most CUs without a workgroup (single
-// matrices and short right-hand sides): latency-bound there, so the tile is small, a barrier
-// covers 32 k, and the four real products go to four accumulators (no dependent MFMA pairs).
+// matrices and short right-hand sides): latency-bound there, so the tile is small and a barrier
+// covers 32 k. Every element is summed in the order of the 64x64 tile, so the two agree to
+// the last bit.
 constexpr int GS_T = 32, GS_K = 32, GS_THREADS = 256;
 
 template <int OPA, int OPB>
@@ -266,7 +267,7 @@ __device__ __forceinline__ void zgemm_tile32(int m, int n, int k, cd alpha, cons
   const int wr = wave >> 1, wc = wave & 1;
   const int row0 = tm * GS_T, col0 = tn * GS_T;
   const bool live = __builtin_amdgcn_readfirstlane(row0 + wr * 16 < m && col0 + wc * 16 < n);
-  d4 rr = d4{0.0, 0.0, 0.0, 0.0}, ii = rr, ri = rr, ir = rr;
+  d4 accR = d4{0.0, 0.0, 0.0, 0.0}, accI = accR;
   // element q of this thread: (x, y) = (t & 31, (t >> 5) + 8 q), x along the operand's columns
   const int x = t & 31, y = t >> 5;
   cd pa[4], pb[4];
@@ -310,10 +311,10 @@ __device__ __forceinline__ void zgemm_tile32(int m, int n, int k, cd alpha, cons
         const int kr = s * 4 + (lane >> 4);
         const double ar = As_re[kr][wr * 16 + (lane & 15)], ai = As_im[kr][wr * 16 + (lane & 15)];
         const double br = Bs_re[kr][wc * 16 + (lane & 15)], bi = Bs_im[kr][wc * 16 + (lane & 15)];
-        rr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, rr, 0, 0, 0);
-        ii = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, ii, 0, 0, 0);
-        ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, ri, 0, 0, 0);
-        ir = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, ir, 0, 0, 0);
+        accR = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, accR, 0, 0, 0);
+        accI = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, accI, 0, 0, 0);
+        accR = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, bi, accR, 0, 0, 0);
+        accI = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, accI, 0, 0, 0);
       }
     }
     __syncthreads();
@@ -325,7 +326,7 @@ __device__ __forceinline__ void zgemm_tile32(int m, int n, int k, cd alpha, cons
   for (int r = 0; r < 4; ++r) {
     const int gr = row0 + wr * 16 + (lane >> 4) + 4 * r;
     if (gr >= m) continue;
-    cd out = cmul(alpha, mk(rr[r] - ii[r], ri[r] + ir[r]));
+    cd out = cmul(alpha, mk(accR[r], accI[r]));
     cd* cp = C + gr + (long)gc * ldc;
     if (!beta0) out = cadd(out, cmul(beta, *cp));
     *cp = out;
