@@ -425,12 +425,104 @@ void init_identity_S(vrc_ctx& c, int N, SMat& S, int batch) {
 }
 }  // namespace
 
+// ===================================================================== cascades
+namespace {
+// One S-matrix by pointers (N x N blocks, ld N).
+struct SPtr {
+  const cd *Tdd, *Tuu, *Rud, *Rdu;
+};
+
+SMat smat_at(cd* p, long blk) {
+  SMat S;
+  S.Tdd = p;
+  S.Tuu = p + blk;
+  S.Rud = p + 2 * blk;
+  S.Rdu = p + 3 * blk;
+  return S;
+}
+
+// Matrices of N x N that a tree of star products may hold (pairs in flight, or all its levels).
+size_t cascade_mats(int N) {  // (8192 products at most in one batch: the grid's y and z limits)
+  return std::max<size_t>(16, ((size_t)8 << 30) / (sizeof(cd) * (size_t)N * N)); }
+
+// Star product of n S-matrices in each of B rows (items[b * n + j], j in cascade order) into out
+// (row stride N^2). The star product is associative: pairs of neighbours are combined level by
+// level, every level one batch over rows and pairs, so a row of n takes about log2(n) batched
+// products instead of n - 1 of batch B. A product's LU panels and substitution steps are serial
+// and hold one CU per matrix: 24 products at N = 126 one after the other took 17.7 ms, as a tree
+// 4.1 ms. A level's products run in chunks of at most cascade_mats matrices of work space; the
+// levels together hold at most 4 B n matrices.
+void cascade_tree(vrc_ctx& c, int N, int B, int n, std::vector<SPtr> items, SMat& out) {
+  hipStream_t st = c.stream;
+  const long NN = (long)N * N;
+  const size_t M = sizeof(cd) * NN;
+  std::vector<DevBuf> keep;
+  while (n > 1) {
+    const int np = n / 2, m = np + (n & 1);
+    const int total = B * np;
+    const int per = std::max(1, std::min<int>(total, (int)std::min<size_t>(8192, cascade_mats(N) / 16)));
+    DevBuf Sb = c.ws.get(4 * M * (size_t)total);
+    std::vector<SPtr> next((size_t)B * m);
+    for (int q0 = 0; q0 < total; q0 += per) {
+      const int P = std::min(per, total - q0);
+      cd* S0 = Sb.as<cd>() + 4 * NN * q0;
+      SMat S = smat_at(S0, P * NN);
+      DevBuf Rb = c.ws.get(4 * M * (size_t)P);
+      std::vector<const void*> left(4 * (size_t)P), right(4 * (size_t)P);
+      for (int q = 0; q < P; ++q) {
+        const int b = (q0 + q) / np, j = (q0 + q) % np;
+        const SPtr &x = items[(size_t)b * n + 2 * j], &y = items[(size_t)b * n + 2 * j + 1];
+        const cd* xs[4] = {x.Tdd, x.Tuu, x.Rud, x.Rdu};
+        const cd* ys[4] = {y.Tdd, y.Tuu, y.Rud, y.Rdu};
+        for (int k = 0; k < 4; ++k) {
+          left[(size_t)k * P + q] = xs[k];
+          right[(size_t)k * P + q] = ys[k];
+        }
+        next[(size_t)b * m + j] = SPtr{S.Tdd + q * NN, S.Tuu + q * NN, S.Rud + q * NN, S.Rdu + q * NN};
+      }
+      gather_ptrs(c, left, M, S0);
+      gather_ptrs(c, right, M, Rb.ptr);
+      const SMat R = smat_at(Rb.as<cd>(), P * NN);
+      star_product(c, N, P, S, R.Tdd, R.Tuu, R.Rud, R.Rdu, NN);
+    }
+    if (n & 1)
+      for (int b = 0; b < B; ++b) next[(size_t)b * m + np] = items[(size_t)b * n + n - 1];
+    keep.push_back(std::move(Sb));
+    items.swap(next);
+    n = m;
+  }
+  cd* dst[4] = {out.Tdd, out.Tuu, out.Rud, out.Rdu};
+  for (int k = 0; k < 4; ++k) {
+    std::vector<const void*> src(B);
+    for (int b = 0; b < B; ++b) {
+      const SPtr& x = items[b];
+      src[b] = k == 0 ? x.Tdd : (k == 1 ? x.Tuu : (k == 2 ? x.Rud : x.Rdu));
+    }
+    gather_ptrs(c, src, M, dst[k]);
+  }
+}
+
+// S <- S * (items' cascade), or the cascade itself when first (S the identity, not read).
+void cascade_onto(vrc_ctx& c, int N, int B, int n, std::vector<SPtr> items, SMat& S, bool first) {
+  if (first) {
+    cascade_tree(c, N, B, n, std::move(items), S);
+    return;
+  }
+  const long NN = (long)N * N;
+  DevBuf Tb = c.ws.get(sizeof(cd) * 4 * NN * (size_t)B);
+  SMat T = smat_at(Tb.as<cd>(), B * NN);
+  cascade_tree(c, N, B, n, std::move(items), T);
+  star_product(c, N, B, S, T.Tdd, T.Tuu, T.Rud, T.Rdu, NN);
+}
+}  // namespace
+
 // RCWAIntegrator::compute (src/core/RCWAIntegrator.cpp:20-87) over explicit slices
 // (midpoint z, width). The slices are independent until the cascade, so their samples,
 // eigensolves and slab S-matrices run in groups of up to g_rcwa_group per launch (one
-// eigensolve per workgroup), the two end media riding with the first group; the star
-// products then follow in slice order, as the reference cascades them. Each matrix's
-// result does not depend on the group it is solved in.
+// eigensolve per workgroup), the two end media riding with the first group; a group's star
+// products then run as a tree, the groups in slice order (the reference cascades slice by
+// slice; the product is associative). Each matrix's result does not depend on the group it is
+// solved in.
 static int g_rcwa_group = 64;
 void rcwa_set_group(int g) { g_rcwa_group = g < 1 ? 1 : g; }
 void Integrator::rcwa(const std::vector<std::pair<double, double>>& slices, bool) {
@@ -476,10 +568,16 @@ void Integrator::rcwa(const std::vector<std::pair<double, double>>& slices, bool
     DevBuf ds = upload(c, sv.data(), sizeof(double) * g);
     layer_smatrix(c, N, g, ds.as<double>(), Wb.as<cd>() + e * NN, Vb.as<cd>() + e * NN, gb.as<cd>() + e * N,
                   W1_.as<cd>(), V1_.as<cd>(), 0, tu.as<cd>(), ru.as<cd>());
-    for (int j = 0; j < g; ++j) {
-      const cd* t = tu.as<cd>() + j * NN;
-      const cd* r = ru.as<cd>() + j * NN;
-      star_product(c, N, 1, S, t, t, r, r, 0);
+    const int tree = (int)std::min<size_t>(g, cascade_mats(N) / 4);
+    for (int j0 = 0; j0 < g; j0 += tree) {
+      std::vector<SPtr> items;
+      for (int j = j0; j < std::min(g, j0 + tree); ++j) {
+        const cd* t = tu.as<cd>() + j * NN;
+        const cd* r = ru.as<cd>() + j * NN;
+        items.push_back(SPtr{t, t, r, r});
+      }
+      const int cnt = (int)items.size();
+      cascade_onto(c, N, 1, cnt, std::move(items), S, i0 + j0 == 0);
     }
   }
   project_left(c, N, 1, S, lu1.pair, W0_.as<cd>(), V0_.as<cd>(), 0);
@@ -568,9 +666,9 @@ void Integrator::redheffer(double pe, int max_depth) { redheffer_many({this}, pe
 // of a level is evaluated (perturbation and error, one readback for all), the accepted
 // ones keep their S-matrices, and the rejected ones are trisected with their new
 // samples taken together and their new reference eigensystems solved in one batched
-// launch. The accepted segments are then projected and star-multiplied in z order,
-// exactly as the recursion does (src/core/RedhefferIntegrator.cpp:248-276), and the
-// right projection follows (:211-223).
+// launch. The accepted segments are then projected to their left neighbours' bases, as the
+// recursion does (src/core/RedhefferIntegrator.cpp:248-276), in batches, and star-multiplied
+// in z order as a tree; the right projection follows (:211-223).
 void Integrator::redheffer_many(const std::vector<Integrator*>& its, double pe, int max_depth) {
   if (its.empty()) return;
   vrc_ctx& c = *its[0]->c_;
@@ -706,21 +804,53 @@ void Integrator::redheffer_many(const std::vector<Integrator*>& its, double pe, 
     init_identity_S(c, N, S, 1);
     const cd* leftW = it.W0_.as<cd>();
     const cd* leftV = it.V0_.as<cd>();
-    for (auto& d : D) {
-      cd* T0 = d.T->as<cd>() + d.off;
-      SMat T;
-      T.Tdd = T0;
-      T.Tuu = T0 + NN;
-      T.Rud = T0 + 2 * NN;
-      T.Rdu = T0 + 3 * NN;
-      const RefSys R = d.R.sys(N);
-      project_left(c, N, 1, T, R.LU, leftW, leftV, 0);
-      leftW = R.W;
-      leftV = R.V;
-      star_product(c, N, 1, S, T.Tdd, T.Tuu, T.Rud, T.Rdu, 0);
-      it.tree_.push_back({d.za, d.zb});
-      ++it.N_;
-      d.T.reset();
+    // the projection of a segment needs its left neighbour's reference only, so the segments
+    // are projected in batches (bounded work space), each batch cascaded as a tree
+    const int per = (int)std::min<size_t>(8192, std::max<size_t>(1, cascade_mats(N) / 24));
+    for (size_t d0 = 0; d0 < D.size(); d0 += per) {
+      const int P = (int)std::min<size_t>(per, D.size() - d0);
+      const size_t M = sizeof(cd) * NN, Pn = sizeof(int) * N;
+      std::vector<const void*> lw(P), lv(P), fw(P), fv(P), pw(P), pv(P), blk(4 * (size_t)P);
+      for (int q = 0; q < P; ++q) {
+        const Done& d = D[d0 + q];
+        const RefSys R = d.R.sys(N);
+        lw[q] = leftW;
+        lv[q] = leftV;
+        fw[q] = R.LU.W;
+        fv[q] = R.LU.V;
+        pw[q] = R.LU.pW;
+        pv[q] = R.LU.pV;
+        for (int k = 0; k < 4; ++k) blk[(size_t)k * P + q] = d.T->as<cd>() + d.off + k * NN;
+        leftW = R.W;
+        leftV = R.V;
+        it.tree_.push_back({d.za, d.zb});
+        ++it.N_;
+      }
+      DevBuf Tb = c.ws.get(4 * M * P), Fb = c.ws.get(2 * M * P), Lb = c.ws.get(2 * M * P), Pb = c.ws.get(2 * Pn * P);
+      cd *F = Fb.as<cd>(), *Lf = Lb.as<cd>();
+      int* pp = Pb.as<int>();
+      gather_ptrs(c, blk, M, Tb.ptr);
+      gather_ptrs(c, fw, M, F);
+      gather_ptrs(c, fv, M, F + P * NN);
+      gather_ptrs(c, lw, M, Lf);
+      gather_ptrs(c, lv, M, Lf + P * NN);
+      gather_ptrs(c, pw, Pn, pp);
+      gather_ptrs(c, pv, Pn, pp + (long)P * N);
+      LUPair lu;
+      lu.W = F;
+      lu.V = F + P * NN;
+      lu.pW = pp;
+      lu.pV = pp + (long)P * N;
+      lu.sM = NN;
+      SMat T = smat_at(Tb.as<cd>(), P * NN);
+      project_left(c, N, P, T, lu, Lf, Lf + P * NN, NN);
+      for (int q = 0; q < P; ++q) D[d0 + q].T.reset();
+      Fb = DevBuf();
+      Lb = DevBuf();
+      std::vector<SPtr> items(P);
+      for (int q = 0; q < P; ++q)
+        items[q] = SPtr{T.Tdd + q * NN, T.Tuu + q * NN, T.Rud + q * NN, T.Rdu + q * NN};
+      cascade_onto(c, N, 1, P, std::move(items), S, d0 == 0);
     }
     LUStore lul;
     lul.make(c, N, leftW, leftV, 1, 0);
@@ -843,6 +973,7 @@ void Integrator::differential(int Nsteps) {
 // the outputs at instance offset I0.
 // tape (optional): receives the prefix before every K-th layer and the cascade before the
 // projection of the group's instances.
+constexpr int CASCADE_SEQ = 128;  // instances from which the layers are cascaded one by one
 static void cascade_group(vrc_ctx& c, int N, int L, int GB, int I0, bool homog, const cd* tu, const cd* ru,
                           const cd* We, const cd* Ve, const cd* ge, cd* S_out, cd* W0o, cd* V0o, cd* g0o, cd* W1o,
                           cd* V1o, cd* g1o, StackTape* tape = nullptr) {
@@ -863,11 +994,22 @@ static void cascade_group(vrc_ctx& c, int N, int L, int GB, int I0, bool homog, 
   S.Tuu = S.Tdd + B * NN;
   S.Rud = S.Tdd + 2 * B * NN;
   S.Rdu = S.Tdd + 3 * B * NN;
+  // A few instances: trees of star products over blocks of layers (between the tape's
+  // checkpoints, within cascade_mats matrices). From 128 instances on, one layer's products
+  // fill the chip by themselves and the sequential form below needs no copies.
+  int tree = 0;
+  if (B < CASCADE_SEQ && L > 2) {
+    tree = (int)std::min<size_t>(L, std::max<size_t>(1, cascade_mats(N) / (4 * (size_t)B)));
+    if (tape && tape->nblocks() > 1) tree = std::min(tree, tape->K);
+    if (tree < 3) tree = 0;
+  }
   // identity * slab 0 = slab 0: the cascade starts from the first slab's S-matrix
+  if (!tree) {
   zgeam(st, N, N, ONE, tu, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Tdd, N, NN, B);
   zgeam(st, N, N, ONE, tu, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Tuu, N, NN, B);
   zgeam(st, N, N, ONE, ru, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Rud, N, NN, B);
   zgeam(st, N, N, ONE, ru, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Rdu, N, NN, B);
+  }
   // tape layout: 4 blocks [Tdd|Tuu|Rud|Rdu] per instance
   auto keep_S = [&](cd* dst, long per_inst) {
     const SMat* src = &S;
@@ -876,7 +1018,21 @@ static void cascade_group(vrc_ctx& c, int N, int L, int GB, int I0, bool homog, 
       zgeam(st, N, N, ONE, blk[q], N, NN, ZERO, nullptr, 0, 0, dst + (long)i0 * per_inst + q * NN, N, per_inst, B);
   };
   const int nb = tape ? tape->nblocks() : 0;
-  for (int l = 1; l < L; ++l) {
+  for (int l0 = 0, l1; tree && l0 < L; l0 = l1) {
+    if (tape && l0 > 0 && l0 % tape->K == 0)
+      keep_S(tape->ckpt.as<cd>() + (long)(l0 / tape->K - 1) * 4 * NN, (long)(nb - 1) * 4 * NN);
+    l1 = std::min(L, l0 + tree);
+    if (tape) l1 = std::min(l1, (l0 / tape->K + 1) * tape->K);  // stop at the next checkpoint
+    std::vector<SPtr> items;
+    for (int b = 0; b < B; ++b)
+      for (int l = l0; l < l1; ++l) {
+        const cd* t = tu + ((long)b * L + l) * NN;
+        const cd* r = ru + ((long)b * L + l) * NN;
+        items.push_back(SPtr{t, t, r, r});
+      }
+    cascade_onto(c, N, B, l1 - l0, std::move(items), S, l0 == 0);
+  }
+  for (int l = 1; !tree && l < L; ++l) {
     if (tape && l % tape->K == 0)
       keep_S(tape->ckpt.as<cd>() + (long)(l / tape->K - 1) * 4 * NN, (long)(nb - 1) * 4 * NN);
     const cd* t = tu + l * NN;

@@ -921,7 +921,7 @@ __global__ void gather_ptr_kernel(long nwords, const double* const* src, double*
     dst[b * nwords + e] = a[e];
 }
 
-static void gather_ptrs(vrc_ctx& c, const std::vector<const void*>& src, size_t nbytes, void* dst) {
+void gather_ptrs(vrc_ctx& c, const std::vector<const void*>& src, size_t nbytes, void* dst) {
   const int B = (int)src.size();
   if (B == 0) return;
   DevBuf p = c.ws.get(sizeof(void*) * B);
