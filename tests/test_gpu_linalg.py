@@ -240,3 +240,33 @@ def _eig_check_values(ctx, A):
     for b in range(batch):
         assert np.abs(A[b] @ V[b] - V[b] * W[b][None, :]).max() < 1e-12 * n * np.linalg.norm(A[b], 2)
     return W, V
+
+
+@pytest.mark.parametrize("n", [200, 242])
+def test_zgeev_team_sizes(ctx, n):
+    """Launches of 1, 9, 70 and 128 matrices give the QR kernel teams of 16, 16, 3 and 2
+    workgroups per matrix, 129 none: the same matrix gives the same bits in all of them (the
+    shares of a window product do not depend on who computes them)."""
+    rng = np.random.default_rng(4000 + n)
+    A = crand(rng, 1, n, n)
+    ref = None
+    for batch in (129, 1, 9, 70, 128):
+        w, V = _eig_check_values(ctx, np.repeat(A, batch, axis=0)) if batch < 9 else _eig_values(ctx, A, batch)
+        if ref is None:
+            ref = (w[0], V[0])
+        for b in (0, batch // 2, batch - 1):
+            assert np.array_equal(w[b], ref[0]) and np.array_equal(V[b], ref[1]), (batch, b)
+
+
+def _eig_values(ctx, A, batch):
+    import torch
+    n = A.shape[-1]
+    dA = to_dev_colmajor(A).expand(batch, n, n).contiguous()
+    w = torch.zeros((batch, n), dtype=torch.complex128, device="cuda")
+    VR = torch.zeros_like(dA)
+    info = torch.zeros(batch, dtype=torch.int32, device="cuda")
+    ctx.check(ctx.lib.vrc_zgeev(ctx.h, n, ptr(dA), n, n * n, ptr(w), n, ptr(VR), n, n * n, ptr(info), batch),
+              "zgeev")
+    ctx.sync()
+    assert info.cpu().numpy().tolist() == [0] * batch
+    return w.cpu().numpy(), from_dev_colmajor(VR)

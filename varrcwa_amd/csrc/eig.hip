@@ -20,6 +20,7 @@
 #include "vrc_common.hpp"
 #include "vrc_internal.hpp"
 #include "vrc_context.hpp"
+#include "vrc_ops.hpp"
 
 namespace vrc {
 
@@ -606,15 +607,17 @@ static_assert(sizeof(QrLds<32, 128>) <= 40 * 1024, "four W = 32 QR workgroups mu
 // D[(l >> 4) + 4 q][l & 15], q < 4. Both products are formed transposed so that a lane's
 // global loads and stores run along a column (16 consecutive rows per instruction).
 //
-// M[r0:r0+w, c0:c1] <- U^H M[...]: as D = M^T conj(U) per 16 columns; wave v owns columns
-// c0 + 16 v + 16 NW k, reads their w rows into registers and writes them back.
-template <int W, int NW>
-__device__ void apply_left_reg(const QMat<W>& U, int w, cd* M, long ld, int r0, int c0, int c1) {
+// M[r0:r0+w, c0:c1] <- U^H M[...]: as D = M^T conj(U) per 16 columns; the wave takes the
+// 16-column strips first, first + step, ..., reads their w rows into registers and writes
+// them back.
+template <int W>
+__device__ void apply_left_reg(const QMat<W>& U, int w, cd* M, long ld, int r0, int c0, int c1, int first,
+                               int step) {
   constexpr int KS = W / 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
   const int kk = lane >> 4, jl = lane & 15;
   const int ks = (w + 3) >> 2, rbn = (w + 15) >> 4;
-  for (int cc = c0 + 16 * wave; cc < c1; cc += 16 * NW) {
+  for (int cc = c0 + 16 * first; cc < c1; cc += 16 * step) {
     cd a[KS];
     {
       const int col = cc + jl;
@@ -649,15 +652,16 @@ __device__ void apply_left_reg(const QMat<W>& U, int w, cd* M, long ld, int r0, 
   }
 }
 
-// M[r0:r1, c0:c0+w] <- M[...] U: as D = U^T M^T per 16 rows; wave v owns rows
-// r0 + 16 v + 16 NW k, reads their w columns into registers and writes them back.
-template <int W, int NW>
-__device__ void apply_right_reg(const QMat<W>& U, int w, cd* M, long ld, int r0, int r1, int c0) {
+// M[r0:r1, c0:c0+w] <- M[...] U: as D = U^T M^T per 16 rows; the wave takes the 16-row strips
+// first, first + step, ..., reads their w columns into registers and writes them back.
+template <int W>
+__device__ void apply_right_reg(const QMat<W>& U, int w, cd* M, long ld, int r0, int r1, int c0, int first,
+                                int step) {
   constexpr int KS = W / 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
   const int kk = lane >> 4, jl = lane & 15;
   const int ks = (w + 3) >> 2, cbn = (w + 15) >> 4;
-  for (int rr = r0 + 16 * wave; rr < r1; rr += 16 * NW) {
+  for (int rr = r0 + 16 * first; rr < r1; rr += 16 * step) {
     const int row = rr + jl;
     cd b[KS];
 #pragma unroll
@@ -1040,10 +1044,11 @@ __device__ __forceinline__ void wave_reflect(Mat& T, Mat& U, const cd* vv, cd ta
 
 // QR kernel configuration: window W, T threads, RA: window products from registers
 // (apply_left_reg / apply_right_reg) instead of through an LDS chunk buffer.
-template <int W_, int T_, bool RA_>
+// TM: a team of workgroups shares the products (hqr_team_kernel).
+template <int W_, int T_, bool RA_, bool TM_ = false>
 struct QrCfg {
   static constexpr int W = W_, T = T_;
-  static constexpr bool RA = RA_;
+  static constexpr bool RA = RA_, TM = TM_;
 };
 
 template <class C>
@@ -1066,23 +1071,148 @@ __device__ void lds_store_block(QrLds<C::W, C::T>& L, cd* H, long ldh, int r0, i
   __syncthreads();
 }
 
-// Apply the window transform U (on indices ws..ws+w-1) to everything outside the window.
-// The three regions (rows of the window right of it, columns of the window above it, Z)
-// are disjoint; the register form needs one barrier at the end only.
+// Wave gw of nw's share of a window transform U (indices ws..ws+w-1) applied to everything
+// outside the window: the rows of the window right of it, its columns above it, and Z. The
+// three regions are disjoint; their 16-wide strips are dealt over the waves as one list.
+template <int W>
+__device__ __forceinline__ void apply_share(const QMat<W>& U, int N, cd* H, long ldh, cd* Z, long ldz, int ws, int w,
+                                            int gw, int nw) {
+  const int we = ws + w;
+  const int nl = (N - we + 15) >> 4, nr = (ws + 15) >> 4;
+  apply_left_reg<W>(U, w, H, ldh, ws, we, N, gw, nw);
+  apply_right_reg<W>(U, w, H, ldh, 0, ws, ws, (gw + nw - nl % nw) % nw, nw);
+  apply_right_reg<W>(U, w, Z, ldz, 0, N, ws, (gw + nw - (nl + nr) % nw) % nw, nw);
+}
+
+// A team: the workgroup that iterates on a matrix (the master) and the workgroups that take part
+// in its window products. A launch of few matrices leaves most CUs idle while the products of
+// one matrix keep one CU's matrix cores busy for two thirds of the iteration. The master
+// publishes a window (its transform in global memory and one 64-bit word: sequence number,
+// members taking part, window size and start); the members apply their shares and count up
+// done. Nobody waits for a workgroup that may not be resident: a member joins only after it
+// has seen the master running (or leaves after TEAM_SPINS looks), the master counts only
+// members that have joined, and the members leave at the master's last word.
+struct TeamCtl {
+  unsigned long long word;
+  int joined, done;
+  int pad[28];  // one line per matrix
+};
+static_assert(sizeof(TeamCtl) == 128, "team control lines");
+constexpr int TEAM_SPINS = 1 << 18;
+constexpr unsigned TEAM_EXIT = 0xffffffffu;
+constexpr long TEAM_WORK = 150000;  // N w^2 from which a window is shared (measured best of 150000 .. 900000)
+struct Team {
+  TeamCtl* ctl;
+  cd* U;
+  unsigned seq;
+  int owed;
+};
+__device__ __forceinline__ unsigned long long team_word(unsigned seq, int members, int w, int ws) {
+  return ((unsigned long long)seq << 32) | ((unsigned)members << 24) | ((unsigned)w << 16) | (unsigned)ws;
+}
+template <class T>
+__device__ __forceinline__ T agent_load(T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// One thread: everything written before (by the workgroup, up to its last barrier) becomes
+// visible to the GPU, then the word is stored.
+__device__ __forceinline__ void team_publish(Team& tm, unsigned long long word) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  __hip_atomic_store(&tm.ctl->word, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Apply the window transform U (on indices ws..ws+w-1) to everything outside the window. The
+// register form needs one barrier at the end only.
 template <class C>
-__device__ void apply_window(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz, int ws, int w) {
+__device__ void apply_window(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz, int ws, int w, Team& tm) {
   const int we = ws + w - 1;
-  if constexpr (C::RA) {
-    constexpr int NW = C::T / 64;
-    if (we + 1 < N) apply_left_reg<C::W, NW>(L.U, w, H, ldh, ws, we + 1, N);
-    if (ws > 0) apply_right_reg<C::W, NW>(L.U, w, H, ldh, 0, ws, ws);
-    apply_right_reg<C::W, NW>(L.U, w, Z, ldz, 0, N, ws);
+  constexpr int NW = C::T / 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if constexpr (C::TM) {
+    const int t = threadIdx.x;
+    int members = 0;
+    if ((long)N * w * w >= TEAM_WORK) {
+      if (t == 0) L.ctl[3] = agent_load(&tm.ctl->joined);
+      __syncthreads();
+      members = L.ctl[3];
+    }
+    if (members > 0) {
+      ++tm.seq;
+      for (int e = t; e < w * w; e += C::T) tm.U[e] = L.U[e % w][e / w];
+      __syncthreads();
+      if (t == 0) team_publish(tm, team_word(tm.seq, members, w, ws));
+    }
+    apply_share<C::W>(L.U, N, H, ldh, Z, ldz, ws, w, wave, NW * (members + 1));
+    __syncthreads();
+    if (members > 0) {
+      tm.owed += members;
+      if (t == 0) {
+        while (agent_load(&tm.ctl->done) < tm.owed) __builtin_amdgcn_s_sleep(1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      }
+      __syncthreads();
+    }
+  } else if constexpr (C::RA) {
+    apply_share<C::W>(L.U, N, H, ldh, Z, ldz, ws, w, wave, NW);
     __syncthreads();
   } else {
     static_assert(C::W == QW && C::T == QT, "the LDS-staged window products are written for W = 64, 512 threads");
     if (we + 1 < N) apply_left_u(L.U, L.Hw, w, H, ldh, ws, we + 1, N);
     if (ws > 0) apply_right_u(L.U, L.Hw, w, H, ldh, 0, ws, ws);
     apply_right_u(L.U, L.Hw, w, Z, ldz, 0, N, ws);
+  }
+}
+
+// A team member's whole run: join, then take part in every published window that counts it.
+template <class C>
+__device__ void team_member(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz, Team tm) {
+  constexpr int NW = C::T / 64;
+  const int t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  unsigned seen = 0;
+  if (t == 0) {
+    int k = 0;
+    for (int spin = 0; spin < TEAM_SPINS; ++spin) {
+      seen = (unsigned)(agent_load(&tm.ctl->word) >> 32);
+      if (seen != 0) break;
+      __builtin_amdgcn_s_sleep(8);
+    }
+    if (seen != 0 && seen != TEAM_EXIT)
+      k = 1 + __hip_atomic_fetch_add(&tm.ctl->joined, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    L.ctl[0] = k;
+  }
+  __syncthreads();
+  const int k = L.ctl[0];
+  if (k == 0) return;
+  for (;;) {
+    __syncthreads();
+    if (t == 0) {
+      unsigned long long word = agent_load(&tm.ctl->word);
+      while ((unsigned)(word >> 32) == seen) {
+        __builtin_amdgcn_s_sleep(2);
+        word = agent_load(&tm.ctl->word);
+      }
+      seen = (unsigned)(word >> 32);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      L.ctl[1] = seen == TEAM_EXIT ? 1 : 0;
+      L.ctl[2] = (int)(unsigned)(word & 0xffffffffu);
+    }
+    __syncthreads();
+    if (L.ctl[1]) return;
+    const unsigned par = (unsigned)L.ctl[2];
+    const int members = (int)(par >> 24), w = (int)((par >> 16) & 0xff), ws = (int)(par & 0xffff);
+    if (members < k) continue;  // published before this member joined
+    for (int e = t; e < C::W * C::W; e += C::T) {
+      const int i = e % C::W, j = e / C::W;
+      L.U[i][j] = (i < w && j < w) ? tm.U[i + j * w] : mk(0.0, 0.0);
+    }
+    __syncthreads();
+    apply_share<C::W>(L.U, N, H, ldh, Z, ldz, ws, w, k * NW + wave, NW * (members + 1));
+    __syncthreads();
+    if (t == 0) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      __hip_atomic_fetch_add(&tm.ctl->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
 }
 
@@ -1095,7 +1225,7 @@ __device__ void apply_window(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z
 // eigenvalues are left in L.aedv[0..*nsa) for use as shifts.
 template <class C>
 __device__ int aed(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz, int lo, int hi, int nw,
-                    int* nsa) {
+                    int* nsa, Team& tm) {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int kwtop = hi - nw + 1;
   const cd spike = (kwtop > lo) ? H[kwtop + (long)(kwtop - 1) * ldh] : mk(0.0, 0.0);
@@ -1186,7 +1316,7 @@ __device__ int aed(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz
   lds_store_block<C>(L, H, ldh, kwtop, nw);
   if (t == 0 && kwtop > lo) H[kwtop + (long)(kwtop - 1) * ldh] = newspike;
   __syncthreads();
-  apply_window<C>(L, N, H, ldh, Z, ldz, kwtop, nw);
+  apply_window<C>(L, N, H, ldh, Z, ldz, kwtop, nw, tm);
   *nsa = ns;
   return nw - ns;
 }
@@ -1366,7 +1496,7 @@ __device__ __forceinline__ void chase_cols(QrLds<C::W, C::T>& L, const ChasePos&
 // after the columns.
 template <class C>
 __device__ void qr_sweep(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz, int lo, int hi, int nbul,
-                         long long* st) {
+                         long long* st, Team& tm) {
   constexpr int NW = C::T / 64;
   constexpr int MB = ((C::W - 9) / 3 < NBUL ? (C::W - 9) / 3 : NBUL) / NW + 1 & ~1;  // bulges per wave, even
   static_assert(MB * NW >= ((C::W - 9) / 3 < NBUL ? (C::W - 9) / 3 : NBUL), "every bulge has a wave");
@@ -1416,7 +1546,7 @@ __device__ void qr_sweep(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, lo
     }
     lds_store_block<C>(L, H, ldh, ws, w);
     const long long c1 = wall_clock64();
-    apply_window<C>(L, N, H, ldh, Z, ldz, ws, w);
+    apply_window<C>(L, N, H, ldh, Z, ldz, ws, w, tm);
     const long long c2 = wall_clock64();
     st[1] += 1;
     st[2] += c1 - c0;
@@ -1430,9 +1560,9 @@ __device__ void qr_sweep(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, lo
 // per sweep (<= NBUL).
 template <class C>
 __device__ void hqr_body(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, long sH, cd* Z, long ldz, long sZ, cd* wout,
-                         long sw, int* info, long long* stats, int use_aed, int max_bul, int max_sweeps) {
+                         long sw, int* info, long long* stats, int use_aed, int max_bul, int max_sweeps, long b,
+                         Team tm) {
   long long st[5] = {0, 0, 0, 0, 0};
-  const long b = blockIdx.x;
   H += b * sH;
   Z += b * sZ;
   wout += b * sw;
@@ -1467,7 +1597,7 @@ __device__ void hqr_body(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, long sH, 
         fail = lo + r;
         break;
       }
-      apply_window<C>(L, N, H, ldh, Z, ldz, lo, m);
+      apply_window<C>(L, N, H, ldh, Z, ldz, lo, m, tm);
       st[4] += wall_clock64() - c0;
       ihi = lo - 1;
       continue;
@@ -1484,7 +1614,7 @@ __device__ void hqr_body(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, long sH, 
     if (use_aed) {
       const long long c0 = wall_clock64();
       const int nw = m - 1 < use_aed ? m - 1 : use_aed;
-      const int nd = aed<C>(L, N, H, ldh, Z, ldz, lo, ihi, nw, &nsa);
+      const int nd = aed<C>(L, N, H, ldh, Z, ldz, lo, ihi, nw, &nsa, tm);
       st[4] += wall_clock64() - c0;
       if (nd > 0) {
         ihi -= nd;
@@ -1532,10 +1662,11 @@ __device__ void hqr_body(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, long sH, 
       if (t < ns) L.shifts[t] = L.Hw[t][t];
       __syncthreads();
     }
-    qr_sweep<C>(L, N, H, ldh, Z, ldz, lo, ihi, nbul, st);
+    qr_sweep<C>(L, N, H, ldh, Z, ldz, lo, ihi, nbul, st, tm);
     ++sweeps;
   }
   __syncthreads();
+  if (C::TM && t == 0) team_publish(tm, team_word(TEAM_EXIT, 0, 0, 0));
   for (int i = t; i < N; i += C::T) wout[i] = H[i + (long)i * ldh];
   if (t == 0) {
     info[b] = fail;
@@ -1552,7 +1683,8 @@ __device__ void hqr_body(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, long sH, 
 #define HQR_ARGS                                                                                       \
   int N, cd *H, long ldh, long sH, cd *Z, long ldz, long sZ, cd *wout, long sw, int *info, long long *stats, \
       int use_aed, int max_bul, int max_sweeps
-#define HQR_PASS N, H, ldh, sH, Z, ldz, sZ, wout, sw, info, stats, use_aed, max_bul, max_sweeps
+#define HQR_PASS \
+  N, H, ldh, sH, Z, ldz, sZ, wout, sw, info, stats, use_aed, max_bul, max_sweeps, (long)blockIdx.x, Team{}
 __global__ __launch_bounds__(512) void hqr_kernel(HQR_ARGS) {
   __shared__ QrLds<64, 512> L;
   hqr_body<QrCfg<64, 512, true>>(L, HQR_PASS);
@@ -1569,6 +1701,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void hqr_w32_kernel(HQR_ARGS) {
   __shared__ QrLds<32, 128> L;
   hqr_body<QrCfg<32, 128, true>>(L, HQR_PASS);
+}
+// The W = 64 kernel with a team of workgroups per matrix, for launches that leave CUs idle.
+// Workgroup i < batch is the master of matrix i; the members of matrix b follow at the ids
+// that keep the team on the master's XCD (workgroups go to the 8 XCDs in turn), so its
+// windows pass through one L2. batch8: the batch rounded up to whole rounds of 8. QR stage of
+// 10 matrices at N = 882 with teams of 16: 305 -> 137 ms (the products 193 -> 25 ms), of 80 at
+// N = 450 with teams of 3: 77.5 -> 62.7 ms, of 91 at N = 270 with teams of 2: 29.6 -> 25.4 ms.
+__global__ __launch_bounds__(512) void hqr_team_kernel(HQR_ARGS, int batch, int batch8, TeamCtl* ctl, cd* Uteam) {
+  __shared__ QrLds<64, 512> L;
+  typedef QrCfg<64, 512, true, true> C;
+  const int id = blockIdx.x, b = id % batch8;
+  if (b >= batch) return;
+  Team tm = {ctl + b, Uteam + (long)b * QW * QW, 1u, 0};
+  if (id >= batch8) {
+    team_member<C>(L, N, H + b * sH, ldh, Z + b * sZ, ldz, tm);
+    return;
+  }
+  if (threadIdx.x == 0) team_publish(tm, team_word(1u, 0, 0, 0));
+  hqr_body<C>(L, N, H, ldh, sH, Z, ldz, sZ, wout, sw, info, stats, use_aed, max_bul, max_sweeps, (long)b, tm);
 }
 #undef HQR_ARGS
 #undef HQR_PASS
@@ -1863,6 +2014,13 @@ static int aed_window_for(int v, int n) {
   return n <= 112 ? 8 : (n <= 144 ? 12 : (n <= 360 ? 16 : 24));
 }
 int zgeev_get_aed() { return g_aed_window; }
+// Workgroups per matrix of the 64-wide kernel: what 32 CUs per XCD hold, at most 16.
+static int team_size(int n, int batch) {
+  if (n < 200 || n > 65535) return 1;
+  const int per_xcd = (batch + 7) / 8;
+  const int g = 32 / per_xcd;
+  return g < 16 ? g : 16;
+}
 int zgeev_get_bulges() { return g_bulges; }
 
 // Schur factors of a strided batch (A destroyed): A = D Z T Z^H D^{-1} with D = diag(dbal)
@@ -1903,6 +2061,12 @@ void zgeev_factors(hipStream_t s, int n, cd* A, long lda, long sA, cd* w, long s
     } else if (qv == 1) {
       hqr_lds_kernel<<<batch, QT, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, aed, g_bulges,
                                           g_max_sweeps);
+    } else if (const int team = team_size(n, batch); team > 1) {
+      const int batch8 = (batch + 7) & ~7;
+      DevBuf tc = ws.get(sizeof(TeamCtl) * (size_t)batch), tu = ws.get(sizeof(cd) * (size_t)QW * QW * batch);
+      fill_int(s, tc.as<int>(), 0, (int)(sizeof(TeamCtl) / sizeof(int)) * batch);
+      hqr_team_kernel<<<batch8 * team, QT, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, aed, g_bulges,
+                                                   g_max_sweeps, batch, batch8, tc.as<TeamCtl>(), tu.as<cd>());
     } else {
       hqr_kernel<<<batch, QT, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, aed, g_bulges,
                                       g_max_sweeps);
