@@ -244,18 +244,32 @@ def _eig_check_values(ctx, A):
 
 @pytest.mark.parametrize("n", [200, 242])
 def test_zgeev_team_sizes(ctx, n):
-    """Launches of 1, 9, 70 and 128 matrices give the QR kernel teams of 16, 16, 3 and 2
-    workgroups per matrix, 129 none: the same matrix gives the same bits in all of them (the
-    shares of a window product do not depend on who computes them)."""
+    """Launches of 1, 9, 40, 70 and 128 matrices give the QR kernel teams of 16, 16, 6, 3 and 2
+    workgroups per matrix, 129 none: the same matrix gives the same bits whatever the team (the
+    shares of a window product do not depend on who computes them). Up to 64 matrices the
+    Hessenberg panel sums in another order, so the two ranges are compared within themselves."""
     rng = np.random.default_rng(4000 + n)
     A = crand(rng, 1, n, n)
-    ref = None
-    for batch in (129, 1, 9, 70, 128):
-        w, V = _eig_check_values(ctx, np.repeat(A, batch, axis=0)) if batch < 9 else _eig_values(ctx, A, batch)
-        if ref is None:
-            ref = (w[0], V[0])
-        for b in (0, batch // 2, batch - 1):
-            assert np.array_equal(w[b], ref[0]) and np.array_equal(V[b], ref[1]), (batch, b)
+    for batches in ((1, 9, 40, 64), (129, 70, 128)):
+        ref = None
+        for batch in batches:
+            w, V = _eig_check_values(ctx, np.repeat(A, batch, axis=0)) if batch < 9 else _eig_values(ctx, A, batch)
+            if ref is None:
+                ref = (w[0], V[0])
+            for b in (0, batch // 2, batch - 1):
+                assert np.array_equal(w[b], ref[0]) and np.array_equal(V[b], ref[1]), (batch, b)
+
+
+@pytest.mark.parametrize("n", [200, 257, 258, 259, 322])
+def test_zgeev_spread_hessenberg(ctx, n):
+    """The Hessenberg panel spread over workgroups at the edges of its row blocks, column tiles
+    and panels (64), with identity reflectors (triangular input) in the batch."""
+    rng = np.random.default_rng(5000 + n)
+    A = crand(rng, 3, n, n)
+    A[1] = np.triu(A[1]) + 3.0 * np.diag(np.arange(n))
+    A[2, n // 2:, : n // 2] = 0.0
+    _eig_check_values(ctx, A)
+    _eig_check(ctx, A[:1])
 
 
 def _eig_values(ctx, A, batch):

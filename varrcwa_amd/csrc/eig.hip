@@ -328,6 +328,240 @@ __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(4))) void g
   }
 }
 
+// ---- the same panel spread over many workgroups, three launches per column
+// With few matrices the one-workgroup panel reads each trailing matrix through one CU (about
+// 100 GB/s) once per column. Here every step of a column runs over blocks of GS_R rows, and
+// the trailing product over tiles of GS_G rows and GS_C columns, so that the chip's bandwidth
+// is used; a step ends where the next needs a sum over all rows (one launch each, no waits
+// between workgroups). Per matrix, work holds the vector b, the row blocks' partial sums and
+// the column tiles' partial products.
+constexpr int GS_R = 64, GS_G = 256, GS_C = 64;
+struct GehrdWork {  // offsets (in cd) into a matrix's work area
+  int nblk, nsp;    // row blocks and column tiles at the panel's first column
+  long dots, z, norm, part, size;
+  __host__ __device__ GehrdWork(int N, int p)
+      : nblk((N - p - 1 + GS_R - 1) / GS_R), nsp((N - p - 1 + GS_C - 1) / GS_C) {
+    dots = N;
+    z = dots + (long)nblk * HB;
+    norm = z + (long)nblk * HB;
+    part = norm + nblk;
+    size = part + (long)nsp * N;
+  }
+};
+
+// out[i] = sum over the blocks of src[blk * HB + i], i < n (256 threads; ends with a barrier).
+__device__ inline void sum_blocks(const cd* src, int nblk, int n, cd (*red)[64], cd* out) {
+  const int i = threadIdx.x & 63, q = threadIdx.x >> 6;
+  cd acc = mk(0.0, 0.0);
+  if (i < n)
+    for (int k = q; k < nblk; k += 4) acc = cadd(acc, src[(long)k * HB + i]);
+  red[q][i] = acc;
+  __syncthreads();
+  if (q == 0) out[i] = cadd(cadd(red[0][i], red[1][i]), cadd(red[2][i], red[3][i]));
+  __syncthreads();
+}
+
+// dst[i] = sum over the block's rows of conj(V[r, p + i]) x(r), i < j; the wave's lanes hold rows.
+__device__ inline void block_dots(int N, int p, int j, const cd* V, int r, cd x, cd* dst) {
+  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+  for (int i0 = q; i0 < j; i0 += 16) {
+    cd v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      v[u] = (r < N && i0 + 4 * u < j) ? V[r + (long)(p + i0 + 4 * u) * N] : mk(0.0, 0.0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const cd d = cmulc(x, v[u]);
+      const double sr = wsum(d.x), si = wsum(d.y);
+      if (lane == 0 && i0 + 4 * u < j) dst[i0 + 4 * u] = mk(sr, si);
+    }
+  }
+}
+
+// Column j's first step: y and T of column j - 1 completed, b = column c of A0 Q_j (rows below
+// p), and the blocks' parts of V^H b. j == nb: only the completion.
+__global__ __launch_bounds__(256) void gehrd_col_a_kernel(int N, int p, int nb, int j, const cd* A, long lda, long sA,
+                                                          const cd* V, long sV, cd* Y, long sY, cd* Tp, long sT,
+                                                          const cd* tau, long sTau, cd* work, GehrdWork gw) {
+  const long m = blockIdx.y;
+  A += m * sA;
+  V += m * sV;
+  Y += m * sY;
+  Tp += m * sT;
+  tau += m * sTau;
+  work += m * gw.size;
+  __shared__ cd red[4][64], zs[64], vc[64], bs[64], ys[64];
+  const int t = threadIdx.x, tr = t & 63, q = t >> 6;
+  const int blk = blockIdx.x, c = p + j;
+  const int r = p + 1 + blk * GS_R + tr;
+  const int jm = j > 0 ? j - 1 : 0;
+  if (t < 64) vc[t] = (t < j && j < nb) ? cconj(V[c + (long)(p + t) * N]) : mk(0.0, 0.0);
+  sum_blocks(work + gw.z, gw.nblk, jm, red, zs);
+  cd ay = mk(0.0, 0.0), ab = mk(0.0, 0.0);
+  if (r < N) {
+    if (j > 0) {
+      const int sp = (N - (c - 1) - 1 + GS_C - 1) / GS_C;
+      for (int k = q; k < sp; k += 4) ay = cadd(ay, work[gw.part + (long)k * N + r]);
+    }
+    for (int i = q; i < jm; i += 4) {
+      const cd y = Y[r + (long)i * N];
+      ay = csub(ay, cmul(y, zs[i]));
+      ab = cadd(ab, cmul(y, vc[i]));
+    }
+  }
+  red[q][tr] = ay;
+  __syncthreads();
+  if (q == 0 && j > 0) {
+    const cd y = cmul(tau[c - 1], cadd(cadd(red[0][tr], red[1][tr]), cadd(red[2][tr], red[3][tr])));
+    ys[tr] = y;
+    if (r < N) Y[r + (long)jm * N] = y;
+  }
+  __syncthreads();
+  red[q][tr] = ab;
+  __syncthreads();
+  if (blk == 0 && j > 0) {  // T(0 .. j-1, j-1)
+    const cd tv = tau[c - 1];
+    if (t < HB) {
+      cd s = mk(0.0, 0.0);
+      for (int l = t; l < jm; ++l) s = cadd(s, cmul(Tp[t + (long)l * HB], zs[l]));
+      Tp[t + (long)jm * HB] = t < jm ? cneg(cmul(tv, s)) : (t == jm ? tv : mk(0.0, 0.0));
+    }
+  }
+  if (j >= nb) return;
+  if (q == 0) {
+    cd b = mk(0.0, 0.0);
+    if (r < N) {
+      b = csub(A[r + (long)c * lda], cadd(cadd(red[0][tr], red[1][tr]), cadd(red[2][tr], red[3][tr])));
+      if (j > 0) b = csub(b, cmul(ys[tr], vc[jm]));
+      work[r] = b;
+    }
+    bs[tr] = b;
+  }
+  __syncthreads();
+  block_dots(N, p, j, V, r, bs[tr], work + gw.dots + (long)blk * HB);
+}
+
+// Second step: b -= V T^H (V^H b), the finished entries of column c (rows up to c), and the
+// blocks' parts of the norm of the rest.
+__global__ __launch_bounds__(256) void gehrd_col_b_kernel(int N, int p, int j, cd* A, long lda, long sA, const cd* V,
+                                                          long sV, const cd* Tp, long sT, cd* work, GehrdWork gw) {
+  const long m = blockIdx.y;
+  A += m * sA;
+  V += m * sV;
+  Tp += m * sT;
+  work += m * gw.size;
+  __shared__ cd red[4][64], ds[64], ss[64];
+  const int t = threadIdx.x, tr = t & 63, q = t >> 6;
+  const int blk = blockIdx.x, c = p + j;
+  const int r = p + 1 + blk * GS_R + tr;
+  cd ab = mk(0.0, 0.0);
+  if (j > 0) {
+    sum_blocks(work + gw.dots, gw.nblk, j, red, ds);
+    cd s = mk(0.0, 0.0);
+    if (tr < j)
+      for (int l = q; l <= tr; l += 4) s = cadd(s, cmulc(ds[l], Tp[l + (long)tr * HB]));
+    red[q][tr] = s;
+    __syncthreads();
+    if (q == 0) ss[tr] = cadd(cadd(red[0][tr], red[1][tr]), cadd(red[2][tr], red[3][tr]));
+    __syncthreads();
+    if (r < N)
+      for (int i = q; i < j; i += 4) ab = cadd(ab, cmul(V[r + (long)(p + i) * N], ss[i]));
+  }
+  red[q][tr] = ab;
+  __syncthreads();
+  if (q > 0) return;
+  double nn = 0.0;
+  if (r < N) {
+    cd b = work[r];
+    if (j > 0) {
+      b = csub(b, cadd(cadd(red[0][tr], red[1][tr]), cadd(red[2][tr], red[3][tr])));
+      work[r] = b;
+    }
+    if (r <= c) A[r + (long)c * lda] = b;
+    if (r >= c + 2) nn = cnorm2(b);
+  }
+  nn = wsum(nn);
+  if (tr == 0) work[gw.norm + blk] = mk(nn, 0.0);
+}
+
+// Third step: the reflector (every workgroup computes it), the trailing product's tiles
+// (workgroups below ngemv: rows x columns), and by the rest its vector in V, column c of A and
+// the blocks' parts of V^H v.
+__global__ __launch_bounds__(256) void gehrd_col_c_kernel(int N, int p, int j, cd* A, long lda, long sA, cd* V, long sV,
+                                                          cd* tau, long sTau, cd* work, GehrdWork gw, int nrow,
+                                                          int ngemv) {
+  const long m = blockIdx.y;
+  A += m * sA;
+  V += m * sV;
+  tau += m * sTau;
+  work += m * gw.size;
+  __shared__ cd vs[GS_C];
+  const int t = threadIdx.x, lane = t & 63, q = t >> 6;
+  const int c = p + j;
+  double nn = 0.0;
+  for (int k = lane; k < gw.nblk; k += 64) nn += work[gw.norm + k].x;
+  const double xnorm = sqrt(wsum(nn));
+  const cd alpha = work[c + 1];
+  double beta;
+  cd tv, scale;
+  house(alpha, xnorm, beta, tv, scale);
+  const bool ident = tv.x == 0.0 && tv.y == 0.0;
+  auto vec = [&](int r) {
+    if (r <= c || r >= N) return mk(0.0, 0.0);
+    if (r == c + 1) return mk(1.0, 0.0);
+    return ident ? mk(0.0, 0.0) : cmul(work[r], scale);
+  };
+  if ((int)blockIdx.x < ngemv) {
+    const int rt = blockIdx.x % nrow, sp = blockIdx.x / nrow;
+    const int c0 = c + 1 + sp * GS_C;
+    if (t < GS_C) vs[t] = vec(c0 + t);
+    __syncthreads();
+    const int r = p + 1 + rt * GS_G + t;
+    if (r >= N) return;
+    const int nc = N - c0 < GS_C ? N - c0 : GS_C;
+    const cd* ar = A + r + (long)c0 * lda;
+    double sr = 0.0, si = 0.0;
+    int k = 0;
+    for (; k + 8 <= nc; k += 8) {
+      cd a[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[u] = ar[(long)(k + u) * lda];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const cd v = vs[k + u];
+        sr += a[u].x * v.x - a[u].y * v.y;
+        si += a[u].x * v.y + a[u].y * v.x;
+      }
+    }
+    for (; k < nc; ++k) {
+      const cd a = ar[(long)k * lda], v = vs[k];
+      sr += a.x * v.x - a.y * v.y;
+      si += a.x * v.y + a.y * v.x;
+    }
+    work[gw.part + (long)sp * N + r] = mk(sr, si);
+    return;
+  }
+  const int blk = blockIdx.x - ngemv;
+  const int r = p + 1 + blk * GS_R + lane;
+  const cd v = vec(r);
+  if (q == 0 && r < N) {
+    V[r + (long)c * N] = v;
+    if (r == c + 1)
+      A[r + (long)c * lda] = ident ? alpha : mk(beta, 0.0);
+    else if (r > c + 1)
+      A[r + (long)c * lda] = mk(0.0, 0.0);
+  }
+  if (blk == 0 && t == 0) tau[c] = tv;
+  block_dots(N, p, j, V, r, v, work + gw.z + (long)blk * HB);
+}
+
+// Spread the panel when the matrices alone would leave most CUs idle and the trailing matrix is
+// large enough to pay for three launches a column. Hessenberg stage, ms, one workgroup / spread:
+// N = 162 1 matrix 4.2 / 4.0, 64 5.3 / 5.6; N = 242 10 8.4 / 6.7, 40 9.9 / 8.9, 100 11.0 / 11.4;
+// N = 450 10 25.0 / 16.6, 40 27.4 / 22.6, 80 30.5 / 30.6; N = 882 1 100 / 28, 10 109 / 41,
+// 60 136 / 107, 130 175 / 196.
+static bool gehrd_spread(int n, int batch) { return n >= 200 && batch <= 64; }
+
 static int n_reflectors(int n) { return n >= 3 ? n - 2 : 0; }
 
 // A <- H (Hessenberg, zeros below the subdiagonal). Vf (n x n) receives the
@@ -345,10 +579,27 @@ static void gehrd(hipStream_t s, int n, cd* A, long lda, long sA, cd* Vf, cd* Ta
   cd* W2 = W2b.as<cd>();
   const long sV = (long)n * n, sY = (long)n * HB, sT = (long)npanel * HB * HB, sW = (long)HB * n;
   const cd one = mk(1.0, 0.0), mone = mk(-1.0, 0.0), zero = mk(0.0, 0.0);
+  const bool spread = gehrd_spread(n, batch);
+  DevBuf workb;
+  if (spread) workb = ws.get(sizeof(cd) * (size_t)GehrdWork(n, 0).size * batch);
   for (int p = 0; p < nref; p += HB) {
     const int nb = nref - p < HB ? nref - p : HB;
     cd* Tp = Tall + (long)(p / HB) * HB * HB;
-    if (n - 1 <= 256)
+    if (spread) {
+      const GehrdWork gw(n, p);
+      cd* work = workb.as<cd>();
+      const int nrow = cdiv_up(n - p - 1, GS_G);
+      const dim3 rows(gw.nblk, batch);
+      for (int j = 0; j <= nb; ++j) {
+        gehrd_col_a_kernel<<<rows, 256, 0, s>>>(n, p, nb, j, A, lda, sA, Vf, sV, Y, sY, Tp, sT, taub.as<cd>(), n, work,
+                                                gw);
+        if (j == nb) break;
+        gehrd_col_b_kernel<<<rows, 256, 0, s>>>(n, p, j, A, lda, sA, Vf, sV, Tp, sT, work, gw);
+        const int ngemv = nrow * cdiv_up(n - (p + j) - 1, GS_C);
+        gehrd_col_c_kernel<<<dim3(ngemv + gw.nblk, batch), 256, 0, s>>>(n, p, j, A, lda, sA, Vf, sV, taub.as<cd>(), n,
+                                                                        work, gw, nrow, ngemv);
+      }
+    } else if (n - 1 <= 256)
       gehrd_panel_kernel<256><<<batch, 256, 2 * sizeof(cd) * n, s>>>(n, p, nb, A, lda, sA, Vf, sV, Y, sY, Tp, sT,
                                                                      taub.as<cd>(), n);
     else if (n - 1 <= 512)
