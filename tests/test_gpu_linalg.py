@@ -115,6 +115,47 @@ def test_getrf_matches_lapack(ctx, n):
         assert np.abs(LU[b] - lu_ref).max() <= 1e-11 * np.abs(lu_ref).max()
 
 
+@pytest.mark.parametrize("kind", ["dense", "ties"])
+@pytest.mark.parametrize("n,batch", [(1, 2), (15, 3), (16, 2), (17, 5), (63, 2), (65, 2), (127, 1), (129, 3),
+                                     (256, 1), (257, 2), (513, 1), (1024, 1)])
+def test_getrf_panel_edges(ctx, n, batch, kind):
+    """Backward error of the factors and of a solve at the edges of the panels (16), diagonal
+    blocks (64), outer blocks (128) and panel thread counts (256, 512, 1024); "ties" has many
+    equal pivot candidates. Bound: |P A - L U| <= gamma_n |L| |U|, gamma_n = 2 sqrt(2) n eps for
+    complex products, here with 4 n eps; the solve's with the two triangular solves (three times
+    that, and inverted 64-blocks whose condition the well-scaled factors keep below n)."""
+    import torch
+    rng = np.random.default_rng(n + batch)
+    A = crand(rng, batch, n, n)
+    if kind == "ties":
+        A = np.round(A) + 0j
+        A[:, np.arange(n), np.arange(n)] += 0.5
+    dA = to_dev_colmajor(A)
+    ipiv = torch.zeros(batch, n, dtype=torch.int32, device="cuda")
+    info = torch.zeros(batch, dtype=torch.int32, device="cuda")
+    ctx.check(ctx.lib.vrc_zgetrf(ctx.h, n, ptr(dA), n, n * n, ptr(ipiv), n, ptr(info), batch), "getrf")
+    assert int(info.abs().max()) == 0
+    LU, pv = from_dev_colmajor(dA), ipiv.cpu().numpy()
+    eps = np.finfo(float).eps
+    for b in range(batch):
+        L, U = np.tril(LU[b], -1) + np.eye(n), np.triu(LU[b])
+        PA = A[b].copy()
+        for i, p in enumerate(pv[b]):
+            assert i <= p < n
+            PA[[i, p]] = PA[[p, i]]
+        assert np.abs(np.tril(LU[b], -1)).max(initial=0.0) <= np.sqrt(2) * (1 + 1e-12)
+        assert np.all(np.abs(PA - L @ U) <= 4 * n * eps * (np.abs(L) @ np.abs(U)))
+    x = crand(rng, batch, n, 3)
+    dB, dX = to_dev_colmajor(A @ x), to_dev_colmajor(x * 0)
+    ctx.check(ctx.lib.vrc_zgetrs(ctx.h, n, 3, ptr(dA), n, n * n, ptr(ipiv), n, ptr(dB), n, 3 * n, ptr(dX), n, 3 * n,
+                                 batch), "getrs")
+    X = from_dev_colmajor(dX)
+    for b in range(batch):
+        r = np.abs(A[b] @ X[b] - A[b] @ x[b]).max()
+        bound = np.abs(np.tril(LU[b], -1) + np.eye(n)) @ np.abs(np.triu(LU[b])) @ np.abs(X[b])
+        assert r <= 12 * n * n * eps * bound.max()
+
+
 def test_getrf_zero_column_info(ctx):
     """A zero column inside a panel: info names it (1-based), as LAPACK's."""
     import torch

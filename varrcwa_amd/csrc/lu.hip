@@ -8,6 +8,8 @@
 // getrs: rows gathered through the final permutation, then blocked forward/backward
 // substitution (64-row diagonal blocks applied through their inverses, off-diagonal
 // updates on ZGEMM).
+#include <type_traits>
+
 #include "vrc_common.hpp"
 #include "vrc_internal.hpp"
 
@@ -88,15 +90,62 @@ __global__ __launch_bounds__(256) void getrf_panel_kernel(int n, int k, int kb, 
 }
 
 // Register-resident panel for n - k <= LUR_ROWS: thread t holds row k + t of the
-// kb <= LUR_NB panel columns. Per column (one barrier): wave arg-max (first index of the
-// largest |re|+|im|) posted with the candidate row, row exchange through LDS, elimination
+// kb <= LUR_NB panel columns. Per column (one barrier): wave maximum and its first row (largest
+// |re|+|im|, first index) posted with the candidate row, row exchange through LDS, elimination
 // in registers. Afterwards the panel's interchanges are applied to the other columns
 // [K, K+KB) of the block and, right of the panel, U12 = L11^{-1} A12 is solved (one
 // thread per column).
+// A panel is a serial chain and bound by its latencies, so nothing in it waits for memory but
+// the first and the last loads: pivots go to memory after the columns (a store before each
+// barrier was waited for), the rows of the other columns that the panel swaps are loaded
+// with the panel, their interchanges are one permutation (all loads, then all stores; in order
+// they were 16 dependent round trips), and U12 is solved by 16-column waves from LDS. Rows keep
+// their thread and exchange their places only; the columns rotate through the registers (a
+// ring, the finished ones behind the active ones), so that the loop over the columns stays one
+// copy of its code; the maximum goes over DPP lane moves. Per panel: n = 98 to 242
+// 43 -> 30-33 us, n = 450 51 -> 38 us, n = 882 67 -> 56 us (the elimination of 16 waves).
 constexpr int LUR_NB = 16;
 constexpr int LUR_ROWS = 1024;
 
-// ROWS threads (one row each; ROWS >= n - k): 256 or 512 for small n, so that four or two
+// x - l * y with the roundings spelled out: which product of the imaginary part is rounded
+// would otherwise be the compiler's choice at each place.
+__device__ __forceinline__ cd sub_mul(cd x, cd l, cd y) {
+  const double rr = l.y * y.y, ri = l.y * y.x;
+  return mk(x.x - __builtin_fma(l.x, y.x, -rr), x.y - __builtin_fma(l.x, y.y, ri));
+}
+
+// v and the value DPP control CTRL brings, lanes without a source keeping v.
+template <int CTRL>
+__device__ __forceinline__ double dpp_max(double v) {
+  const int hi = __double2hiint(v), lo = __double2loint(v);
+  const double o = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false),
+                                    __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false));
+  return fmax(v, o);
+}
+__device__ __forceinline__ double read_lane(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// Largest value of the first 16 lanes (no NaN among the lanes' values), in every lane.
+__device__ __forceinline__ double row_max_dpp(double v) {
+  v = dpp_max<0x111>(v);  // row_shr 1, 2, 4, 8: the last lane of every 16 has its row's maximum
+  v = dpp_max<0x112>(v);
+  v = dpp_max<0x114>(v);
+  v = dpp_max<0x118>(v);
+  return read_lane(v, 15);
+}
+// Largest value of the wavefront (no NaN among the lanes' values), in every lane.
+__device__ __forceinline__ double wave_max_dpp(double v) {
+  v = dpp_max<0x111>(v);
+  v = dpp_max<0x112>(v);
+  v = dpp_max<0x114>(v);
+  v = dpp_max<0x118>(v);
+  v = dpp_max<0x142>(v);  // row_bcast 15, 31: lane 63 has the wavefront's
+  v = dpp_max<0x143>(v);
+  return read_lane(v, 63);
+}
+
+// ROWS threads (one row each; ROWS >= n - k): 256 or 512 for small n, so that three or two
 // matrices share a CU (at most 128 VGPRs).
 template <int ROWS>
 __global__ __launch_bounds__(ROWS) __attribute__((amdgpu_waves_per_eu(4))) void getrf_panel_reg_kernel(
@@ -105,112 +154,209 @@ __global__ __launch_bounds__(ROWS) __attribute__((amdgpu_waves_per_eu(4))) void 
   A += b * sA;
   ipiv += b * sP;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int r = k + t;
-  const bool own = r < n;
-  // One barrier per column: every wave posts its best candidate and that candidate's
-  // row, the owner of row c posts row c; buffers alternate between columns.
+  const bool own = k + t < n;
+  // One barrier per column: every wave posts its best candidate and that candidate's row;
+  // buffers alternate between columns.
   constexpr int NW = ROWS / 64;
   __shared__ double wv[2][NW];
   __shared__ int wi[2][NW];
   __shared__ cd wrow[2][NW][LUR_NB];
-  __shared__ cd crow[2][LUR_NB];
   __shared__ cd L11[LUR_NB][LUR_NB + 1];
   __shared__ int pvs[LUR_NB];
+  __shared__ int top[LUR_NB], lowdst[LUR_NB], lowsrc[LUR_NB];  // the panel's interchanges
+  __shared__ cd seg[LUR_NB][LU_NB2 + 1];                       // rows k .. k+15 of the other columns
+  const int nleft = k - K, nother = KB - kb;
+  auto column = [&](int c) { return A + (long)(c < nleft ? K + c : k + kb + (c - nleft)) * lda; };
+  // a ring: a[q] is column j + q of the panel at step j, finished columns follow the active ones
   cd a[LUR_NB];
+  {
+    const cd* ar = A + (own ? k + t : k);
 #pragma unroll
-  for (int j = 0; j < LUR_NB; ++j) a[j] = (own && j < kb) ? A[r + (long)(k + j) * lda] : mk(0.0, 0.0);
+    for (int q = 0; q < LUR_NB; ++q) a[q] = ar[(long)(k + (q < kb ? q : 0)) * lda];
+  }
+  constexpr int EPT = LUR_NB * LU_NB2 / ROWS;  // elements of seg per thread
+  if (nother > 0) {
+    double wx[EPT], wy[EPT];
 #pragma unroll
-  for (int j = 0; j < LUR_NB; ++j) {
-    if (j < kb) {
-      const int par = j & 1;
-      const int c = k + j;
-      double v = -1.0;
-      int vi = 0x7fffffff;
-      if (own && r >= c) {
-        const double m = cabs1(a[j]);
-        if (m > v) { v = m; vi = r; }  // NaN never wins
-      }
-      for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(v, o, 64);
-        const int oi = __shfl_xor(vi, o, 64);
-        if (ov > v || (ov == v && oi < vi)) { v = ov; vi = oi; }
-      }
-      if (lane == 0) { wv[par][wave] = v; wi[par][wave] = vi; }
-      if (own && r == vi) {
+    for (int r = 0; r < EPT; ++r) {
+      const int e = t + r * ROWS, i = e % LUR_NB, c = e / LUR_NB;
+      const cd w = column(c < nother ? c : 0)[k + (i < kb ? i : 0)];
+      wx[r] = w.x;
+      wy[r] = w.y;
+    }
 #pragma unroll
-        for (int jj = 0; jj < LUR_NB; ++jj) wrow[par][wave][jj] = a[jj];
-      }
-      if (own && r == c) {
-#pragma unroll
-        for (int jj = 0; jj < LUR_NB; ++jj) crow[par][jj] = a[jj];
-      }
-      __syncthreads();
-      double best = wv[par][0];
-      int bi = wi[par][0], bw = 0;
-      for (int w = 1; w < NW; ++w) {
-        const double ov = wv[par][w];
-        const int oi = wi[par][w];
-        if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; bw = w; }
-      }
-      const int p = (bi >= c && bi < n) ? bi : c;
-      if (t == 0) { ipiv[c] = p; pvs[j] = p; }
-      const bool nonsing = best > 0.0;
-      if (!nonsing && t == 0 && info && info[b] == 0) info[b] = c + 1;  // getf2 semantics: no elimination
-      if (nonsing) {
-        const cd* prow = wrow[par][bw];  // row p
-        if (p != c && r == c) {
-#pragma unroll
-          for (int jj = 0; jj < LUR_NB; ++jj) a[jj] = prow[jj];
-        } else if (p != c && r == p) {
-#pragma unroll
-          for (int jj = 0; jj < LUR_NB; ++jj) a[jj] = crow[par][jj];
-        }
-        if (own && r > c) {
-          const cd l = cmul(a[j], crecip(prow[j]));
-          a[j] = l;
-#pragma unroll
-          for (int jj = 0; jj < LUR_NB; ++jj)
-            if (jj > j && jj < kb) a[jj] = csub(a[jj], cmul(l, prow[jj]));
-        }
-      }
+    for (int r = 0; r < EPT; ++r) {
+      const int e = t + r * ROWS;
+      seg[e % LUR_NB][e / LUR_NB] = mk(wx[r], wy[r]);
     }
   }
+  int pos = own ? k + t : 0x7fffffff;  // the row's place after the exchanges so far
+  int sing = -1;                       // first column without a pivot
+  for (int e = t; e < LUR_NB * (LUR_NB + 1); e += ROWS) (&L11[0][0])[e] = mk(0.0, 0.0);
+#pragma unroll 1
+  for (int j = 0; j < kb; ++j) {
+    const int par = j & 1;
+    const int c = k + j;
+    double v = -1.0;
+    if (own && pos >= c) {
+      const double m = cabs1(a[0]);
+      if (m > v) v = m;  // NaN never wins
+    }
+    const double vm = wave_max_dpp(v);
+    unsigned long long eq = __ballot(v == vm);
+    int best_pos = 0x7fffffff;
+    if (vm >= 0.0) {
+      best_pos = __builtin_amdgcn_readlane(pos, __ffsll(eq) - 1);
+      for (eq &= eq - 1; eq; eq &= eq - 1) {  // equal values: the first row
+        const int o = __builtin_amdgcn_readlane(pos, __ffsll(eq) - 1);
+        best_pos = o < best_pos ? o : best_pos;
+      }
+    }
+    if (lane == 0) {
+      wv[par][wave] = vm;
+      wi[par][wave] = best_pos;
+    }
+    if (own && pos == best_pos) {
+#pragma unroll
+      for (int q = 0; q < LUR_NB; ++q) wrow[par][wave][q] = a[q];
+    }
+    __syncthreads();
+    const double ov = wv[par][lane & (NW - 1)];
+    const int oi = wi[par][lane & (NW - 1)];
+    const double best = row_max_dpp(ov);
+    unsigned win = (unsigned)__ballot(ov == best) & ((1u << NW) - 1u);
+    int bw = __ffs(win) - 1;
+    int bi = __builtin_amdgcn_readlane(oi, bw);
+    for (win &= win - 1; win; win &= win - 1) {
+      const int w = __ffs(win) - 1;
+      const int o = __builtin_amdgcn_readlane(oi, w);
+      if (o < bi) {
+        bi = o;
+        bw = w;
+      }
+    }
+    const int p = (bi >= c && bi < n) ? bi : c;
+    if (t == 0) pvs[j] = p;
+    const bool nonsing = best > 0.0;
+    const cd* prow = wrow[par][bw];
+    cd l = a[0];
+    bool below = false;
+    if (!nonsing) {  // getf2 semantics: no elimination
+      if (sing < 0) sing = c;
+    } else {
+      pos = pos == p ? c : (pos == c ? p : pos);
+      below = own && pos > c;
+      const cd m = cmul(a[0], crecip(prow[0]));
+      l.x = below ? m.x : l.x;
+      l.y = below ? m.y : l.y;
+    }
+    const int act = kb - j;  // ring places 1 .. act - 1 are eliminated
+#pragma unroll
+    for (int q = 1; q < LUR_NB; ++q) {
+      const cd x = a[q], y = csub(x, cmul(l, prow[q]));
+      const bool u = below & (q < act);
+      a[q - 1].x = u ? y.x : x.x;
+      a[q - 1].y = u ? y.y : x.y;
+    }
+    a[LUR_NB - 1] = l;
+  }
+  for (int j = kb; j < LUR_NB; ++j) {  // the ring's full turn
+    const cd l = a[0];
+#pragma unroll
+    for (int q = 1; q < LUR_NB; ++q) a[q - 1] = a[q];
+    a[LUR_NB - 1] = l;
+  }
+  if (own && pos < k + kb) {
+#pragma unroll
+    for (int j = 0; j < LUR_NB; ++j) L11[pos - k][j] = a[j];
+  }
+  if (t == 0 && sing >= 0 && info && info[b] == 0) info[b] = sing + 1;
+  __syncthreads();
+  if (t < kb) ipiv[k + t] = pvs[t];
   if (own) {
 #pragma unroll
     for (int j = 0; j < LUR_NB; ++j)
-      if (j < kb) A[r + (long)(k + j) * lda] = a[j];
+      if (j < kb) A[pos + (long)(k + j) * lda] = a[j];
   }
-  if (t < kb) {
-#pragma unroll
-    for (int j = 0; j < LUR_NB; ++j) L11[t][j] = a[j];
+  // The interchanges as one permutation, by the first wave: lane i < 16 stands for row k + i,
+  // lane 16 + j for the row p_j below the panel's (its first j if several columns chose it);
+  // each lane holds the row whose values are there after the swaps so far. A row below ends
+  // with the values of one of the rows k .. k+kb-1 (or its own).
+  if (nother == 0) return;
+  if (wave == 0) {
+    const int pj = lane < kb ? pvs[lane] : -1;
+    int slot = pj >= k + kb ? LUR_NB + lane : pj - k;
+    for (int q = kb - 2; q >= 0; --q) {
+      const int pq = __builtin_amdgcn_readlane(pj, q);
+      if (lane > q && lane < kb && pj == pq && pj >= k + kb) slot = LUR_NB + q;
+    }
+    const int far = __shfl(pj, lane & (LUR_NB - 1), 64);
+    int row = lane < LUR_NB ? k + lane : far;
+    const int home = row;
+    for (int j = 0; j < kb; ++j) {
+      const int sj = __builtin_amdgcn_readlane(slot, j);
+      const int x = __builtin_amdgcn_readlane(row, j), y = __builtin_amdgcn_readlane(row, sj);
+      if (lane == j) row = y;
+      if (lane == sj) row = x;
+    }
+    const int mine = __shfl(slot, lane & (LUR_NB - 1), 64);  // lane 16 + j: the slot column j swapped with
+    if (lane < LUR_NB) top[lane] = lane < kb ? row : k;
+    if (lane >= LUR_NB && lane < 2 * LUR_NB) {
+      const int j = lane - LUR_NB;
+      lowdst[j] = (j < kb && mine == lane && row != home) ? home : -1;
+      lowsrc[j] = row - k;
+    }
   }
   __syncthreads();
-  // the block's other columns: interchanges, and U12 right of the panel
-  const int nleft = k - K, nother = KB - kb;
-  if (t < nother) {
-    const int col = t < nleft ? K + t : k + kb + (t - nleft);
-    cd* ac = A + (long)col * lda;
-    for (int j = 0; j < kb; ++j) {
-      const int p = pvs[j];
-      if (p != k + j) {
-        const cd tmp = ac[k + j];
-        ac[k + j] = ac[p];
-        ac[p] = tmp;
+  // The block's other columns: all values are read before any is written.
+  double yx[EPT], yy[EPT], zx[EPT], zy[EPT];
+  int dst[EPT];
+#pragma unroll
+  for (int r = 0; r < EPT; ++r) {
+    const int e = t + r * ROWS, i = e % LUR_NB, c = e / LUR_NB;
+    const cd y = column(c < nother ? c : 0)[top[i]];
+    yx[r] = y.x;
+    yy[r] = y.y;
+    dst[r] = c < nother ? lowdst[i] : -1;
+    const cd z = seg[dst[r] >= 0 ? lowsrc[i] : 0][c];
+    zx[r] = z.x;
+    zy[r] = z.y;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < EPT; ++r) {
+    const int e = t + r * ROWS, i = e % LUR_NB, c = e / LUR_NB;
+    seg[i][c] = mk(yx[r], yy[r]);
+    if (dst[r] >= 0) column(c)[dst[r]] = mk(zx[r], zy[r]);
+    if (c < nleft && i < kb) column(c)[k + i] = mk(yx[r], yy[r]);
+  }
+  __syncthreads();
+  // Right of the panel U12 = L11^{-1} A12: 16 columns per wave, lane (g, c) has the rows
+  // 4 q + g of column c.
+  const int g = lane >> 4;
+  for (int c0 = nleft + 16 * wave; c0 < nother; c0 += 16 * NW) {
+    const int c = c0 + (lane & 15);
+    cd x[LUR_NB / 4];
+#pragma unroll
+    for (int q = 0; q < LUR_NB / 4; ++q) x[q] = seg[4 * q + g][c < nother ? c : c0];
+#pragma unroll
+    for (int i = 0; i < LUR_NB - 1; ++i) {
+      asm volatile("" ::: "memory");  // L11 column by column: all of it at once would not fit in registers
+      const int src = (i & 3) * 16 + (lane & 15);
+      const cd xi = mk(__shfl(x[i >> 2].x, src, 64), __shfl(x[i >> 2].y, src, 64));
+#pragma unroll
+      for (int q = i >> 2; q < LUR_NB / 4; ++q) {
+        const cd d = sub_mul(x[q], xi, L11[4 * q + g][i]);
+        const bool u = 4 * q + g > i;
+        x[q].x = u ? d.x : x[q].x;
+        x[q].y = u ? d.y : x[q].y;
       }
     }
-    if (col >= k + kb) {
-      cd x[LUR_NB];
+    if (c < nother) {
 #pragma unroll
-      for (int i = 0; i < LUR_NB; ++i) {
-        if (i < kb) {
-          cd xi = ac[k + i];
-#pragma unroll
-          for (int j = 0; j < LUR_NB; ++j)
-            if (j < i) xi = csub(xi, cmul(L11[i][j], x[j]));
-          x[i] = xi;
-          ac[k + i] = xi;
-        }
-      }
+      for (int q = 0; q < LUR_NB / 4; ++q)
+        if (4 * q + g < kb) column(c)[k + 4 * q + g] = x[q];
     }
   }
 }
@@ -459,46 +605,101 @@ __global__ void gather_rows_kernel(int n, int nrhs, const int* perm, long sPerm,
 
 // Inverse of every TRS_NB x TRS_NB diagonal block of a triangular factor (UPPER=0: unit
 // lower, UPPER=1: non-unit upper) into Dinv[b][blk] (TRS_NB x TRS_NB, zero padded past
-// the block size). One workgroup per block: thread (column j, quarter q) substitutes
-// the identity column j, rows split over the four quarters.
+// the block size). One workgroup per block, 16 columns per wave: lane (g, c) holds the rows
+// j = 4 q + g of column c in registers, so that the substitution of a column stays within its
+// wave: a lane exchange per step where X in LDS took two barriers and a read and write of X
+// (lower 50 -> 25 us, upper 60 -> 33 us per launch; now bound by the 64 dependent steps, for
+// the upper with a division each). The rows rotate through the registers (x[q] is row group
+// iq + q, from the other end for UPPER), which keeps the code one copy per four groups; the
+// divisors of cdiv are prepared once per row.
 template <int UPPER>
 __global__ __launch_bounds__(256) void trtri_blocks_kernel(int n, const cd* T, long ldt, long sT, cd* Dinv,
                                                            long sD) {
+  constexpr int NQ = TRS_NB / 4;
   const long b = blockIdx.y;
   const int blk = blockIdx.x;
   const int k0 = blk * TRS_NB;
   const int bs = n - k0 < TRS_NB ? n - k0 : TRS_NB;
   T += b * sT;
   cd* D = Dinv + b * sD + (long)blk * TRS_NB * TRS_NB;
-  __shared__ cd Ls[TRS_NB][TRS_NB + 1];
-  __shared__ cd Xs[TRS_NB][TRS_NB + 1];
+  // PAD rows of other values beyond the end the substitution runs to: read, never used
+  constexpr int PAD = 12, LO = UPPER ? PAD : 0;
+  __shared__ cd Ls[TRS_NB + PAD][TRS_NB + 1];
+  __shared__ double ratio[TRS_NB], den[TRS_NB];  // cdiv by the diagonal (Smith): ratio, divisor
+  __shared__ int ybig[TRS_NB];
   const int t = threadIdx.x;
-  for (int e = t; e < TRS_NB * TRS_NB; e += 256) {
-    const int i = e % TRS_NB, j = e / TRS_NB;
-    Ls[i][j] = (i < bs && j < bs) ? T[(k0 + i) + (long)(k0 + j) * ldt] : mk(0.0, 0.0);
-    Xs[i][j] = (i == j && i < bs) ? mk(1.0, 0.0) : mk(0.0, 0.0);
+#pragma unroll 8
+  for (int r = 0; r < TRS_NB * TRS_NB / 256; ++r) {
+    const int e = t + 256 * r, i = e % TRS_NB, j = e / TRS_NB;
+    const bool in = i < bs && j < bs;
+    const cd v = T[(k0 + (i < bs ? i : 0)) + (long)(k0 + (j < bs ? j : 0)) * ldt];
+    Ls[LO + i][j] = mk(in ? v.x : 0.0, in ? v.y : 0.0);
   }
   __syncthreads();
-  const int col = t & 63, grp = t >> 6;
-  if (!UPPER) {
-    for (int i = 0; i < bs; ++i) {
-      const cd xi = Xs[i][col];
-      for (int j = i + 1 + grp; j < bs; j += 4) Xs[j][col] = csub(Xs[j][col], cmul(Ls[j][i], xi));
-      __syncthreads();
+  if (UPPER) {
+    if (t < bs) {
+      const cd d = Ls[LO + t][t];
+      const bool yb = !(fabs(d.y) <= fabs(d.x));
+      const double big = yb ? d.y : d.x, small = yb ? d.x : d.y;
+      const double r = small / big;
+      ratio[t] = r;
+      den[t] = big + small * r;
+      ybig[t] = yb ? 1 : 0;
     }
-  } else {
-    for (int i = bs - 1; i >= 0; --i) {
-      if (grp == 0 && col < bs) Xs[i][col] = cdiv(Xs[i][col], Ls[i][i]);
-      __syncthreads();
-      const cd xi = Xs[i][col];
-      for (int j = grp; j < i; j += 4) Xs[j][col] = csub(Xs[j][col], cmul(Ls[j][i], xi));
-      __syncthreads();
+    __syncthreads();
+  }
+  const int lane = t & 63, g = lane >> 4;
+  const int col = (t >> 6) * 16 + (lane & 15);
+  // x[q]: row group q from the end the substitution starts at
+  cd x[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int j = 4 * (UPPER ? NQ - 1 - q : q) + g;
+    x[q] = mk(j == col && col < bs ? 1.0 : 0.0, 0.0);
+  }
+  // Four row groups of the substitution from group FROM on; x[0 .. LEFT) can still change. The
+  // group of row i itself is the only one of which some rows are done; rows past the block
+  // size meet zeros of Ls.
+  auto run = [&](auto from) {
+    constexpr int FROM = decltype(from)::value, LEFT = NQ - FROM;
+#pragma unroll 1
+    for (int iq = FROM; iq < FROM + 4; ++iq) {
+      const int grp = UPPER ? NQ - 1 - iq : iq;
+#pragma unroll 1
+      for (int s = 0; s < 4; ++s) {
+        const int ig = UPPER ? 3 - s : s;
+        const int i = 4 * grp + ig;
+        if (i >= bs) continue;
+        cd xi = x[0];
+        if (UPPER) {
+          const double r = ratio[i], dd = den[i];
+          const bool yb = ybig[i] != 0;
+          const double nx = yb ? xi.x * r + xi.y : xi.x + xi.y * r;
+          const double ny = yb ? xi.y * r - xi.x : xi.y - xi.x * r;
+          xi = mk(nx / dd, ny / dd);
+          x[0].x = g == ig ? xi.x : x[0].x;
+          x[0].y = g == ig ? xi.y : x[0].y;
+        }
+        const int src = ig * 16 + (lane & 15);
+        xi = mk(__shfl(xi.x, src, 64), __shfl(xi.y, src, 64));
+        const cd* lc = &Ls[LO + 4 * grp + g][i];
+        const cd y = sub_mul(x[0], lc[0], xi);
+        const bool upd = UPPER ? g < ig : g > ig;
+        x[0].x = upd ? y.x : x[0].x;
+        x[0].y = upd ? y.y : x[0].y;
+#pragma unroll
+        for (int q = 1; q < LEFT; ++q)
+          x[q] = sub_mul(x[q], lc[(UPPER ? -4 : 4) * q * (TRS_NB + 1)], xi);
+      }
+      D[4 * grp + g + (long)col * TRS_NB] = x[0];
+#pragma unroll
+      for (int q = 1; q < LEFT; ++q) x[q - 1] = x[q];
     }
-  }
-  for (int e = t; e < TRS_NB * TRS_NB; e += 256) {
-    const int i = e % TRS_NB, j = e / TRS_NB;
-    D[i + (long)j * TRS_NB] = Xs[i][j];
-  }
+  };
+  run(std::integral_constant<int, 0>{});
+  run(std::integral_constant<int, NQ / 4>{});
+  run(std::integral_constant<int, NQ / 2>{});
+  run(std::integral_constant<int, 3 * NQ / 4>{});
 }
 
 // In-place triangular solve on Y (n x nrhs): UPPER=0 -> L (unit) ; UPPER=1 -> U (non-unit).
