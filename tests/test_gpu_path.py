@@ -11,7 +11,7 @@ import pytest
 
 from oracle import rcwa_oracle as O
 from tests import geometries as G
-from varrcwa_amd import api
+from varrcwa_amd import VrcError, api
 from varrcwa_amd._lib import from_dev_colmajor, to_dev_colmajor
 
 pytestmark = pytest.mark.gpu
@@ -93,6 +93,31 @@ def test_fourier_pixel_grids_fft_path(ctx):
                 ref = O.fourier2d(x, y, eps, nx, ny, opt)
                 got = fe[k, i].T
                 assert rel(got, ref) < 1e-12, (nx, ny, i, k, rel(got, ref))
+
+
+@pytest.mark.parametrize("crossing", [False, True])
+def test_fourier_cell_order(ctx, crossing):
+    """Layers of unequal sizes in one batch (cells at the edges of the 16 x 16 transposition),
+    with sorted and with crossing x coordinates (painter's order), against the oracle at the
+    1e-12 of the other assembly checks."""
+    rng = np.random.default_rng(23)
+    layers = []
+    for ncx, ncy in [(1, 1), (15, 17), (16, 16), (17, 15), (33, 2), (1, 31)]:
+        x = np.concatenate([[0.0], np.sort(rng.uniform(0.05, 0.75, ncx - 1)), [0.8]])
+        y = np.concatenate([[0.0], np.sort(rng.uniform(0.05, 0.75, ncy - 1)), [0.8]])
+        if crossing and ncx > 4:
+            x[2:5] = x[[4, 2, 3]]
+        layers.append((x, y, 1 + 11.25 * rng.random((ncy, ncx)) + 0.3j * rng.random((ncy, ncx))))
+    fe = api.assemble_toeplitz(ctx, 5, 7, layers).cpu().numpy()
+    for i, (x, y, eps) in enumerate(layers):
+        for k, opt in enumerate([O.DISCONTINUOUS_X, O.DISCONTINUOUS_Y, O.CONTINUOUS_XY]):
+            ref = O.fourier2d(x, y, eps, 5, 7, opt)
+            assert rel(fe[k, i].T, ref) < 1e-12, (i, k, rel(fe[k, i].T, ref))
+    bad = [(x, y, np.where(np.arange(e.size).reshape(e.shape) == e.size - 1, v, e)) for (x, y, e), v in
+           zip(layers, [np.nan, np.inf, 0.0, np.nan * 1j, 0.0, -np.inf])]
+    for i, l in enumerate(bad):
+        with pytest.raises(VrcError):
+            api.assemble_toeplitz(ctx, 5, 7, layers[:i] + [l] + layers[i + 1:])
 
 
 @pytest.mark.parametrize("which", ["metasurface", "var12"])

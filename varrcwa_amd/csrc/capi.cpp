@@ -231,9 +231,13 @@ struct vrc_integrator {
 };
 
 namespace {
-HostLayer to_host(const vrc_layer* l) {
+LayerView view(const vrc_layer* l) {
   if (!l || !l->x || !l->y || !l->eps) throw ArgFailure("null layer field");
   if (l->ncoord_x < 2 || l->ncoord_y < 2) throw ArgFailure("layer needs >= 2 coordinates per axis");
+  return LayerView(l->x, l->ncoord_x, l->y, l->ncoord_y, l->eps);
+}
+HostLayer to_host(const vrc_layer* l) {
+  view(l);
   HostLayer h;
   h.x.assign(l->x, l->x + l->ncoord_x);
   h.y.assign(l->y, l->y + l->ncoord_y);
@@ -279,14 +283,12 @@ int vrc_assemble_toeplitz(vrc_ctx* c, int nx, int ny, int nlayers, const vrc_lay
     need(nlayers >= 0 && fe11 && fe22 && fe33, "bad arguments");
     const long n = (long)nx * ny;
     need(stride >= n * n || nlayers <= 1, "stride smaller than n*n");
-    std::vector<HostLayer> hl = to_host(layers, nlayers);
-    AssemblyBatch a;
-    a.nx = nx;
-    a.ny = ny;
-    a.nlayers = nlayers;
-    for (auto& l : hl) a.layers.push_back(&l);
+    need(nlayers == 0 || layers, "bad layer array");
     if (nlayers == 0) return;
-    assemble_fe(*c, a, (cd*)fe11, (cd*)fe22, (cd*)fe33, stride);
+    std::vector<LayerView> v;
+    v.reserve(nlayers);
+    for (int l = 0; l < nlayers; ++l) v.push_back(view(layers + l));
+    assemble_fe(*c, nx, ny, v, (cd*)fe11, (cd*)fe22, (cd*)fe33, stride);
   });
 }
 

@@ -298,7 +298,7 @@ void Sampler::shape_derivatives(const HostLayer& L, int nvar, const int* var_ind
 
 VarSampler::VarSampler(vrc_ctx* c, double lambda, int nx, int ny, HostLayer base, bool pml)
     : Sampler(c, lambda, nx, ny, pml), base_(std::move(base)) {
-  prepare_layer(base_);  // validates shapes
+  validate_layer(base_);
   post_init(base_.x, base_.y);
 }
 
@@ -323,9 +323,9 @@ StackSampler::StackSampler(vrc_ctx* c, double lambda, int nx, int ny, std::vecto
   if (ze_.size() != layers_.size() + 1) throw ArgFailure("need nlayers+1 z edges");
   for (size_t i = 0; i + 1 < ze_.size(); ++i)
     if (!(ze_[i + 1] > ze_[i])) throw ArgFailure("z edges must increase");
-  for (auto& l : layers_) prepare_layer(l);
-  prepare_layer(bottom_);
-  prepare_layer(top_);
+  for (auto& l : layers_) validate_layer(l);
+  validate_layer(bottom_);
+  validate_layer(top_);
   post_init(bottom_.x, bottom_.y);
 }
 
@@ -1194,8 +1194,8 @@ static void batch_stack_solve(vrc_ctx& c, int nx, int ny, const std::vector<Stac
       throw ArgFailure("all instances of one batch must have the same layer count");
     if (!I.bottom || !I.top) throw ArgFailure("instance without bottom/top medium");
     if (!(I.lambda > 0)) throw ArgFailure("wavelength must be positive");
-    prepare_layer(*I.bottom);  // validates the half-space media (their eps may take the closed form)
-    prepare_layer(*I.top);
+    validate_layer(*I.bottom);  // the half-space media (their eps may take the closed form)
+    validate_layer(*I.top);
   }
   // End media given by one permittivity value get their eigen-system in closed form.
   bool homog = true;

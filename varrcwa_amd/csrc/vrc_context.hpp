@@ -2,6 +2,7 @@
 #pragma once
 
 #include <atomic>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -23,6 +24,8 @@ struct PinnedPool {
   ~PinnedPool();
   // Copies host[0, bytes) into a pinned block and enqueues its copy to dst on stream s.
   void upload(hipStream_t s, void* dst, const void* host, size_t bytes);
+  // The same with the pinned block written by fill(block).
+  void upload_with(hipStream_t s, void* dst, size_t bytes, const std::function<void(char*)>& fill);
 };
 }  // namespace vrc
 

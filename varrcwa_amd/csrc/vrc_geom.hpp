@@ -18,6 +18,19 @@ struct HostLayer {
   cd at(int i, int j) const { return eps[(size_t)i + (size_t)j * ncy()]; }
 };
 
+// A layer's host arrays where they are: coordinates and interleaved permittivities (re, im),
+// ncy x ncx column-major.
+struct LayerView {
+  const double *x, *y, *eps;
+  int ncoord_x, ncoord_y;
+  size_t neps;
+  LayerView(const double* x_, int nx, const double* y_, int ny, const double* e)
+      : x(x_), y(y_), eps(e), ncoord_x(nx), ncoord_y(ny), neps((size_t)(nx - 1) * (ny - 1)) {}
+  LayerView(const HostLayer& L)
+      : x(L.x.data()), y(L.y.data()), eps((const double*)L.eps.data()), ncoord_x((int)L.x.size()),
+        ncoord_y((int)L.y.size()), neps(L.eps.size()) {}
+};
+
 constexpr int FOURIER_FFT_MAX = 2048;  // longest grid axis transformed by FFT (1.5 x that in LDS: 48 KB)
 
 // Device arrays for a batch of layers (capacities MX cells, MY strips per layer).

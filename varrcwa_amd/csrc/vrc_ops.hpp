@@ -32,14 +32,16 @@ void info_to_owner(hipStream_t s, const int* info, const int* owner, int njobs, 
 
 // ---------------------------------------------------------------- geometry (host)
 // FourierSolver1D::reorder/refill semantics (src/rcwa/FourierSolver1D.cpp:145-193)
-// applied to one layer: painter-order values and the two interval lists.
+// applied to one layer: painter-order cells and the two interval lists.
 struct PreparedLayer {
   std::vector<double> xu, xs, ys;
-  std::vector<cd> val;  // [strip][cell], ncy x ncx
+  std::vector<int> src;  // the given cell whose values each sorted cell ends with
   double Lx, Ly;
   int ncx, ncy;
 };
-PreparedLayer prepare_layer(const HostLayer& L);
+PreparedLayer prepare_layer(const LayerView& L);
+// Throws ArgFailure for shapes that do not fit and for a permittivity that is not finite or zero.
+void validate_layer(const HostLayer& L);
 
 // alpha/beta of LayerSampler::evaluateAlphaBeta (src/core/LayerSampler.cpp:9-32).
 void alpha_beta(int nx, int ny, double Lx, double Ly, std::vector<cd>& alpha, std::vector<cd>& beta);
@@ -69,6 +71,8 @@ struct AssemblyBatch {
   double k0sq_uniform = 0.0;
 };
 void assemble_fe(vrc_ctx& c, const AssemblyBatch& a, cd* fe11, cd* fe22, cd* fe33, long sfe);
+void assemble_fe(vrc_ctx& c, int nx, int ny, const std::vector<LayerView>& layers, cd* fe11, cd* fe22, cd* fe33,
+                 long sfe);
 
 // Uploaded layer batch and workspace of the Fourier kernels (device view in g).
 struct FourierStage {
@@ -77,6 +81,7 @@ struct FourierStage {
   int L = 0;
 };
 FourierStage fourier_prepare(vrc_ctx& c, int nx, int ny, const std::vector<const HostLayer*>& layers);
+FourierStage fourier_prepare(vrc_ctx& c, int nx, int ny, const std::vector<LayerView>& layers);
 // P, Q of every layer (N x N, stride N^2); PQ (optional) also receives P Q, for periodic
 // cells without the N x N product.
 void assemble_pq(vrc_ctx& c, const AssemblyBatch& a, cd* P, cd* Q, cd* PQ = nullptr);

@@ -140,12 +140,16 @@ PinnedPool::~PinnedPool() {
 }
 
 void PinnedPool::upload(hipStream_t s, void* dst, const void* host, size_t bytes) {
+  upload_with(s, dst, bytes, [&](char* p) { std::memcpy(p, host, bytes); });
+}
+
+void PinnedPool::upload_with(hipStream_t s, void* dst, size_t bytes, const std::function<void(char*)>& fill) {
   if (bytes == 0) return;
   void* p = nullptr;
   if (hold) {  // recording a graph: the block belongs to the recording
     VRC_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
     hold->push_back(p);
-    std::memcpy(p, host, bytes);
+    fill((char*)p);
     VRC_HIP(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, s));
     return;
   }
@@ -159,7 +163,7 @@ void PinnedPool::upload(hipStream_t s, void* dst, const void* host, size_t bytes
     blocks.push_back(b);
     blk = &blocks.back();
   }
-  std::memcpy(blk->p, host, bytes);
+  fill((char*)blk->p);
   VRC_HIP(hipMemcpyAsync(dst, blk->p, bytes, hipMemcpyHostToDevice, s));
   VRC_HIP(hipEventRecord(blk->ev, s));
 }
