@@ -287,18 +287,33 @@ def _eig_check_values(ctx, A):
 def test_zgeev_team_sizes(ctx, n):
     """Launches of 1, 9, 40, 70 and 128 matrices give the QR kernel teams of 16, 16, 6, 3 and 2
     workgroups per matrix, 129 none: the same matrix gives the same bits whatever the team (the
-    shares of a window product do not depend on who computes them). Up to 64 matrices the
-    Hessenberg panel sums in another order, so the two ranges are compared within themselves."""
+    shares of a window product do not depend on who computes them)."""
     rng = np.random.default_rng(4000 + n)
     A = crand(rng, 1, n, n)
-    for batches in ((1, 9, 40, 64), (129, 70, 128)):
-        ref = None
-        for batch in batches:
-            w, V = _eig_check_values(ctx, np.repeat(A, batch, axis=0)) if batch < 9 else _eig_values(ctx, A, batch)
-            if ref is None:
-                ref = (w[0], V[0])
-            for b in (0, batch // 2, batch - 1):
-                assert np.array_equal(w[b], ref[0]) and np.array_equal(V[b], ref[1]), (batch, b)
+    ref = None
+    for batch in (1, 9, 40, 64, 129, 70, 128):
+        w, V = _eig_check_values(ctx, np.repeat(A, batch, axis=0)) if batch < 9 else _eig_values(ctx, A, batch)
+        if ref is None:
+            ref = (w[0], V[0])
+        for b in (0, batch // 2, batch - 1):
+            assert np.array_equal(w[b], ref[0]) and np.array_equal(V[b], ref[1]), (batch, b)
+
+
+@pytest.mark.parametrize("n", [3, 17, 66, 67, 130, 162])
+def test_zgeev_wide_hessenberg(ctx, n):
+    """Up to 512 matrices take the Hessenberg panel with more loads in flight, more of them the
+    one with four workgroups per CU: the sums are the same, so are the bits. Sizes at the edges
+    of its column groups (8, 16), rows (64) and panels (64)."""
+    rng = np.random.default_rng(6000 + n)
+    A = crand(rng, 1, n, n)
+    assert ctx.lib.vrc_tune_set(b"zgeev.qr_variant", 4) == 0
+    try:
+        few, many = _eig_values(ctx, A, 2), _eig_values(ctx, A, 513)
+    finally:
+        ctx.lib.vrc_tune_set(b"zgeev.qr_variant", -1)
+    for b in (0, 512):
+        assert np.array_equal(few[0][0], many[0][b]) and np.array_equal(few[1][0], many[1][b])
+    _eig_check(ctx, A)
 
 
 @pytest.mark.parametrize("n", [200, 257, 258, 259, 322])

@@ -114,12 +114,64 @@ __device__ inline cd load_stream(const cd* p) {
   return mk(v.x, v.y);
 }
 
+// Sums v[0 .. NV) over the wavefront: the sum of v[k] ends in v[0] of the lanes with
+// lane / (64 / NV) = k. Each step pairs the same lanes as a butterfly over all values would
+// (the same sums), but lane halves keep half of the values each: 17 exchanges for 16 values
+// instead of 96.
+template <int NV>
+__device__ __forceinline__ void wave_sums(double (&v)[NV]) {
+  const int lane = threadIdx.x & 63;
+  int off = 32;
+#pragma unroll
+  for (int h = NV / 2; h >= 1; h /= 2, off /= 2) {
+    const bool up = lane & off;
+#pragma unroll
+    for (int k = 0; k < h; ++k) {
+      const double keep = up ? v[h + k] : v[k], send = up ? v[k] : v[h + k];
+      v[k] = keep + __shfl_xor(send, off, 64);
+    }
+  }
+#pragma unroll
+  for (; off >= 1; off /= 2) v[0] += __shfl_xor(v[0], off, 64);
+}
+
 // out[i] = sum_{r >= r0} conj(Vf[r, p+i]) x[r] for i < j (x in LDS): wave w reduces the
-// columns i = w, w + PTT/64, ... (the columns proceed in parallel, four loads in flight per
-// lane, rows summed in increasing order within a lane).
-template <int PTT>
+// columns i = w, w + PTT/64, ... (rows summed in increasing order within a lane). WIDE: NC = 8
+// columns at a time share the waits for loads and lane exchanges. Otherwise one at a time, four
+// loads in flight: the registers of the wide form would cost workgroups per CU (n = 882, 250
+// matrices, four columns at a time: 263 -> 289 ms).
+template <int PTT, bool WIDE>
 __device__ void panel_multi_dot(int N, int r0, int p, int j, const cd* Vf, const cd* x, cd* out) {
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if constexpr (WIDE) {
+    constexpr int NW = PTT / 64, NC = 8, LPV = 32 / NC;  // LPV lanes share a sum
+#pragma unroll 1
+    for (int i0 = wave; i0 < j; i0 += NC * NW) {
+      double s[2 * NC];
+#pragma unroll
+      for (int c = 0; c < 2 * NC; ++c) s[c] = 0.0;
+#pragma unroll 1
+      for (int r = r0 + lane; r < N; r += 64) {
+        cd a[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const int i = i0 + c * NW;
+          a[c] = Vf[r + (long)(p + (i < j ? i : i0)) * N];
+        }
+        const cd xb = x[r];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          s[2 * c] += a[c].x * xb.x + a[c].y * xb.y;
+          s[2 * c + 1] += a[c].x * xb.y - a[c].y * xb.x;
+        }
+      }
+      wave_sums<2 * NC>(s);
+      const int k = lane / LPV, i = i0 + (k >> 1) * NW;
+      if (lane % LPV == 0 && i < j) reinterpret_cast<double*>(out + i)[k & 1] = s[0];
+    }
+    __syncthreads();
+    return;
+  }
   for (int i = wave; i < j; i += PTT / 64) {
     const cd* vc = Vf + (long)(p + i) * N;
     double sr = 0.0, si = 0.0;
@@ -147,24 +199,42 @@ __device__ void panel_multi_dot(int N, int r0, int p, int j, const cd* Vf, const
   __syncthreads();
 }
 
-// acc - sum_{i < j} M[r + i ld] v[i], summed in increasing i with eight loads in flight.
-__device__ inline cd sub_row_dot(cd acc, const cd* M, long ld, int r, int j, const cd* v) {
-  int i = 0;
-  for (; i + 8 <= j; i += 8) {
-    cd m[8];
+// acc - sum_{i < j} M[r + i ld] v[i], summed in increasing i with W loads in flight (the last
+// group too: its loads stay within the j columns).
+template <int W>
+__device__ __forceinline__ cd sub_row_dot(cd acc, const cd* M, long ld, int r, int j, const cd* v) {
+#pragma unroll 1
+  for (int i = 0; i < j; i += W) {
+    cd m[W], x[W];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) m[u] = M[r + (long)(i + u) * ld];
+    for (int u = 0; u < W; ++u) {
+      const int c = i + u < j ? i + u : j - 1;
+      m[u] = M[r + (long)c * ld];
+      x[u] = v[c];
+    }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) acc = csub(acc, cmul(m[u], v[i + u]));
+    for (int u = 0; u < W; ++u) {
+      const cd y = csub(acc, cmul(m[u], x[u]));
+      acc.x = i + u < j ? y.x : acc.x;
+      acc.y = i + u < j ? y.y : acc.y;
+    }
   }
-  for (; i < j; ++i) acc = csub(acc, cmul(M[r + (long)i * ld], v[i]));
   return acc;
 }
 
+// Up to two matrices per CU; with more the narrow form runs four (N = 98, 640 matrices: wide 4.96,
+// narrow 4.48 ms; N = 162: 11.9 and 11.0).
+constexpr int GEHRD_WIDE_BATCH = 512;
+
 // PTT threads: 1024 (16 waves) in general, 256 or 512 when N - 1 fits, so that several
 // matrices share a CU (at most 128 VGPRs; the panel's T factor packed upper-triangular).
-template <int PTT>
-__global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(4))) void gehrd_panel_kernel(
+// WIDE (256 threads, up to two matrices per CU): a column is a chain of products that each wait
+// for memory, so more of it is in flight in 256 VGPRs: 16 loads per row product, two column
+// groups of the trailing product, eight columns per dot product. Same sums in the same order.
+// Reduction of one batch, N = 98: 300 matrices 3.44 -> 3.00 ms; N = 162: 60 matrices
+// 5.27 -> 4.34; N = 242: 100 matrices 11.0 -> 8.6, 200 matrices 12.8 -> 10.2.
+template <int PTT, bool WIDE>
+__global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(WIDE ? 2 : 4))) void gehrd_panel_kernel(
     int N, int p, int nb, cd* A, long lda, long sA, cd* Vf,
                                                           long sV, cd* Y, long sY, cd* Tp, long sT, cd* tau,
                                                           long sTau) {
@@ -184,6 +254,7 @@ __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(4))) void g
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   // rows below the panel; when they fit in the workgroup, the columns of the trailing
   // product are split over G groups of R threads (partial sums reduced through LDS)
+  constexpr int SRD = WIDE ? 16 : 8;
   const int R = N - p - 1;
   const int G = (R > 0 && R <= PTT) ? (PTT / R < GV_MAXG ? PTT / R : GV_MAXG) : 1;
 
@@ -192,18 +263,33 @@ __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(4))) void g
     if (t < j) vec1[t] = cconj(Vf[c + (long)(p + t) * N]);
     __syncthreads();
     // column c of A0*Q_j, rows below p (rows <= p are updated after the panel)
-    for (int r = p + 1 + t; r < N; r += PTT) bvec[r] = sub_row_dot(A[r + (long)c * lda], Y, N, r, j, vec1);
+    for (int r = p + 1 + t; r < N; r += PTT) bvec[r] = sub_row_dot<SRD>(A[r + (long)c * lda], Y, N, r, j, vec1);
     __syncthreads();
     if (j > 0) {
       // left transform by Q_j^H on rows >= p+1
-      panel_multi_dot<PTT>(N, p + 1, p, j, Vf, bvec, vec2);
+      panel_multi_dot<PTT, WIDE>(N, p + 1, p, j, Vf, bvec, vec2);
       if (t < j) {
         cd s = mk(0.0, 0.0);
-        for (int l = 0; l <= t; ++l) s = cadd(s, cmul(cconj(Tl[t * (t + 1) / 2 + l]), vec2[l]));
+#pragma unroll 1
+        for (int l0 = 0; l0 <= t; l0 += 4) {
+          cd T4[4], z4[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int l = l0 + u <= t ? l0 + u : t;
+            T4[u] = Tl[t * (t + 1) / 2 + l];
+            z4[u] = vec2[l];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const cd y = cadd(s, cmul(cconj(T4[u]), z4[u]));
+            s.x = l0 + u <= t ? y.x : s.x;
+            s.y = l0 + u <= t ? y.y : s.y;
+          }
+        }
         vec1[t] = s;
       }
       __syncthreads();
-      for (int r = p + 1 + t; r < N; r += PTT) bvec[r] = sub_row_dot(bvec[r], Vf + (long)p * N, N, r, j, vec1);
+      for (int r = p + 1 + t; r < N; r += PTT) bvec[r] = sub_row_dot<SRD>(bvec[r], Vf + (long)p * N, N, r, j, vec1);
       __syncthreads();
     }
     // final entries of column c and the reflector from rows c+1..N-1
@@ -235,7 +321,7 @@ __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(4))) void g
     if (t == 0) tau[c] = tv;
     __syncthreads();
     // z = V_j^H v  (rows >= c+1)
-    if (j > 0) panel_multi_dot<PTT>(N, c + 1, p, j, Vf, vvec, vec2);
+    if (j > 0) panel_multi_dot<PTT, WIDE>(N, c + 1, p, j, Vf, vvec, vec2);
     // y_j = tau*(A0[:, c+1:] v - Y_j z) for the rows below p (the rows above are one
     // ZGEMM after the panel). The trailing-matrix product is the memory-bound part.
     if (R > 0 && R <= PTT) {
@@ -244,18 +330,23 @@ __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(4))) void g
       double sr = 0.0, si = 0.0;
       if (g < G) {
         const int r = p + 1 + i;
-        for (int col0 = c + 1 + GV_W * g; col0 < N; col0 += GV_W * G) {
-          cd a[GV_W];
+        constexpr int GB = WIDE ? 2 : 1;  // groups of GV_W columns in flight
+#pragma unroll 1
+        for (int col0 = c + 1 + GV_W * g; col0 < N; col0 += GB * GV_W * G) {
+          cd a[GB * GV_W];
 #pragma unroll
-          for (int u = 0; u < GV_W; ++u) {
-            const bool in = col0 + u < N;
-            a[u] = in ? load_stream(A + r + (long)(col0 + u) * lda) : mk(0.0, 0.0);
+          for (int u = 0; u < GB * GV_W; ++u) {
+            const int col = col0 + u % GV_W + (u / GV_W) * GV_W * G;
+            a[u] = load_stream(A + r + (long)(col < N ? col : N - 1) * lda);
           }
 #pragma unroll
-          for (int u = 0; u < GV_W; ++u) {
-            const cd v = col0 + u < N ? vvec[col0 + u] : mk(0.0, 0.0);
-            sr += a[u].x * v.x - a[u].y * v.y;
-            si += a[u].x * v.y + a[u].y * v.x;
+          for (int u = 0; u < GB * GV_W; ++u) {
+            const int col = col0 + u % GV_W + (u / GV_W) * GV_W * G;
+            const bool in = col < N;
+            const cd v = vvec[in ? col : N - 1];
+            const double dr = a[u].x * v.x - a[u].y * v.y, di = a[u].x * v.y + a[u].y * v.x;
+            sr = in ? sr + dr : sr;
+            si = in ? si + di : si;
           }
         }
       }
@@ -265,7 +356,7 @@ __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(4))) void g
         const int r = p + 1 + t;
         cd acc = gpart[t];
         for (int q = 1; q < G; ++q) acc = cadd(acc, gpart[q * R + t]);
-        acc = sub_row_dot(acc, Y, N, r, j, vec2);
+        acc = sub_row_dot<SRD>(acc, Y, N, r, j, vec2);
         Y[r + (long)j * N] = cmul(tv, acc);
       }
     } else
@@ -316,7 +407,22 @@ __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(4))) void g
     }
     if (t < j) {
       cd s = mk(0.0, 0.0);
-      for (int l = t; l < j; ++l) s = cadd(s, cmul(Tl[l * (l + 1) / 2 + t], vec2[l]));
+#pragma unroll 1
+      for (int l0 = t; l0 < j; l0 += 4) {
+        cd T4[4], z4[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int l = l0 + u < j ? l0 + u : j - 1;
+          T4[u] = Tl[l * (l + 1) / 2 + t];
+          z4[u] = vec2[l];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const cd y = cadd(s, cmul(T4[u], z4[u]));
+          s.x = l0 + u < j ? y.x : s.x;
+          s.y = l0 + u < j ? y.y : s.y;
+        }
+      }
       Tl[j * (j + 1) / 2 + t] = cneg(cmul(tv, s));
     }
     if (t == 0) Tl[j * (j + 1) / 2 + j] = tv;
@@ -555,12 +661,12 @@ __global__ __launch_bounds__(256) void gehrd_col_c_kernel(int N, int p, int j, c
   block_dots(N, p, j, V, r, v, work + gw.z + (long)blk * HB);
 }
 
-// Spread the panel when the matrices alone would leave most CUs idle and the trailing matrix is
-// large enough to pay for three launches a column. Hessenberg stage, ms, one workgroup / spread:
-// N = 162 1 matrix 4.2 / 4.0, 64 5.3 / 5.6; N = 242 10 8.4 / 6.7, 40 9.9 / 8.9, 100 11.0 / 11.4;
+// Spread the panel when the matrices alone would leave most CUs idle and are too large for the
+// wide form of the panel in one workgroup. Hessenberg stage, ms, one workgroup / spread:
+// N = 242 (wide) 1 matrix 6.0 / 6.2, 10 6.6 / 6.7, 40 7.9 / 8.8, 60 8.1 / 9.8;
 // N = 450 10 25.0 / 16.6, 40 27.4 / 22.6, 80 30.5 / 30.6; N = 882 1 100 / 28, 10 109 / 41,
 // 60 136 / 107, 130 175 / 196.
-static bool gehrd_spread(int n, int batch) { return n >= 200 && batch <= 64; }
+static bool gehrd_spread(int n, int batch) { return n > 257 && batch <= 64; }
 
 static int n_reflectors(int n) { return n >= 3 ? n - 2 : 0; }
 
@@ -599,15 +705,18 @@ static void gehrd(hipStream_t s, int n, cd* A, long lda, long sA, cd* Vf, cd* Ta
         gehrd_col_c_kernel<<<dim3(ngemv + gw.nblk, batch), 256, 0, s>>>(n, p, j, A, lda, sA, Vf, sV, taub.as<cd>(), n,
                                                                         work, gw, nrow, ngemv);
       }
-    } else if (n - 1 <= 256)
-      gehrd_panel_kernel<256><<<batch, 256, 2 * sizeof(cd) * n, s>>>(n, p, nb, A, lda, sA, Vf, sV, Y, sY, Tp, sT,
-                                                                     taub.as<cd>(), n);
+    } else if (n - 1 <= 256 && batch <= GEHRD_WIDE_BATCH)
+      gehrd_panel_kernel<256, true><<<batch, 256, 2 * sizeof(cd) * n, s>>>(n, p, nb, A, lda, sA, Vf, sV, Y, sY, Tp,
+                                                                           sT, taub.as<cd>(), n);
+    else if (n - 1 <= 256)
+      gehrd_panel_kernel<256, false><<<batch, 256, 2 * sizeof(cd) * n, s>>>(n, p, nb, A, lda, sA, Vf, sV, Y, sY, Tp,
+                                                                            sT, taub.as<cd>(), n);
     else if (n - 1 <= 512)
-      gehrd_panel_kernel<512><<<batch, 512, 2 * sizeof(cd) * n, s>>>(n, p, nb, A, lda, sA, Vf, sV, Y, sY, Tp, sT,
-                                                                     taub.as<cd>(), n);
+      gehrd_panel_kernel<512, false><<<batch, 512, 2 * sizeof(cd) * n, s>>>(n, p, nb, A, lda, sA, Vf, sV, Y, sY, Tp,
+                                                                            sT, taub.as<cd>(), n);
     else
-      gehrd_panel_kernel<PT><<<batch, PT, 2 * sizeof(cd) * n, s>>>(n, p, nb, A, lda, sA, Vf, sV, Y, sY, Tp, sT,
-                                                                   taub.as<cd>(), n);
+      gehrd_panel_kernel<PT, false><<<batch, PT, 2 * sizeof(cd) * n, s>>>(n, p, nb, A, lda, sA, Vf, sV, Y, sY, Tp,
+                                                                          sT, taub.as<cd>(), n);
     launch_check("gehrd_panel");
     // rows 0..p: Y = A0 V T, then the panel columns' A0 Q = A0 - Y V^H
     zgemm_strided(s, OP_N, OP_N, p + 1, nb, n - p - 1, one, A + (long)(p + 1) * lda, lda, sA,
