@@ -299,6 +299,38 @@ def test_zgeev_team_sizes(ctx, n):
             assert np.array_equal(w[b], ref[0]) and np.array_equal(V[b], ref[1]), (batch, b)
 
 
+@pytest.mark.parametrize("batches", [(1, 9, 40, 64), (129, 70, 128)])
+@pytest.mark.parametrize("n", [338, 450])
+def test_zgeev_team_hand_over(ctx, n, batches):
+    """Windows of many strips handed between the workgroups of a team, at sizes that are no
+    multiple of the strips' 16: three different matrices in turn, each with the same bits in teams
+    of 16, 16, 6 and 4 workgroups, and in teams of 3 and 2 as in none (129 matrices). Up to 64
+    matrices and more of them take different forms of the Hessenberg panel, hence two groups."""
+    import torch
+    rng = np.random.default_rng(7000 + n)
+    A = to_dev_colmajor(crand(rng, 3, n, n))
+    ref = None
+    for batch in batches:
+        pick = torch.arange(batch, device="cuda") % 3
+        dA = A[pick].contiguous()
+        w = torch.zeros((batch, n), dtype=torch.complex128, device="cuda")
+        VR = torch.zeros_like(dA)
+        info = torch.zeros(batch, dtype=torch.int32, device="cuda")
+        ctx.check(ctx.lib.vrc_zgeev(ctx.h, n, ptr(dA), n, n * n, ptr(w), n, ptr(VR), n, n * n, ptr(info), batch),
+                  "zgeev")
+        ctx.sync()
+        assert int(info.abs().max()) == 0
+        first = min(batch, 3)
+        if ref is None or len(ref[0]) < first:
+            assert ref is None or (torch.equal(w[:1], ref[0]) and torch.equal(VR[:1], ref[1]))
+            ref = (w[:first].clone(), VR[:first].clone())
+        assert torch.equal(w, ref[0][pick]) and torch.equal(VR, ref[1][pick]), batch
+    B = from_dev_colmajor(A)
+    V, W = from_dev_colmajor(ref[1]), ref[0].cpu().numpy()
+    for b in range(len(V)):
+        assert np.abs(B[b] @ V[b] - V[b] * W[b][None, :]).max() < 1e-12 * n * np.linalg.norm(B[b], 2)
+
+
 @pytest.mark.parametrize("n", [3, 17, 66, 67, 130, 162])
 def test_zgeev_wide_hessenberg(ctx, n):
     """Up to 512 matrices take the Hessenberg panel with more loads in flight, more of them the
