@@ -120,6 +120,35 @@ def test_fourier_cell_order(ctx, crossing):
             api.assemble_toeplitz(ctx, 5, 7, layers[:i] + [l] + layers[i + 1:])
 
 
+@pytest.mark.parametrize("crossing", [False, True])
+@pytest.mark.parametrize("ncx,ncy,count", [(1, 1, 3), (63, 65, 1), (65, 63, 2), (64, 64, 1), (32, 32, 12), (32, 32, 13)])
+def test_fourier_cell_order_sides(ctx, crossing, ncx, ncy, count):
+    """Both writers of the painter's order, host and device, at the counts where one takes over
+    (4096 cells per layer, 12288 in all), one layer of each batch smaller than the others, against
+    the oracle at the 1e-12 of the other assembly checks; bad values are refused by both."""
+    rng = np.random.default_rng(100 * ncx + count)
+    layers = []
+    for i in range(count):
+        cx, cy = (ncx, ncy) if i != count - 1 or count == 1 else (max(1, ncx - 3), max(1, ncy - 5))
+        x = np.concatenate([[0.0], np.sort(rng.uniform(0.05, 0.75, cx - 1)), [0.8]])
+        y = np.concatenate([[0.0], np.sort(rng.uniform(0.05, 0.75, cy - 1)), [0.8]])
+        if crossing and cx > 4:
+            x[2:5] = x[[4, 2, 3]]
+        layers.append((x, y, 1 + 11.25 * rng.random((cy, cx)) + 0.3j * rng.random((cy, cx))))
+    fe = api.assemble_toeplitz(ctx, 3, 5, layers).cpu().numpy()
+    for i in {0, count - 1}:
+        x, y, eps = layers[i]
+        for k, opt in enumerate([O.DISCONTINUOUS_X, O.DISCONTINUOUS_Y, O.CONTINUOUS_XY]):
+            ref = O.fourier2d(x, y, eps, 3, 5, opt)
+            assert rel(fe[k, i].T, ref) < 1e-12, (i, k, rel(fe[k, i].T, ref))
+    for bad in (np.nan, np.inf * 1j, 0.0):
+        x, y, eps = layers[-1]
+        eps = eps.copy()
+        eps[-1, -1] = bad
+        with pytest.raises(VrcError):
+            api.assemble_toeplitz(ctx, 3, 5, layers[:-1] + [(x, y, eps)])
+
+
 @pytest.mark.parametrize("which", ["metasurface", "var12"])
 def test_pq_matches_oracle(ctx, which):
     g = G.metasurface(2) if which == "metasurface" else G.var12(2, 2)

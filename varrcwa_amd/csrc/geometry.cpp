@@ -212,6 +212,12 @@ __global__ __launch_bounds__(256) void order_cells_kernel(const cd* raw, const l
   if (j0 + a < MX && s0 + b < MY) val[((long)l * MY + s0 + b) * MX + j0 + a] = tile[a][b];
 }
 
+// Does the host write the cells in painter's order? Up to these counts (padded) the strided write
+// costs less than order_cells_kernel (us, host / kernel, 3 x 3 harmonics): 1 layer of 1 cell 42 / 62, 64
+// of 8 x 8 124 / 149, 2 of 20 x 20 69 / 80, 3 of 50 x 50 130 / 136, 8 of 32 x 32 100 / 105;
+// 16 of 32 x 32 124 / 121, 1 of 64 x 64 90 / 84, 2 of 64 x 64 104 / 88, 2 of 128 x 128 239 / 123.
+static bool host_orders_cells(size_t per_layer, int layers) { return per_layer < 4096 && per_layer * layers <= 12288; }
+
 FourierStage fourier_prepare(vrc_ctx& c, int nx, int ny, const std::vector<const HostLayer*>& layers) {
   std::vector<LayerView> v;
   v.reserve(layers.size());
@@ -258,14 +264,17 @@ FourierStage fourier_prepare(vrc_ctx& c, int nx, int ny, const std::vector<Layer
     fft_max = std::max(fft_max, std::max(fx[l] ? 1 << fx[l] : 0, fy[l] ? 1 << fy[l] : 0));
   }
   // One upload: the geometry, then the layers' values as they were given, checked and written
-  // straight into the pinned block; the device puts the cells into painter's order. 64 layers
-  // of 256 x 256 cells, assembled: 3.3 ms, of which 1.3 are the copy to the device; through six
-  // host arrays and a strided transpose it took 56.
+  // straight into the pinned block; the device (for few cells the host, host_orders_cells) puts
+  // the cells into painter's order. 64 layers of 256 x 256 cells, assembled: 3.3 ms, of which 1.3
+  // are the copy to the device; through six host arrays and a strided transpose it took 56.
   const size_t od = sizeof(int) * 4 * L, ox = od + sizeof(double) * 2 * L,
                oy = ox + sizeof(double) * 2 * (size_t)L * (MX + 1), oo = oy + sizeof(double) * (size_t)L * (MY + 1),
                os = oo + sizeof(long) * L, geo_bytes = (os + sizeof(int) * (size_t)L * MX + 15) & ~(size_t)15;
-  fs.geo = c.ws.get(geo_bytes + sizeof(cd) * (size_t)cells);
-  c.pinned.upload_with(s, fs.geo.ptr, geo_bytes + sizeof(cd) * (size_t)cells, [&](char* h) {
+  const size_t nval = (size_t)MY * MX;
+  const bool host_order = host_orders_cells(nval, L);
+  const size_t val_bytes = sizeof(cd) * (host_order ? nval * L : (size_t)cells);
+  fs.geo = c.ws.get(geo_bytes + val_bytes);
+  c.pinned.upload_with(s, fs.geo.ptr, geo_bytes + val_bytes, [&](char* h) {
     std::memset(h, 0, geo_bytes);
     int* hi = (int*)h;
     double *hd = (double*)(h + od), *hx = (double*)(h + ox), *hy = (double*)(h + oy);
@@ -286,7 +295,20 @@ FourierStage fourier_prepare(vrc_ctx& c, int nx, int ny, const std::vector<Layer
       std::copy(p.src.begin(), p.src.end(), hs + (size_t)l * MX);
     }
     double* hv = (double*)(h + geo_bytes);
-    for (int l = 0; l < L; ++l) scan_permittivity<true>(layers[l], hv + 2 * off[l]);
+    if (!host_order) {
+      for (int l = 0; l < L; ++l) scan_permittivity<true>(layers[l], hv + 2 * off[l]);
+      return;
+    }
+    cd* v = (cd*)hv;
+    std::fill(v, v + nval * L, mk(1.0, 0.0));
+    for (int l = 0; l < L; ++l, v += nval) {
+      const PreparedLayer& p = pl[l];
+      scan_permittivity<false>(layers[l], nullptr);
+      for (int j = 0; j < p.ncx; ++j) {
+        const double* e = layers[l].eps + 2 * (size_t)p.src[j] * p.ncy;  // 8-byte aligned only
+        for (int i = 0; i < p.ncy; ++i) v[(size_t)i * MX + j] = mk(e[2 * i], e[2 * i + 1]);
+      }
+    }
   });
   char* d = (char*)fs.geo.ptr;
   FourierDev& g = fs.g;
@@ -309,14 +331,17 @@ FourierStage fourier_prepare(vrc_ctx& c, int nx, int ny, const std::vector<Layer
                ntx = (size_t)MY * nx * nx, nty = (size_t)MX * ny * ny, nF2 = (size_t)M1 * M2,
                nG11 = (size_t)nx * nx * M2, nG22 = (size_t)ny * ny * M1;
   const size_t per = 2 * nFX + nFY1 + nFYi + nFX1 + ntx + nty + nF2 + nG11 + nG22;
-  const size_t nval = (size_t)MY * MX;
-  fs.wk = c.ws.get(sizeof(cd) * (per + nval) * L);
-  cd* val = fs.wk.as<cd>();
-  cd* w = val + nval * L;
-  g.val = val;
-  order_cells_kernel<<<dim3(cdiv_up(MX, 16), cdiv_up(MY, 16), L), 256, 0, s>>>(
-      (const cd*)(d + geo_bytes), (const long*)(d + oo), (const int*)(d + os), g.ncx, g.ncy, MX, MY, val);
-  launch_check("order_cells");
+  fs.wk = c.ws.get(sizeof(cd) * (per + (host_order ? 0 : nval)) * L);
+  cd* w = fs.wk.as<cd>();
+  if (host_order) {
+    g.val = (const cd*)(d + geo_bytes);
+  } else {
+    order_cells_kernel<<<dim3(cdiv_up(MX, 16), cdiv_up(MY, 16), L), 256, 0, s>>>(
+        (const cd*)(d + geo_bytes), (const long*)(d + oo), (const int*)(d + os), g.ncx, g.ncy, MX, MY, w);
+    launch_check("order_cells");
+    g.val = w;
+    w += nval * L;
+  }
   g.FX = w;
   g.FXi = g.FX + nFX * L;
   g.FY1 = g.FXi + nFX * L;
