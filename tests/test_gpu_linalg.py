@@ -156,6 +156,28 @@ def test_getrf_panel_edges(ctx, n, batch, kind):
         assert r <= 12 * n * n * eps * bound.max()
 
 
+@pytest.mark.parametrize("n", [1, 4, 31, 32, 33, 47, 48, 49, 80, 96, 97, 112, 113])
+def test_getrs_last_block(ctx, n):
+    """Solves whose last 64-row diagonal block holds one to four runs of 16 rows: the backward
+    error of two triangular solves through inverted blocks, with the bound of the test above."""
+    import torch
+    rng = np.random.default_rng(900 + n)
+    A, x = crand(rng, 2, n, n), crand(rng, 2, n, 5)
+    dA = to_dev_colmajor(A)
+    ipiv = torch.zeros(2, n, dtype=torch.int32, device="cuda")
+    info = torch.zeros(2, dtype=torch.int32, device="cuda")
+    ctx.check(ctx.lib.vrc_zgetrf(ctx.h, n, ptr(dA), n, n * n, ptr(ipiv), n, ptr(info), 2), "getrf")
+    dB, dX = to_dev_colmajor(A @ x), to_dev_colmajor(x * 0)
+    ctx.check(ctx.lib.vrc_zgetrs(ctx.h, n, 5, ptr(dA), n, n * n, ptr(ipiv), n, ptr(dB), n, 5 * n, ptr(dX), n, 5 * n, 2),
+              "getrs")
+    LU, X = from_dev_colmajor(dA), from_dev_colmajor(dX)
+    eps = np.finfo(float).eps
+    for b in range(2):
+        r = np.abs(A[b] @ X[b] - A[b] @ x[b]).max()
+        bound = np.abs(np.tril(LU[b], -1) + np.eye(n)) @ np.abs(np.triu(LU[b])) @ np.abs(X[b])
+        assert r <= 12 * n * n * eps * bound.max()
+
+
 def test_getrf_zero_column_info(ctx):
     """A zero column inside a panel: info names it (1-based), as LAPACK's."""
     import torch

@@ -604,8 +604,8 @@ __global__ void gather_rows_kernel(int n, int nrhs, const int* perm, long sPerm,
 }
 
 // Inverse of every TRS_NB x TRS_NB diagonal block of a triangular factor (UPPER=0: unit
-// lower, UPPER=1: non-unit upper) into Dinv[b][blk] (TRS_NB x TRS_NB, zero padded past
-// the block size). One workgroup per block, 16 columns per wave: lane (g, c) holds the rows
+// lower, UPPER=1: non-unit upper) into Dinv[b][blk] (ld TRS_NB; what is past the block size is
+// not written, or not defined). One workgroup per block, 16 columns per wave: lane (g, c) holds the rows
 // j = 4 q + g of column c in registers, so that the substitution of a column stays within its
 // wave: a lane exchange per step where X in LDS took two barriers and a read and write of X
 // (lower 50 -> 25 us, upper 60 -> 33 us per launch; now bound by the 64 dependent steps, for
@@ -628,12 +628,15 @@ __global__ __launch_bounds__(256) void trtri_blocks_kernel(int n, const cd* T, l
   __shared__ double ratio[TRS_NB], den[TRS_NB];  // cdiv by the diagonal (Smith): ratio, divisor
   __shared__ int ybig[TRS_NB];
   const int t = threadIdx.x;
-#pragma unroll 8
-  for (int r = 0; r < TRS_NB * TRS_NB / 256; ++r) {
-    const int e = t + 256 * r, i = e % TRS_NB, j = e / TRS_NB;
-    const bool in = i < bs && j < bs;
-    const cd v = T[(k0 + (i < bs ? i : 0)) + (long)(k0 + (j < bs ? j : 0)) * ldt];
-    Ls[LO + i][j] = mk(in ? v.x : 0.0, in ? v.y : 0.0);
+#pragma unroll 1
+  for (int r0 = 0; 4 * r0 < bs; r0 += 8) {  // columns 4 r0 .. 4 r0 + 31
+#pragma unroll
+    for (int r = r0; r < r0 + 8; ++r) {
+      const int e = t + 256 * r, i = e % TRS_NB, j = e / TRS_NB;
+      const bool in = i < bs && j < bs;
+      const cd v = T[(k0 + (i < bs ? i : 0)) + (long)(k0 + (j < bs ? j : 0)) * ldt];
+      Ls[LO + i][j] = mk(in ? v.x : 0.0, in ? v.y : 0.0);
+    }
   }
   __syncthreads();
   if (UPPER) {
@@ -650,11 +653,15 @@ __global__ __launch_bounds__(256) void trtri_blocks_kernel(int n, const cd* T, l
   }
   const int lane = t & 63, g = lane >> 4;
   const int col = (t >> 6) * 16 + (lane & 15);
-  // x[q]: row group q from the end the substitution starts at
+  // A block of up to 48 rows (a small matrix, or the last block) leaves waves without columns and
+  // runs of four row groups without rows: neither is run (solves of n = 4: 39 us with them).
+  if ((t >> 6) * 16 >= bs) return;
+  const int live = (bs + 15) / 16, skip = UPPER ? 4 * (4 - live) : 0;
+  // x[q]: row group q from the end the substitution starts at (UPPER: of the live rows)
   cd x[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
-    const int j = 4 * (UPPER ? NQ - 1 - q : q) + g;
+    const int j = 4 * (UPPER ? NQ - 1 - q - skip : q) + g;
     x[q] = mk(j == col && col < bs ? 1.0 : 0.0, 0.0);
   }
   // Four row groups of the substitution from group FROM on; x[0 .. LEFT) can still change. The
@@ -662,6 +669,7 @@ __global__ __launch_bounds__(256) void trtri_blocks_kernel(int n, const cd* T, l
   // size meet zeros of Ls.
   auto run = [&](auto from) {
     constexpr int FROM = decltype(from)::value, LEFT = NQ - FROM;
+    if (UPPER ? FROM < skip : FROM >= 4 * live) return;
 #pragma unroll 1
     for (int iq = FROM; iq < FROM + 4; ++iq) {
       const int grp = UPPER ? NQ - 1 - iq : iq;
