@@ -353,6 +353,53 @@ def test_zgeev_team_hand_over(ctx, n, batches):
         assert np.abs(B[b] @ V[b] - V[b] * W[b][None, :]).max() < 1e-12 * n * np.linalg.norm(B[b], 2)
 
 
+def test_zgeev_team_streams(ctx):
+    """Contexts on several streams divide the CUs between their teams (16 workgroups per matrix with
+    one, 8, 5 and 4 with two to four): the bits stay the same, alone and with all contexts at
+    work at once."""
+    import threading
+
+    import torch
+    from varrcwa_amd._lib import Context
+    rng = np.random.default_rng(4900)
+    n, batch = 242, 8
+    A = to_dev_colmajor(crand(rng, batch, n, n))
+    out = {}
+
+    def solve(key, c, stream):
+        with torch.cuda.stream(stream):
+            dA = A.clone()
+            w = torch.zeros((batch, n), dtype=torch.complex128, device="cuda")
+            VR = torch.zeros_like(dA)
+            info = torch.zeros(batch, dtype=torch.int32, device="cuda")
+            rc = c.lib.vrc_zgeev(c.h, n, ptr(dA), n, n * n, ptr(w), n, ptr(VR), n, n * n, ptr(info), batch)
+            c.sync()
+            out[key] = (rc, int(info.abs().max()), w.cpu().numpy(), VR.cpu().numpy())
+
+    torch.cuda.synchronize()
+    solve("one", ctx, torch.cuda.current_stream())
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    more = []
+    try:
+        for s in streams:
+            more.append(Context(0, s.cuda_stream))
+            solve(len(more), ctx, torch.cuda.current_stream())
+        threads = [threading.Thread(target=solve, args=(("thread", k), c, s)) for k, (c, s) in
+                   enumerate(zip(more, streams))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        for c in more:
+            c.close()
+    solve("after", ctx, torch.cuda.current_stream())
+    assert len(out) == 8
+    for key, (rc, bad, w, V) in out.items():
+        assert rc == 0 and bad == 0, key
+        assert np.array_equal(w, out["one"][2]) and np.array_equal(V, out["one"][3]), key
+
+
 @pytest.mark.parametrize("n", [3, 17, 66, 67, 130, 162])
 def test_zgeev_wide_hessenberg(ctx, n):
     """Up to 512 matrices take the Hessenberg panel with more loads in flight, more of them the

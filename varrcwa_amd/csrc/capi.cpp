@@ -60,6 +60,8 @@ int vrc_ctx_create(int device, void* stream, vrc_ctx** out) {
     delete c;
     return rc;
   }
+  c->bound = c->stream;
+  ctx_list(c);
   *out = c;
   return 0;
 }

@@ -2387,11 +2387,17 @@ static int aed_window_for(int v, int n) {
   return n <= 112 ? 8 : (n <= 144 ? 12 : (n <= 360 ? 16 : 24));
 }
 int zgeev_get_aed() { return g_aed_window; }
-// Workgroups per matrix of the 64-wide kernel: what 32 CUs per XCD hold, at most 16.
-static int team_size(int n, int batch) {
+// Workgroups per matrix of the 64-wide kernel: what 32 CUs per XCD hold, at most 16. A member keeps
+// its CU for the whole iteration, also while its master chases alone, so contexts on several streams
+// of the process share the CUs out (up to four ways: HIP's hardware queues per process, by
+// default); one launch holding all of them would make the others wait. Four contexts, ms a round
+// with all CUs for each / a quarter / before there were teams: a stack of 10 layers each at N = 882
+// 689 / 345 / 626, four at N = 450 300 / 181 / 227; a single matrix each at N = 882 179 / 193 / 483.
+// The bits do not depend on the team.
+static int team_size(int n, int batch, int streams) {
   if (n < 200 || n > 65535) return 1;
   const int per_xcd = (batch + 7) / 8;
-  const int g = 32 / per_xcd;
+  const int g = 32 / std::min(streams, 4) / per_xcd;
   return g < 16 ? g : 16;
 }
 int zgeev_get_bulges() { return g_bulges; }
@@ -2434,7 +2440,7 @@ void zgeev_factors(hipStream_t s, int n, cd* A, long lda, long sA, cd* w, long s
     } else if (qv == 1) {
       hqr_lds_kernel<<<batch, QT, 0, s>>>(n, A, lda, sA, Z, n, nn, w, sw, info, stp, aed, g_bulges,
                                           g_max_sweeps);
-    } else if (const int team = team_size(n, batch); team > 1) {
+    } else if (const int team = team_size(n, batch, gpu_streams(c ? c->device : 0)); team > 1) {
       const int batch8 = (batch + 7) & ~7;
       DevBuf tc = ws.get(sizeof(TeamCtl) * (size_t)batch), tu = ws.get(sizeof(cd) * (size_t)QW * QW * batch);
       fill_int(s, tc.as<int>(), 0, (int)(sizeof(TeamCtl) / sizeof(int)) * batch);

@@ -8,6 +8,8 @@
 
 #include "vrc_internal.hpp"
 
+struct vrc_ctx;
+
 namespace vrc {
 // Pinned host staging for host -> device copies: a block is reused once the copy that
 // read it has completed (an event recorded after the copy), so uploads need no host
@@ -27,6 +29,11 @@ struct PinnedPool {
   // The same with the pinned block written by fill(block).
   void upload_with(hipStream_t s, void* dst, size_t bytes, const std::function<void(char*)>& fill);
 };
+// The live contexts, and the number of different streams that those of a device are bound to (at
+// least 1): work of contexts on different streams may run at the same time.
+void ctx_list(vrc_ctx* c);
+void ctx_unlist(vrc_ctx* c);
+int gpu_streams(int device);
 }  // namespace vrc
 
 // Reference counted: samplers and integrators hold a reference, so the pool and the
@@ -38,6 +45,8 @@ struct vrc_ctx {
   vrc::PinnedPool pinned;
   std::string last_error;
   std::atomic<int> refs{1};
+  hipStream_t bound = nullptr;  // the stream it was created for (stream changes while a recording is made)
+  bool listed = false;          // among the live contexts that gpu_streams counts
   // stage timers (HIP events on the context stream), see vrc::StageScope
   bool timing = false;
   struct Rec {
@@ -55,6 +64,7 @@ struct vrc_ctx {
   int host_code = 0;
   std::string host_msg;
   ~vrc_ctx() {
+    if (listed) vrc::ctx_unlist(this);
     if (health) (void)hipFree(health);
     for (auto& r : recs) {
       (void)hipEventDestroy(r.a);

@@ -126,6 +126,7 @@ void Workspace::trim() {
 // ---------------------------------------------------------------- stage timers
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 
 #include "vrc_context.hpp"
 
@@ -166,6 +167,35 @@ void PinnedPool::upload_with(hipStream_t s, void* dst, size_t bytes, const std::
   fill((char*)blk->p);
   VRC_HIP(hipMemcpyAsync(dst, blk->p, bytes, hipMemcpyHostToDevice, s));
   VRC_HIP(hipEventRecord(blk->ev, s));
+}
+
+namespace {
+std::mutex g_list_mutex;
+// never destroyed: contexts may go after the library's own statics
+std::vector<vrc_ctx*>& live() {
+  static auto* list = new std::vector<vrc_ctx*>;
+  return *list;
+}
+}  // namespace
+
+void ctx_list(vrc_ctx* c) {
+  std::lock_guard<std::mutex> lock(g_list_mutex);
+  live().push_back(c);
+  c->listed = true;
+}
+
+void ctx_unlist(vrc_ctx* c) {
+  std::lock_guard<std::mutex> lock(g_list_mutex);
+  live().erase(std::remove(live().begin(), live().end(), c), live().end());
+  c->listed = false;
+}
+
+int gpu_streams(int device) {
+  std::lock_guard<std::mutex> lock(g_list_mutex);
+  std::vector<hipStream_t> seen;
+  for (const vrc_ctx* c : live())
+    if (c->device == device && std::find(seen.begin(), seen.end(), c->bound) == seen.end()) seen.push_back(c->bound);
+  return std::max<int>(1, (int)seen.size());
 }
 
 vrc_ctx*& tl_ctx() {
