@@ -67,7 +67,9 @@ int vrc_timing_enable(vrc_ctx* ctx, int on);
  * RCWAIntegrator::compute solved per eigensolve launch (1: one slice at a time, as the
  * reference's GPU integrator); "stack.cascade_group" (default 512, fewer when their slab
  * S-matrices would exceed 96 GiB): instances of vrc_batch_stack_rcwa whose star products
- * and projections run in one batch;
+ * and projections run in one batch; "cascade.matrices" (default 0 = as many as 8 GiB hold, at
+ * least 16): N x N matrices that a tree of star products or a batch of varRCWA projections may
+ * hold, more work goes in several trees and batches;
  * "zgeev.qr_variant" (default -1: automatic, variant 4 for N <= 256 in launches of at least
  * 384 matrices and for N <= 512 in launches of at least 768, variant 2 for N <= 1024 in
  * launches of at least 384, else 0): the QR (Schur) kernel, 0: 64-wide window on 512 threads,

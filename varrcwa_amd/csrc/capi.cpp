@@ -131,6 +131,11 @@ int vrc_tune_set(const char* key, long long value) {
     rcwa_set_group((int)value);
     return 0;
   }
+  if (std::strcmp(key, "cascade.matrices") == 0) {
+    if (value < 0 || value > (1 << 30)) return -1;
+    cascade_set_matrices((int)value);
+    return 0;
+  }
   if (std::strcmp(key, "stack.cascade_group") == 0) {
     stack_set_cascade_group((int)value);
     return 0;

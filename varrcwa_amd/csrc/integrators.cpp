@@ -441,9 +441,13 @@ SMat smat_at(cd* p, long blk) {
   return S;
 }
 
-// Matrices of N x N that a tree of star products may hold (pairs in flight, or all its levels).
-size_t cascade_mats(int N) {  // (8192 products at most in one batch: the grid's y and z limits)
-  return std::max<size_t>(16, ((size_t)8 << 30) / (sizeof(cd) * (size_t)N * N)); }
+// Matrices of N x N that a tree of star products may hold (pairs in flight, or all its levels): what
+// 8 GiB hold unless "cascade.matrices" says otherwise; at most 8192 products in one batch.
+int g_cascade_mats = 0;
+size_t cascade_mats(int N) {
+  if (g_cascade_mats > 0) return (size_t)g_cascade_mats;
+  return std::max<size_t>(16, ((size_t)8 << 30) / (sizeof(cd) * (size_t)N * N));
+}
 
 // Star product of n S-matrices in each of B rows (items[b * n + j], j in cascade order) into out
 // (row stride N^2). The star product is associative: pairs of neighbours are combined level by
@@ -516,6 +520,8 @@ void cascade_onto(vrc_ctx& c, int N, int B, int n, std::vector<SPtr> items, SMat
 }
 }  // namespace
 
+void cascade_set_matrices(int n) { g_cascade_mats = n < 0 ? 0 : n; }
+
 // RCWAIntegrator::compute (src/core/RCWAIntegrator.cpp:20-87) over explicit slices
 // (midpoint z, width). The slices are independent until the cascade, so their samples,
 // eigensolves and slab S-matrices run in groups of up to g_rcwa_group per launch (one
@@ -568,7 +574,7 @@ void Integrator::rcwa(const std::vector<std::pair<double, double>>& slices, bool
     DevBuf ds = upload(c, sv.data(), sizeof(double) * g);
     layer_smatrix(c, N, g, ds.as<double>(), Wb.as<cd>() + e * NN, Vb.as<cd>() + e * NN, gb.as<cd>() + e * N,
                   W1_.as<cd>(), V1_.as<cd>(), 0, tu.as<cd>(), ru.as<cd>());
-    const int tree = (int)std::min<size_t>(g, cascade_mats(N) / 4);
+    const int tree = (int)std::min<size_t>(g, std::max<size_t>(1, cascade_mats(N) / 4));
     for (int j0 = 0; j0 < g; j0 += tree) {
       std::vector<SPtr> items;
       for (int j = j0; j < std::min(g, j0 + tree); ++j) {
@@ -1005,10 +1011,10 @@ static void cascade_group(vrc_ctx& c, int N, int L, int GB, int I0, bool homog, 
   }
   // identity * slab 0 = slab 0: the cascade starts from the first slab's S-matrix
   if (!tree) {
-  zgeam(st, N, N, ONE, tu, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Tdd, N, NN, B);
-  zgeam(st, N, N, ONE, tu, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Tuu, N, NN, B);
-  zgeam(st, N, N, ONE, ru, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Rud, N, NN, B);
-  zgeam(st, N, N, ONE, ru, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Rdu, N, NN, B);
+    zgeam(st, N, N, ONE, tu, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Tdd, N, NN, B);
+    zgeam(st, N, N, ONE, tu, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Tuu, N, NN, B);
+    zgeam(st, N, N, ONE, ru, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Rud, N, NN, B);
+    zgeam(st, N, N, ONE, ru, N, (long)L * NN, ZERO, nullptr, 0, 0, S.Rdu, N, NN, B);
   }
   // tape layout: 4 blocks [Tdd|Tuu|Rud|Rdu] per instance
   auto keep_S = [&](cd* dst, long per_inst) {

@@ -154,6 +154,7 @@ struct RefSys {
 void gather_mats(hipStream_t s, long nn, const cd* src, long ss, const int* d_idx, cd* dst, long sd, int batch);
 // dst[b] (nbytes each, contiguous, a multiple of 8) = *src[b].
 void gather_ptrs(vrc_ctx& c, const std::vector<const void*>& src, size_t nbytes, void* dst);
+void cascade_set_matrices(int n);     // matrices a tree of star products may hold (0: 8 GiB)
 void stack_set_cascade_group(int n);  // instances per batched cascade of batch_stack_rcwa
 void rcwa_set_group(int g);           // slices per eigensolve launch of RCWAIntegrator (1: one at a time)
 // Slab S-matrix (src/rcwa/RCWAScatterMatrix.cpp:26-85); d_s[b] = dz_b / k0_b.
