@@ -321,13 +321,13 @@ def test_zgeev_team_sizes(ctx, n):
             assert np.array_equal(w[b], ref[0]) and np.array_equal(V[b], ref[1]), (batch, b)
 
 
-@pytest.mark.parametrize("batches", [(1, 9, 40, 64), (129, 70, 128)])
-@pytest.mark.parametrize("n", [338, 450])
+@pytest.mark.parametrize("n,batches", [(338, (1, 9, 40)), (338, (129, 64, 70, 128)), (450, (1, 9, 40, 64)),
+                                       (450, (129, 70, 128))])
 def test_zgeev_team_hand_over(ctx, n, batches):
     """Windows of many strips handed between the workgroups of a team, at sizes that are no
     multiple of the strips' 16: three different matrices in turn, each with the same bits in teams
-    of 16, 16, 6 and 4 workgroups, and in teams of 3 and 2 as in none (129 matrices). Up to 64
-    matrices and more of them take different forms of the Hessenberg panel, hence two groups."""
+    of 16, 16, 6 and 4 workgroups, and in teams of 4, 3 and 2 as in none (129 matrices). Few matrices
+    and many take different forms of the Hessenberg panel, hence two groups."""
     import torch
     rng = np.random.default_rng(7000 + n)
     A = to_dev_colmajor(crand(rng, 3, n, n))
@@ -427,6 +427,25 @@ def test_zgeev_spread_hessenberg(ctx, n):
     A[2, n // 2:, : n // 2] = 0.0
     _eig_check_values(ctx, A)
     _eig_check(ctx, A[:1])
+
+
+@pytest.mark.parametrize("n,batch", [(258, 23), (322, 46), (373, 64), (500, 64)])
+def test_zgeev_spread_line(ctx, n, batch):
+    """The last count of matrices whose Hessenberg panel is spread over workgroups, and one more, in
+    one workgroup each: sums in another order, so the eigenvalues agree to the rounding of the
+    reduction (backward error n eps |A|, condition numbers of a random matrix below 1e4) and the
+    residuals stay as small; with the spread one some matrices differ in the last bits."""
+    rng = np.random.default_rng(8000 + n)
+    A = crand(rng, 1, n, n)
+    (w0, V0), (w1, V1) = _eig_values(ctx, A, batch), _eig_values(ctx, A, batch + 1)
+    size = np.linalg.norm(A[0], 2)
+    for w, V in ((w0, V0), (w1, V1)):
+        assert np.array_equal(w[0], w[-1]) and np.array_equal(V[0], V[-1])
+        assert np.abs(A[0] @ V[0] - V[0] * w[0][None, :]).max() < 1e-12 * n * size
+    d = np.abs(w0[0][:, None] - w1[0][None, :])
+    assert len(set(d.argmin(axis=1))) == n
+    assert d.min(axis=1).max() < 1e4 * n * np.finfo(float).eps * size
+    assert not np.array_equal(w0[0], w1[0])  # the two forms, not one of them twice
 
 
 def _eig_values(ctx, A, batch):

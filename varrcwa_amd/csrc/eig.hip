@@ -663,10 +663,11 @@ __global__ __launch_bounds__(256) void gehrd_col_c_kernel(int N, int p, int j, c
 
 // Spread the panel when the matrices alone would leave most CUs idle and are too large for the
 // wide form of the panel in one workgroup. Hessenberg stage, ms, one workgroup / spread:
-// N = 242 (wide) 1 matrix 6.0 / 6.2, 10 6.6 / 6.7, 40 7.9 / 8.8, 60 8.1 / 9.8;
-// N = 450 10 25.0 / 16.6, 40 27.4 / 22.6, 80 30.5 / 30.6; N = 882 1 100 / 28, 10 109 / 41,
-// 60 136 / 107, 130 175 / 196.
-static bool gehrd_spread(int n, int batch) { return n > 257 && batch <= 64; }
+// N = 242 (wide) 1 matrix 6.0 / 6.2, 10 6.6 / 6.7, 40 7.9 / 8.8, 60 8.1 / 9.8; N = 258 8 7.7 / 7.1,
+// 24 8.2 / 8.2, 64 9.1 / 10.4; N = 338 24 13.0 / 11.4, 40 13.8 / 13.0, 56 14.4 / 14.5, 64 14.5 / 15.1;
+// N = 450 8 20.5 / 13.8, 64 26.4 / 24.6, 80 27.6 / 28.1; N = 882 8 103 / 35, 64 129 / 104, 96 147 / 144,
+// 112 156 / 164. The line follows the crossings up to N = 373 and stays at 64 matrices from there.
+static bool gehrd_spread(int n, int batch) { return n > 257 && batch <= 64 && 20 * batch <= 7 * (n - 190); }
 
 static int n_reflectors(int n) { return n >= 3 ? n - 2 : 0; }
 
