@@ -111,6 +111,21 @@ def test_unconverged_eigensolver(ctx):
     assert ctx.lib.vrc_rcwa_compute(it.h, 2) == 0
 
 
+def test_unconverged_eigensolver_team(ctx):
+    """The same at N = 242, where every matrix has a team of workgroups: the team leaves with its
+    master, every instance is flagged, and the next call solves cleanly."""
+    tune(ctx, "zgeev.max_sweeps", 1)
+    try:
+        rc, info, _ = raw_batch(ctx, 11, [rect_instance(0.9), rect_instance(1.2)])
+        msg = ctx.lib.vrc_last_error(ctx.h).decode()
+        assert rc == 1 and list(info) == [1, 1], (rc, info, msg)
+        assert "did not converge" in msg
+    finally:
+        tune(ctx, "zgeev.max_sweeps", 0)
+    rc, info, S = raw_batch(ctx, 11, [rect_instance(0.9), rect_instance(1.2)])
+    assert rc == 0 and (info == 0).all() and bool(S.isfinite().all())
+
+
 def test_varrcwa_depth_limit(ctx):
     """varRCWA that cannot meet pe within the depth limit accepts the segments and says so."""
     g = G.metasurface(1)
