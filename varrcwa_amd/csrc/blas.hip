@@ -1,5 +1,5 @@
-// Complex128 dense kernels for gfx950: FP64-MFMA ZGEMM (strided and descriptor
-// batched) and the elementwise matrix kernels used between the factorizations.
+// Complex128 dense kernels for gfx950: FP64-MFMA ZGEMM (strided batches)
+// and the elementwise matrix kernels used between the factorizations.
 //
 // ZGEMM tiles: 64x64 output per workgroup (8 wavefronts by default; a 4-wave variant
 // selectable), or 32x32 where few tiles would leave CUs idle, from v_mfma_f64_16x16x4f64
@@ -333,7 +333,7 @@ __device__ __forceinline__ void zgemm_tile32(int m, int n, int k, cd alpha, cons
   }
 }
 
-// Scale-only path for k == 0 (C = beta*C), shared by both batch modes.
+// Scale-only path for k == 0 (C = beta*C).
 __device__ __forceinline__ void scale_tile(int m, int n, cd beta, cd* C, long ldc, int tm, int tn) {
   const bool beta0 = (beta.x == 0.0 && beta.y == 0.0);
   for (int e = threadIdx.x; e < GT_M * GT_N; e += GT_THREADS) {
@@ -362,9 +362,9 @@ __global__ __launch_bounds__(GT_THREADS) void zgemm_strided_kernel(int m, int n,
 // Transposed operands: six waves per SIMD (80 registers) measured 63.2 TFLOP/s at 250 x 882^3 (C,
 // N) against 59.9; plain operands run best as the compiler allocates them (64.8 against 63.4).
 template <int OPA, int OPB>
-__global__ __launch_bounds__(512, OPA == OP_N && OPB == OP_N ? 1 : 6) void zgemm_strided8_kernel(int m, int n, int k, cd alpha, const cd* A, long lda,
-                                                            long sA, const cd* B, long ldb, long sB, cd beta, cd* C,
-                                                            long ldc, long sC) {
+__global__ __launch_bounds__(512, OPA == OP_N && OPB == OP_N ? 1 : 6) void zgemm_strided8_kernel(
+    int m, int n, int k, cd alpha, const cd* A, long lda, long sA, const cd* B, long ldb, long sB, cd beta, cd* C,
+    long ldc, long sC) {
   const int tm = blockIdx.x, tn = blockIdx.y;
   const long b = blockIdx.z;
   zgemm_tile8<OPA, OPB>(m, n, k, alpha, A + b * sA, lda, B + b * sB, ldb, beta, C + b * sC, ldc, tm, tn);
@@ -379,19 +379,6 @@ __global__ __launch_bounds__(GS_THREADS) void zgemm_small_kernel(int m, int n, i
   zgemm_tile32<OPA, OPB>(m, n, k, alpha, A + b * sA, lda, B + b * sB, ldb, beta, C + b * sC, ldc, tm, tn);
 }
 
-template <int OPA, int OPB>
-__global__ __launch_bounds__(GT_THREADS) void zgemm_desc_kernel(const GemmDesc* __restrict__ desc) {
-  const GemmDesc d = desc[blockIdx.z];
-  const int tm = blockIdx.x, tn = blockIdx.y;
-  if (d.m <= 0 || d.n <= 0) return;
-  if (tm * GT_M >= d.m || tn * GT_N >= d.n) return;
-  if (d.k <= 0) {
-    scale_tile(d.m, d.n, d.beta, d.C, d.ldc, tm, tn);
-    return;
-  }
-  zgemm_tile<OPA, OPB>(d.m, d.n, d.k, d.alpha, d.A, d.lda, d.B, d.ldb, d.beta, d.C, d.ldc, tm, tn);
-}
-
 static int g_small_waves = 8;   // wavefronts of the 64x64-tile kernel (4 or 8)
 void zgemm_set_small_waves(int w) { g_small_waves = w == 8 ? 8 : 4; }
 int zgemm_get_small_waves() { return g_small_waves; }
@@ -400,10 +387,12 @@ int zgemm_get_small_waves() { return g_small_waves; }
 // 0.054 us, one per CU at a time either way while workgroups are few, so the smaller tile wins
 // while its rounds over the 256 CUs cost less (single matrices and short right-hand sides;
 // us with 64 / 32: 162^3 26 / 12, 450^3 65 / 27, 882^3 126 / 141, 64 x 484 x 64 12 / 6, 16
-// products of 242^3 43 / 54), or where 64 fits the edges so badly that 32 saves a third of the
-// tiles (256 products 81 x 81 x 128: 74 / 56). Tiles of 128x64 and 128x128 were slower than 64x64
-// at every size measured (N = 242 .. 1250, batches of 1 .. 2000; 250 products of 882^3: 22.2 ms
-// against 21.3) and are gone.
+// products of 242^3 43 / 54), or where 64 fits the edges so badly that 32 saves more than an eighth
+// of the tiles' area (37 and 129 are the costs of one tile with the chip full; 256 products
+// 81 x 81 x 128: 74 / 56). Tiles of 128x64 and 128x128 are gone: slower than 64x64 with plain
+// operands at every size measured (N = 242 .. 1250, batches of 1 .. 2000; 250 products of 882^3:
+// 22.2 ms against 21.3) and with transposed ones at most (N = 128 .. 882, batches of 8 .. 150: 0.94 to
+// 2.7 times their speed; below 1 only where 200 to 256 tiles of 128x128 made one full round).
 static bool zgemm_use_32(int m, int n, int k, int batch) {
   const long n64 = (long)cdiv_up(m, GT_M) * cdiv_up(n, GT_N) * batch;
   const long n32 = (long)cdiv_up(m, GS_T) * cdiv_up(n, GS_T) * batch;
@@ -466,23 +455,6 @@ void zgemm_strided(hipStream_t s, int opA, int opB, int m, int n, int k, cd alph
     default: zgemm_strided_kernel<OP_C, OP_C><<<grid, GT_THREADS, 0, s>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC); break;
   }
   launch_check("zgemm_strided");
-}
-
-void zgemm_desc(hipStream_t s, int opA, int opB, const GemmDesc* d_desc, int count, int max_m, int max_n) {
-  if (count <= 0 || max_m <= 0 || max_n <= 0) return;
-  dim3 grid(cdiv_up(max_m, GT_M), cdiv_up(max_n, GT_N), count);
-  switch (opA * 3 + opB) {
-    case 0: zgemm_desc_kernel<OP_N, OP_N><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-    case 1: zgemm_desc_kernel<OP_N, OP_T><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-    case 2: zgemm_desc_kernel<OP_N, OP_C><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-    case 3: zgemm_desc_kernel<OP_T, OP_N><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-    case 4: zgemm_desc_kernel<OP_T, OP_T><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-    case 5: zgemm_desc_kernel<OP_T, OP_C><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-    case 6: zgemm_desc_kernel<OP_C, OP_N><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-    case 7: zgemm_desc_kernel<OP_C, OP_T><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-    default: zgemm_desc_kernel<OP_C, OP_C><<<grid, GT_THREADS, 0, s>>>(d_desc); break;
-  }
-  launch_check("zgemm_desc");
 }
 
 // ============================================================ elementwise kernels

@@ -88,17 +88,6 @@ inline int cdiv_up(long a, long b) { return (int)((a + b - 1) / b); }
 // Operation on an operand of a matrix product.
 enum Op : int { OP_N = 0, OP_T = 1, OP_C = 2 };
 
-// One entry of a descriptor-driven batched GEMM: C = alpha*op(A)*op(B) + beta*C.
-// Entries with m<=0, n<=0 are skipped; k<=0 scales C by beta.
-struct GemmDesc {
-  int m, n, k, pad_;
-  const cd* A;
-  const cd* B;
-  cd* C;
-  long lda, ldb, ldc;
-  cd alpha, beta;
-};
-
 // gamma = sqrt(lambda) with the branch rule of WaveEquationSolver's GammaSqrtOp
 // (src/rcwa/WaveEquationSolver.cpp:8-22): Im >= 0, flipped if |Im| < |Re| and Re < 0.
 __device__ inline cd gamma_branch(cd lam) {
