@@ -419,8 +419,9 @@ def test_zgeev_wide_hessenberg(ctx, n):
 
 @pytest.mark.parametrize("n", [200, 257, 258, 259, 322])
 def test_zgeev_spread_hessenberg(ctx, n):
-    """The Hessenberg panel spread over workgroups at the edges of its row blocks, column tiles
-    and panels (64), with identity reflectors (triangular input) in the batch."""
+    """The Hessenberg panel spread over workgroups (from N = 258) at the edges of its row blocks,
+    column tiles and panels (64), and the largest sizes that are not spread, with identity
+    reflectors (triangular input) in the batch."""
     rng = np.random.default_rng(5000 + n)
     A = crand(rng, 3, n, n)
     A[1] = np.triu(A[1]) + 3.0 * np.diag(np.arange(n))

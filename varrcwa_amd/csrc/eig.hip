@@ -103,7 +103,6 @@ __device__ __forceinline__ void house_small(cd alpha, cd y, cd z, double& beta, 
 }
 
 // ===================================================================== Hessenberg
-// out[i] = sum_{r>=r0} conj(Vf[r, p+i]) * x[r] for i < j, x in LDS.
 constexpr int GV_W = 8;  // trailing-product loads in flight per thread
 
 // One complex value read with the non-temporal hint (streamed once per column, not reused
@@ -235,9 +234,8 @@ constexpr int GEHRD_WIDE_BATCH = 512;
 // 5.27 -> 4.34; N = 242: 100 matrices 11.0 -> 8.6, 200 matrices 12.8 -> 10.2.
 template <int PTT, bool WIDE>
 __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(WIDE ? 2 : 4))) void gehrd_panel_kernel(
-    int N, int p, int nb, cd* A, long lda, long sA, cd* Vf,
-                                                          long sV, cd* Y, long sY, cd* Tp, long sT, cd* tau,
-                                                          long sTau) {
+    int N, int p, int nb, cd* A, long lda, long sA, cd* Vf, long sV, cd* Y, long sY, cd* Tp, long sT, cd* tau,
+    long sTau) {
   const long b = blockIdx.x;
   A += b * sA;
   Vf += b * sV;
@@ -2337,9 +2335,12 @@ void zgeev_set_bulges(int nb) { g_bulges = nb < 1 ? 1 : (nb > NBUL ? NBUL : nb);
 // window products staged through LDS), 2: hqr_w48_kernel (W = 48, two matrices per CU),
 // 4: hqr_w32_kernel (W = 32, four matrices per CU); -1: automatic, 4 for N <= 256 in launches
 // of at least 384 matrices and for N <= 512 in launches of at least 768, 2 for N <= 1024 in
-// launches of at least 384, else 0 (measured: at N = 98 and 242 the four-per-CU kernel wins
-// from about 1.5 matrices per CU, at N = 450 from about 3; at N = 882 the two-per-CU kernel in
-// 512-matrix launches is 2.7 % faster than the one-per-CU kernel in 256-matrix launches)
+// launches of at least 384, else 0. The lines are those of earlier kernels; with the present ones
+// (QR stage of random matrices, ms, variants 0 / 2 / 4): N = 98 128 matrices 6.7 / 10.0 / 8.5, 384
+// 13.3 / 12.1 / 10.8, 640 20.0 / 20.4 / 11.0; N = 162 384 29.1 / 24.1 / 28.5, 640 43.4 / 40.9 / 31.1;
+// N = 242 384 54.4 / 46.4 / 67.4, 640 81.8 / 77.4 / 70.5, 1024 111 / 92 / 77; N = 338 384 101 / 86 / 150, 768
+// 154 / 143 / 165; N = 450 384 174 / 158 / 313; N = 882 512 800 / 833. So variant 4 is early at N = 242 and 338,
+// variant 2 late from N = 162 to 450 and, on these matrices, early at N = 882.
 static int g_qr_variant = -1;
 static int qr_variant_for(int n, int batch) {
   if (g_qr_variant >= 0) return g_qr_variant;
@@ -2394,7 +2395,8 @@ int zgeev_get_aed() { return g_aed_window; }
 // default); one launch holding all of them would make the others wait. Four contexts, ms a round
 // with all CUs for each / a quarter / before there were teams: a stack of 10 layers each at N = 882
 // 689 / 345 / 626, four at N = 450 300 / 181 / 227; a single matrix each at N = 882 179 / 193 / 483.
-// The bits do not depend on the team.
+// The bits do not depend on the team. QR stage without / with a team below the line, ms: 8 matrices
+// of N = 98 6.55 / 6.61, 126 9.76 / 9.82, 162 14.1 / 14.0, 198 19.2 / 18.3; 128 of N = 162 14.8 / 15.2.
 static int team_size(int n, int batch, int streams) {
   if (n < 200 || n > 65535) return 1;
   const int per_xcd = (batch + 7) / 8;

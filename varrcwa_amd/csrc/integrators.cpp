@@ -442,7 +442,9 @@ SMat smat_at(cd* p, long blk) {
 }
 
 // Matrices of N x N that a tree of star products may hold (pairs in flight, or all its levels): what
-// 8 GiB hold unless "cascade.matrices" says otherwise; at most 8192 products in one batch.
+// 8 GiB hold unless "cascade.matrices" says otherwise; at most 8192 products in one batch. 25 stacks
+// of 10 layers at N = 882, star products: 281 ms with 1 GiB, 273 with 8, 256 with 16, 250 with 32;
+// 8 of the GPU's 288 GB leave room for callers that share it.
 int g_cascade_mats = 0;
 size_t cascade_mats(int N) {
   if (g_cascade_mats > 0) return (size_t)g_cascade_mats;
@@ -527,8 +529,9 @@ void cascade_set_matrices(int n) { g_cascade_mats = n < 0 ? 0 : n; }
 // eigensolves and slab S-matrices run in groups of up to g_rcwa_group per launch (one
 // eigensolve per workgroup), the two end media riding with the first group; a group's star
 // products then run as a tree, the groups in slice order (the reference cascades slice by
-// slice; the product is associative). Each matrix's result does not depend on the group it is
-// solved in.
+// slice; the product is associative). Results depend on the groups at rounding level: the trees
+// differ, and for N > 257 the Hessenberg panel's sums do where a launch of few matrices spreads it
+// (with 64 slices a group the first launch also holds the end media, so it takes the other form).
 static int g_rcwa_group = 64;
 void rcwa_set_group(int g) { g_rcwa_group = g < 1 ? 1 : g; }
 void Integrator::rcwa(const std::vector<std::pair<double, double>>& slices, bool) {
@@ -979,7 +982,11 @@ void Integrator::differential(int Nsteps) {
 // the outputs at instance offset I0.
 // tape (optional): receives the prefix before every K-th layer and the cascade before the
 // projection of the group's instances.
-constexpr int CASCADE_SEQ = 128;  // instances from which the layers are cascaded one by one
+// Instances from which the layers are cascaded one by one: their products fill the CUs by then, and
+// a tree's copies cost memory. Star products of 10 layers, ms, tree / one by one: N = 18 127
+// instances 0.67 / 1.22; N = 98 64 3.8 / 5.6, 127 6.0 / 7.6; N = 242 24 10.2 / 15.5, 64 20 / 24, 127 38 / 41;
+// N = 450 8 21 / 29, 64 111 / 117 (small N would still gain beyond 128).
+constexpr int CASCADE_SEQ = 128;
 static void cascade_group(vrc_ctx& c, int N, int L, int GB, int I0, bool homog, const cd* tu, const cd* ru,
                           const cd* We, const cd* Ve, const cd* ge, cd* S_out, cd* W0o, cd* V0o, cd* g0o, cd* W1o,
                           cd* V1o, cd* g1o, StackTape* tape = nullptr) {

@@ -93,8 +93,7 @@ __global__ __launch_bounds__(256) void getrf_panel_kernel(int n, int k, int kb, 
 // kb <= LUR_NB panel columns. Per column (one barrier): wave maximum and its first row (largest
 // |re|+|im|, first index) posted with the candidate row, row exchange through LDS, elimination
 // in registers. Afterwards the panel's interchanges are applied to the other columns
-// [K, K+KB) of the block and, right of the panel, U12 = L11^{-1} A12 is solved (one
-// thread per column).
+// [K, K+KB) of the block and, right of the panel, U12 = L11^{-1} A12 is solved.
 // A panel is a serial chain and bound by its latencies, so nothing in it waits for memory but
 // the first and the last loads: pivots go to memory after the columns (a store before each
 // barrier was waited for), the rows of the other columns that the panel swaps are loaded
@@ -102,8 +101,9 @@ __global__ __launch_bounds__(256) void getrf_panel_kernel(int n, int k, int kb, 
 // they were 16 dependent round trips), and U12 is solved by 16-column waves from LDS. Rows keep
 // their thread and exchange their places only; the columns rotate through the registers (a
 // ring, the finished ones behind the active ones), so that the loop over the columns stays one
-// copy of its code; the maximum goes over DPP lane moves. Per panel: n = 98 to 242
-// 43 -> 30-33 us, n = 450 51 -> 38 us, n = 882 67 -> 56 us (the elimination of 16 waves).
+// copy of its code; the maximum goes over DPP lane moves. Per panel, up to one matrix per
+// CU: n = 98 to 242 43 -> 30-33 us, n = 450 51 -> 38 us, n = 882 67 -> 56 us (the elimination of 16
+// waves); where CUs hold two or three (640 of n = 98, 480 of n = 242) 37 and 41 us.
 constexpr int LUR_NB = 16;
 constexpr int LUR_ROWS = 1024;
 
