@@ -90,8 +90,8 @@ int vrc_timing_read(vrc_ctx* ctx, double* ms, int* counts, int nstages);
  * the given instances (a sample of the batch to be solved; a few hundred slabs make full
  * launches) under candidate kernel switch settings, one switch at a time (the QR kernel
  * (zgeev.qr_variant 0, 2 or 4), the QR iteration's deflation window, the bulge count of
- * each QR kernel the sample launches, the ZGEMM tile shape, wavefronts and large-tile
- * threshold; settings that cannot change what runs are skipped), keeping a candidate only
+ * each QR kernel the sample launches, the wavefronts of the 64x64-tile ZGEMM;
+ * settings that cannot change what runs are skipped), keeping a candidate only
  * when it is >= 1 % faster, until
  * budget_s seconds have been spent. The winners are kept for N = 2 nx ny and put in
  * place before every later call that solves N x N systems (other N keep the values set
