@@ -952,7 +952,7 @@ int vrc_batch_plan_create(vrc_ctx* c, int nx, int ny, int ninst, const vrc_stack
           : c(cc), prev(cc->stream), cap(cs), timing(cc->timing) {
         c->stream = cs;
         c->timing = false;
-        c->pinned.hold = hold;
+        c->pinned.record(hold);
         c->ws.track_begin();
       }
       ~Recording() {
@@ -967,7 +967,7 @@ int vrc_batch_plan_create(vrc_ctx* c, int nx, int ny, int ninst, const vrc_stack
         }
         c->stream = prev;
         c->timing = timing;
-        c->pinned.hold = nullptr;
+        c->pinned.record(nullptr);
         (void)hipStreamSynchronize(cap);
         (void)hipStreamDestroy(cap);
       }

@@ -462,18 +462,23 @@ void cascade_tree(vrc_ctx& c, int N, int B, int n, std::vector<SPtr> items, SMat
   hipStream_t st = c.stream;
   const long NN = (long)N * N;
   const size_t M = sizeof(cd) * NN;
-  std::vector<DevBuf> keep;
+  // one buffer for the products of all levels (n - 1 a row), one for the right operands of a chunk
+  const int most = (int)std::min<size_t>(8192, std::max<size_t>(1, cascade_mats(N) / 16));
+  DevBuf Sb, Rb;
+  if (n > 1) {
+    Sb = c.ws.get(4 * M * (size_t)B * (n - 1));
+    Rb = c.ws.get(4 * M * (size_t)std::min(most, B * (n / 2)));
+  }
+  cd* Sl = Sb.as<cd>();  // the level's products
   while (n > 1) {
     const int np = n / 2, m = np + (n & 1);
     const int total = B * np;
-    const int per = std::max(1, std::min<int>(total, (int)std::min<size_t>(8192, cascade_mats(N) / 16)));
-    DevBuf Sb = c.ws.get(4 * M * (size_t)total);
+    const int per = std::min(total, most);
     std::vector<SPtr> next((size_t)B * m);
     for (int q0 = 0; q0 < total; q0 += per) {
       const int P = std::min(per, total - q0);
-      cd* S0 = Sb.as<cd>() + 4 * NN * q0;
+      cd* S0 = Sl + 4 * NN * q0;
       SMat S = smat_at(S0, P * NN);
-      DevBuf Rb = c.ws.get(4 * M * (size_t)P);
       std::vector<const void*> left(4 * (size_t)P), right(4 * (size_t)P);
       for (int q = 0; q < P; ++q) {
         const int b = (q0 + q) / np, j = (q0 + q) % np;
@@ -493,7 +498,7 @@ void cascade_tree(vrc_ctx& c, int N, int B, int n, std::vector<SPtr> items, SMat
     }
     if (n & 1)
       for (int b = 0; b < B; ++b) next[(size_t)b * m + np] = items[(size_t)b * n + n - 1];
-    keep.push_back(std::move(Sb));
+    Sl += 4 * NN * total;
     items.swap(next);
     n = m;
   }

@@ -23,6 +23,13 @@ struct PinnedPool {
   };
   std::vector<Block> blocks;
   std::vector<void*>* hold = nullptr;
+  char* hold_at = nullptr;  // what is left of the newest block of the recording
+  size_t hold_left = 0;
+  // Blocks go to the recording h from now on (nullptr: to the pool).
+  void record(std::vector<void*>* h) {
+    hold = h;
+    hold_left = 0;
+  }
   ~PinnedPool();
   // Copies host[0, bytes) into a pinned block and enqueues its copy to dst on stream s.
   void upload(hipStream_t s, void* dst, const void* host, size_t bytes);

@@ -148,8 +148,25 @@ void PinnedPool::upload_with(hipStream_t s, void* dst, size_t bytes, const std::
   if (bytes == 0) return;
   void* p = nullptr;
   if (hold) {  // recording a graph: the block belongs to the recording
-    VRC_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
-    hold->push_back(p);
+    // Small uploads share blocks: a tree of star products makes many of them, and with a block each
+    // (and a buffer per level) recording 4 stacks of 3 layers took 1.5 ms at N = 50 and 3.3 at
+    // N = 98, now 0.6 and 1.1 (layer by layer, a block each, 0.8 and 1.4).
+    constexpr size_t SHARED = 256 << 10;
+    const size_t need = (bytes + 255) & ~(size_t)255;
+    if (need > SHARED / 4 || need > hold_left) {
+      const size_t size = need > SHARED / 4 ? need : SHARED;
+      VRC_HIP(hipHostMalloc(&p, size, hipHostMallocDefault));
+      hold->push_back(p);
+      if (size == SHARED) {
+        hold_at = (char*)p;
+        hold_left = SHARED;
+      }
+    }
+    if (need <= SHARED / 4) {
+      p = hold_at;
+      hold_at += need;
+      hold_left -= need;
+    }
     fill((char*)p);
     VRC_HIP(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, s));
     return;
