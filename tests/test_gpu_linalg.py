@@ -286,6 +286,28 @@ def test_zgeev_window_edges(ctx, variant, n):
         assert ctx.lib.vrc_tune_set(b"zgeev.qr_variant", -1) == 0
 
 
+@pytest.mark.parametrize("n", [5, 50, 98])
+def test_zgeev_defective(ctx, n):
+    """Nilpotent Jordan blocks: one eigenvector for n equal eigenvalues, so the back substitution of
+    the others overflows. The eigenvalues of these triangular matrices are their diagonal, every
+    finite vector is an eigenvector, and a vector without a finite component is NaN throughout."""
+    import torch
+    for A in (np.diag(np.ones(n - 1), 1) + 0j, np.diag(np.ones(n - 1), 1) + 2.0 * np.eye(n)):
+        dA = to_dev_colmajor(A[None])
+        w = torch.zeros((1, n), dtype=torch.complex128, device="cuda")
+        VR = torch.zeros_like(dA)
+        info = torch.zeros(1, dtype=torch.int32, device="cuda")
+        ctx.check(ctx.lib.vrc_zgeev(ctx.h, n, ptr(dA), n, n * n, ptr(w), n, ptr(VR), n, n * n, ptr(info), 1), "zgeev")
+        ctx.sync()
+        assert int(info[0]) == 0
+        assert np.array_equal(np.sort_complex(w.cpu().numpy()[0]), np.sort_complex(np.diag(A)))
+        V = from_dev_colmajor(VR)[0]
+        ok = np.isfinite(V).all(axis=0)
+        assert ok[0]
+        assert np.abs(A @ V[:, ok] - V[:, ok] * w.cpu().numpy()[0][ok]).max() < 1e-12 * n
+        assert np.isnan(V[:, ~ok]).all()
+
+
 def _eig_check_values(ctx, A):
     """Eigenvalues and vectors with the residual checked (no comparison of sorted spectra:
     eigenvalues of one modulus sort arbitrarily)."""

@@ -2223,6 +2223,7 @@ __global__ __launch_bounds__(256) void normalize_cols_kernel(int N, cd* V, long 
     int oi = __shfl_xor(bi, o, 64);
     if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
   }
+  if (bi >= N) bi = 0;  // no component compares (NaN): the vector stays NaN
   const cd vk = cscale(v[bi], scl);
   const cd rot = cscale(cconj(vk), 1.0 / sqrt(best));
   for (int r = lane; r < N; r += 64) {
