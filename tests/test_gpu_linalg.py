@@ -308,6 +308,22 @@ def test_zgeev_defective(ctx, n):
         assert np.isnan(V[:, ~ok]).all()
 
 
+@pytest.mark.parametrize("n,batch", [(98, 513), (300, 2), (300, 60), (530, 65)])
+@pytest.mark.parametrize("tiny", [1e-170, 1e-200])
+def test_zgeev_tiny_coupling(ctx, n, batch, tiny):
+    """Eigenvalues of order one coupled by entries whose squares underflow: the reflector of such a
+    column has to be unitary all the same, in the Hessenberg panel of one workgroup per matrix
+    (256, 512 and 1024 threads) and in the one spread over workgroups (300, 2)."""
+    rng = np.random.default_rng(9000 + n)
+    A = tiny * crand(rng, 1, n, n)
+    A[:, np.arange(n), np.arange(n)] = np.arange(n)
+    w, V = _eig_values(ctx, A, batch)
+    for b in (0, batch - 1):
+        assert np.abs(np.sort(w[b].real) - np.arange(n)).max() < 1e-13 * n
+        assert np.abs(np.linalg.norm(V[b], axis=0) - 1.0).max() < 1e-13 * n
+        assert np.abs(A[0] @ V[b] - V[b] * w[b][None, :]).max() < 1e-12 * n * n
+
+
 def _eig_check_values(ctx, A):
     """Eigenvalues and vectors with the residual checked (no comparison of sorted spectra:
     eigenvalues of one modulus sort arbitrarily)."""

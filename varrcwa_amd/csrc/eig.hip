@@ -70,6 +70,28 @@ __device__ __forceinline__ double rcp_nr(double v) {
 }
 // Squares of values whose sum lies in this range neither overflow nor lose small parts.
 __device__ __forceinline__ bool squares_safe(double s) { return s <= 0x1p800 && s >= 0x1p-800; }
+__device__ __forceinline__ double wmax(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  return v;
+}
+// |x / m|^2 for m > 0, the largest |re|, |im| of the values summed: their norm is m sqrt(sum) where
+// the squares themselves are out of range (a norm that underflows to zero beside a reflector's
+// nonzero first entry gives a reflector that is not unitary).
+__device__ __forceinline__ double scaled_norm2(cd x, double m) { return cnorm2(mk(x.x / m, x.y / m)); }
+
+// |x|_2 of x[0 .. n) where the squares are out of range; every wave computes it by itself.
+__device__ inline double wave_norm(const cd* x, int n) {
+  const int lane = threadIdx.x & 63;
+  double m = 0.0, s = 0.0;
+#pragma unroll 1
+  for (int r = lane; r < n; r += 64) m = fmax(m, fmax(fabs(x[r].x), fabs(x[r].y)));
+  m = wmax(m);
+  if (!(m > 0.0)) m = 1.0;
+#pragma unroll 1
+  for (int r = lane; r < n; r += 64) s += scaled_norm2(x[r], m);
+  return m * sqrt(wsum(s));
+}
 
 // The reflector of house() for |x|^2 = xn2 without a division or a square root in the
 // chain: 1/|(alpha, x)| from one reciprocal square root, 1/(alpha - beta) as conj(d) / |d|^2.
@@ -91,6 +113,17 @@ __device__ __forceinline__ void house_fast(cd alpha, double xn2, double& beta, c
     beta = alpha.x;
     tau = scale = mk(0.0, 0.0);
   }
+}
+
+// The same for a vector spread over the wavefront (x: this lane's component).
+__device__ __forceinline__ void wave_house(cd alpha, cd x, double& beta, cd& tau, cd& scale) {
+  const double xn2 = wsum(cnorm2(x));
+  if (__builtin_expect(squares_safe(cnorm2(alpha) + xn2), 1)) {
+    house_fast(alpha, xn2, beta, tau, scale);
+    return;
+  }
+  const double m = wmax(fmax(fabs(x.x), fabs(x.y)));
+  house(alpha, m > 0.0 ? m * sqrt(wsum(scaled_norm2(x, m))) : sqrt(xn2), beta, tau, scale);
 }
 
 // The same for x = (y, z) (z = 0 for a 2-vector).
@@ -301,7 +334,12 @@ __global__ __launch_bounds__(PTT) __attribute__((amdgpu_waves_per_eu(WIDE ? 2 : 
     __syncthreads();
     double xn2 = 0.0;
     for (int w = 0; w < PTT / 64; ++w) xn2 += rn[w];
-    const double xnorm = sqrt(xn2);
+    double xnorm = sqrt(xn2);
+    // Not in the wide form: any use of xn2 there costs 24 registers and 3 to 8 % of the reduction
+    // (N = 162, 2 matrices 3.31 -> 3.57 ms), so a column whose squares underflow beside a nonzero
+    // entry is not reduced accurately for N <= 257 in launches of up to 512 matrices.
+    if constexpr (!WIDE)
+      if (__builtin_expect(!squares_safe(xn2), 0)) xnorm = wave_norm(bvec + c + 2, N - c - 2);
     double beta;
     cd tv, scale;
     house(bvec[c + 1], xnorm, beta, tv, scale);
@@ -574,7 +612,7 @@ __global__ __launch_bounds__(256) void gehrd_col_b_kernel(int N, int p, int j, c
   red[q][tr] = ab;
   __syncthreads();
   if (q > 0) return;
-  double nn = 0.0;
+  cd x = mk(0.0, 0.0);
   if (r < N) {
     cd b = work[r];
     if (j > 0) {
@@ -582,10 +620,15 @@ __global__ __launch_bounds__(256) void gehrd_col_b_kernel(int N, int p, int j, c
       work[r] = b;
     }
     if (r <= c) A[r + (long)c * lda] = b;
-    if (r >= c + 2) nn = cnorm2(b);
+    if (r >= c + 2) x = b;
   }
-  nn = wsum(nn);
-  if (tr == 0) work[gw.norm + blk] = mk(nn, 0.0);
+  // the block's part: a sum of squares and the scale of the values squared (0: all zero)
+  double nn = wsum(cnorm2(x)), big = 1.0;
+  if (!squares_safe(nn)) {
+    big = wmax(fmax(fabs(x.x), fabs(x.y)));
+    if (big > 0.0) nn = wsum(scaled_norm2(x, big));
+  }
+  if (tr == 0) work[gw.norm + blk] = mk(nn, big);
 }
 
 // Third step: the reflector (every workgroup computes it), the trailing product's tiles
@@ -602,9 +645,15 @@ __global__ __launch_bounds__(256) void gehrd_col_c_kernel(int N, int p, int j, c
   __shared__ cd vs[GS_C];
   const int t = threadIdx.x, lane = t & 63, q = t >> 6;
   const int c = p + j;
-  double nn = 0.0;
-  for (int k = lane; k < gw.nblk; k += 64) nn += work[gw.norm + k].x;
-  const double xnorm = sqrt(wsum(nn));
+  double nn = 0.0, big = 0.0;
+  for (int k = lane; k < gw.nblk; k += 64) big = fmax(big, work[gw.norm + k].y);
+  big = wmax(big);
+  for (int k = lane; k < gw.nblk; k += 64) {
+    const cd part = work[gw.norm + k];
+    const double f = big > 0.0 ? part.y / big : 1.0;
+    nn += part.x * (f * f);
+  }
+  const double xnorm = (big > 0.0 ? big : 1.0) * sqrt(wsum(nn));
   const cd alpha = work[c + 1];
   double beta;
   cd tv, scale;
@@ -1636,11 +1685,10 @@ __device__ int aed(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz
         if (ns > 1) {
           // reflect the spike s * conj(U[0][0..ns)) onto e1 (zlaqr3 "reflect spike back")
           cd w = lane < ns ? cconj(U[0][lane]) : mk(0.0, 0.0);
-          const double xn2 = wsum(lane >= 1 && lane < ns ? cnorm2(w) : 0.0);
           const cd alpha = cconj(U[0][0]);
           double beta;
           cd tau, scale;
-          house_fast(alpha, xn2, beta, tau, scale);
+          wave_house(alpha, lane >= 1 && lane < ns ? w : mk(0.0, 0.0), beta, tau, scale);
           wave_sync();
           L.aedv[lane] = lane == 0 ? mk(1.0, 0.0) : (lane < ns ? cmul(w, scale) : mk(0.0, 0.0));
           wave_sync();
@@ -1650,10 +1698,9 @@ __device__ int aed(QrLds<C::W, C::T>& L, int N, cd* H, long ldh, cd* Z, long ldz
             const int len = ns - c - 1;
             const cd a0 = T[c + 1][c];
             const cd xv = (lane >= c + 2 && lane < ns) ? T[lane][c] : mk(0.0, 0.0);
-            const double xnc2 = wsum(cnorm2(xv));
             double bc;
             cd tc, sc;
-            house_fast(a0, xnc2, bc, tc, sc);
+            wave_house(a0, xv, bc, tc, sc);
             wave_sync();
             if (lane < len) L.aedv[lane] = lane == 0 ? mk(1.0, 0.0) : cmul(T[c + 1 + lane][c], sc);
             wave_sync();
